@@ -41,6 +41,12 @@ extern "C" {
 #define MOEGEMM_PRECISION_IEEE 0 /* operands used as given */
 #define MOEGEMM_PRECISION_TF32 1 /* fp32 operands rounded to a 10-bit mantissa (ties away) */
 
+/* Values of `vector_layout` for transposed 16-bit operands (see moegemm_grouped_gemm); any other
+ * non-zero value means the row-major vector layout. */
+#define MOEGEMM_LAYOUT_AT 0x10001   /* A stored [K, M] (unit row stride), B row-major */
+#define MOEGEMM_LAYOUT_BT 0x20001   /* A row-major, B stored [N, K] (unit row stride) */
+#define MOEGEMM_LAYOUT_ATBT 0x30001 /* both transposed */
+
 /* Size of the tile queue of the work-stealing launches (17 int32 counters, each in a 256-byte
  * block of its own; the buffer is 256-byte aligned). */
 #define MOEGEMM_QUEUE_BYTES 4352
@@ -77,6 +83,12 @@ int moegemm_kernel_info(int dtype, int index, int32_t* out7);
  * pitches and K, N multiples of 8 elements, C row pitch a multiple of 4, 16-byte aligned A/B and
  * 8-byte aligned C bases, A and C row pitches under 2^22 elements (256 rows under 2 GiB; any
  * number of rows) and B under 2 GiB: the launch then uses the LDS-DMA kernel.
+ * In generic mode the MOEGEMM_LAYOUT_* values promise the same of transposed operands: a transposed
+ * A has a unit M stride and a transposed B a unit K stride, with a pitch multiple of 8 elements and at least its
+ * extent, 16-byte alignment, an extent multiple of 8 (K for an operand whose rows run along K, M or
+ * N for one whose rows run along it), 256 rows of a K-contiguous operand and all K + 1024 rows of
+ * the other kind under 2 GiB; tiles compiled for that layout (moegemm_kernel_layouts) then run the
+ * LDS-DMA kernel, others the general one.
  * Otherwise (or for fp32) the general kernel runs, which accepts any strides and alignment.
  */
 int moegemm_grouped_gemm(const int64_t* a_ptrs, const int64_t* b_ptrs, const int64_t* c_ptrs,
@@ -150,6 +162,17 @@ int moegemm_matmul_splitk(const void* a, const void* b, void* c, int32_t m, int3
                           int32_t block_m, int32_t block_n, int32_t block_k, int32_t group_size_m,
                           int32_t num_warps, int32_t num_stages, int32_t splits, int32_t grid_size,
                           void* workspace, int64_t workspace_bytes, int32_t b_stream, void* stream);
+/* moegemm_matmul_splitk for every operand layout the LDS-DMA kernels take: row-major operands as
+ * above, and transposed ones (the layouts of MOEGEMM_LAYOUT_*, found from the strides) on the tiles
+ * compiled for them (moegemm_kernel_layouts).  It serves launch_matmul (reference
+ * kernels/matmul.py:332-392) on transposed views: a linear layer's [N, K] weight, and the products
+ * of a backward pass. */
+int moegemm_matmul_splitk_transposed(const void* a, const void* b, void* c, int32_t m, int32_t n, int32_t k,
+                                     int64_t stride_am, int64_t stride_ak, int64_t stride_bk, int64_t stride_bn,
+                                     int64_t stride_cm, int64_t stride_cn, int32_t dtype, int32_t block_m,
+                                     int32_t block_n, int32_t block_k, int32_t group_size_m, int32_t num_warps,
+                                     int32_t num_stages, int32_t splits, int32_t grid_size, void* workspace,
+                                     int64_t workspace_bytes, int32_t b_stream, void* stream);
 /*
  * moegemm_matmul_splitk without the workspace argument: the partials and tile counters live in a
  * static device array of MOEGEMM_NOALLOC_SCRATCH_BYTES inside the library (one per GPU, held until
@@ -220,6 +243,11 @@ int moegemm_grouped_gemm_streamk(const int64_t* a_ptrs, const int64_t* b_ptrs, c
 /* 1 when compiled kernel `index` of `dtype` can run the SwiGLU epilogue, 0 when not, < 0 on a bad
  * index.  No counterpart in the reference (its Triton pools have no fused epilogue). */
 int moegemm_kernel_swiglu(int dtype, int index);
+
+/* Operand layouts compiled kernel `index` of `dtype` runs on the LDS-DMA path, as a bit mask: bit 0
+ * row-major, bit 1 A transposed, bit 2 B transposed, bit 3 both; < 0 on a bad index.  No counterpart
+ * in the reference (its Triton kernels take strides). */
+int moegemm_kernel_layouts(int dtype, int index);
 
 /*
  * Grouped GEMM over the expert-sorted layout of torch.nn.functional.grouped_mm (2-D A, 3-D B):

@@ -72,18 +72,21 @@ int check_common(int dtype, int input_precision, int group_size_m, const KernelE
   return MOEGEMM_OK;
 }
 
-int launch(const KernelEntry* e, KParams& p, int grid, bool vector_layout, int32_t b_stream, void* stream) {
+// `layout`: the operands' OperandLayout when they meet the LDS-DMA preconditions, else kGeneral.
+constexpr int kGeneral = -1;
+
+int launch(const KernelEntry* e, KParams& p, int grid, int layout, int32_t b_stream, void* stream) {
   if (b_stream != 0 && b_stream != 1) return fail(MOEGEMM_ERR_INVALID, "b_stream must be 0 or 1 (got %d)", b_stream);
   p.b_stream = b_stream;
-  LaunchFn fn = (vector_layout && e->launch_fast) ? e->launch_fast : e->launch_general;
+  LaunchFn fast = layout == 0 ? e->launch_fast : layout > 0 ? e->launch_transposed[layout - 1] : nullptr;
+  LaunchFn fn = fast ? fast : e->launch_general;
   if (p.sk_tiles > 0) {  // stream-K tail: the fast path's stream-K kernel (the callers checked the layout)
-    if (!vector_layout || !e->launch_fast_streamk)
+    if (layout != 0 || !e->launch_fast_streamk)
       return fail(MOEGEMM_ERR_INVALID, "stream-K needs fp16/bf16 operands in the vector layout");
     fn = e->launch_fast_streamk;
   } else if (p.splits > 1) {  // split-K units: the fast path's split kernel (the callers checked the layout)
-    if (!vector_layout || !e->launch_fast_split)
-      return fail(MOEGEMM_ERR_INVALID, "split-K needs fp16/bf16 operands in the vector layout");
-    fn = e->launch_fast_split;
+    fn = layout == 0 ? e->launch_fast_split : layout > 0 ? e->launch_transposed_split[layout - 1] : nullptr;
+    if (!fn) return fail(MOEGEMM_ERR_INVALID, "split-K needs fp16/bf16 operands in the vector layout");
   }
   hipError_t err = fn(p, grid, reinterpret_cast<hipStream_t>(stream));
   if (err != hipSuccess) return fail(MOEGEMM_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(err));
@@ -239,6 +242,8 @@ bool panels_fit(int64_t k, int64_t sam, int64_t sbk, int64_t scm) {
   return kPanelRows * sam * 2 < kTwoGiB && kPanelRows * scm * 2 < kTwoGiB && k * sbk * 2 < kTwoGiB;
 }
 
+bool aligned(const void* p, uintptr_t bytes) { return (reinterpret_cast<uintptr_t>(p) & (bytes - 1)) == 0; }
+
 // Preconditions of the LDS-DMA fast path for one problem (see gemm_fast.h).
 bool vector_layout_ok(const void* a, const void* b, const void* c, int64_t m, int64_t n, int64_t k, int64_t sam,
                       int64_t sak, int64_t sbk, int64_t sbn, int64_t scm, int64_t scn, int dtype) {
@@ -246,10 +251,43 @@ bool vector_layout_ok(const void* a, const void* b, const void* c, int64_t m, in
   if (dtype != DT_BF16 && dtype != DT_F16) return false;
   if (sak != 1 || sbn != 1 || scn != 1) return false;
   if (k % 8 || n % 8 || sam % 8 || sbk % 8 || scm % 4 || sam < k || sbk < n || scm < n) return false;
-  if ((reinterpret_cast<uintptr_t>(a) & 15) || (reinterpret_cast<uintptr_t>(b) & 15) ||
-      (reinterpret_cast<uintptr_t>(c) & 7))
-    return false;
+  if (!aligned(a, 16) || !aligned(b, 16) || !aligned(c, 8)) return false;
   return panels_fit(k, sam, sbk, scm);
+}
+
+// One operand of the transposed LDS-DMA kernels: x_extent rows or columns of it times k, element
+// (x, k) at x * sx + k * sk.  Returns 0 for a K-contiguous panel (rows of x, at most kPanelRows of
+// them in one resource), 1 for an X-contiguous one (rows of k, one resource over all of them, up to
+// the zero slices a tile copies past K), -1 when neither can be copied in aligned 16-byte chunks.
+constexpr int64_t kCopiedPastK = 1024;  // rows past K a tile's copies may address (stages x block_k)
+int operand_layout(const void* base, int64_t x_extent, int64_t k, int64_t sx, int64_t sk) {
+  if (!aligned(base, 16)) return -1;
+  if (sk == 1 && sx % 8 == 0 && sx >= k && k % 8 == 0 && kPanelRows * sx * 2 < kTwoGiB) return 0;
+  if (sx == 1 && sk % 8 == 0 && sk >= x_extent && x_extent % 8 == 0 && (k + kCopiedPastK) * sk * 2 < kTwoGiB) return 1;
+  return -1;
+}
+
+// The OperandLayout of one problem for the LDS-DMA kernels, or kGeneral.
+int fast_layout(const void* a, const void* b, const void* c, int64_t m, int64_t n, int64_t k, int64_t sam, int64_t sak,
+                int64_t sbk, int64_t sbn, int64_t scm, int64_t scn, int dtype) {
+  if (vector_layout_ok(a, b, c, m, n, k, sam, sak, sbk, sbn, scm, scn, dtype)) return 0;
+  if (dtype != DT_BF16 && dtype != DT_F16) return kGeneral;
+  if (scn != 1 || n % 8 || scm % 4 || scm < n || !aligned(c, 8) || kPanelRows * scm * 2 >= kTwoGiB) return kGeneral;
+  const int la = operand_layout(a, m, k, sam, sak), lb = operand_layout(b, n, k, sbn, sbk);
+  if (la < 0 || lb < 0) return kGeneral;
+  const int layout = (la == 1 ? kAT : 0) | (lb == 0 ? kBT : 0);
+  return layout == 0 ? kGeneral : layout;  // layout 0 is vector_layout_ok's rule alone
+}
+
+// The layout a caller of the grouped launches promises (see MOEGEMM_LAYOUT_* in moegemm.h).
+int promised_layout(int32_t vector_layout) {
+  switch (vector_layout) {
+    case 0: return kGeneral;
+    case MOEGEMM_LAYOUT_AT: return kAT;
+    case MOEGEMM_LAYOUT_BT: return kBT;
+    case MOEGEMM_LAYOUT_ATBT: return kAT | kBT;
+    default: return 0;
+  }
 }
 
 }  // namespace
@@ -304,10 +342,13 @@ int grouped_impl(const int64_t* a_ptrs, const int64_t* b_ptrs, const int64_t* c_
   const KernelEntry* e = nullptr;
   int rc = check_common(dtype, input_precision, group_size_m, &e, block_m, block_n, block_k, num_warps, num_stages);
   if (rc != MOEGEMM_OK) return rc;
+  const int layout = promised_layout(vector_layout);
+  if (layout > 0 && homogeneous)
+    return fail(MOEGEMM_ERR_INVALID, "homogeneous groups are row-major: transposed operands need the strides table");
   if (swiglu) {
     if (dtype != DT_BF16 && dtype != DT_F16)
       return fail(MOEGEMM_ERR_INVALID, "the SwiGLU epilogue needs fp16 or bf16 operands");
-    if (!vector_layout)
+    if (layout != 0)
       return fail(MOEGEMM_ERR_INVALID, "the SwiGLU epilogue needs the vector layout (LDS-DMA kernel)");
     if (!e->swiglu_ok)
       return fail(MOEGEMM_ERR_INVALID,
@@ -349,7 +390,7 @@ int grouped_impl(const int64_t* a_ptrs, const int64_t* b_ptrs, const int64_t* c_
   if (rc != MOEGEMM_OK) return rc;
   if (p.total_tiles == 0) return MOEGEMM_OK;
   int grid = grid_size <= 0 ? p.total_tiles : (grid_size < p.total_tiles ? grid_size : p.total_tiles);
-  return launch(e, p, grid, vector_layout != 0, b_stream, stream);
+  return launch(e, p, grid, layout, b_stream, stream);
 }
 
 }  // namespace
@@ -400,15 +441,17 @@ static int matmul_splitk_impl(const void* a, const void* b, void* c, int32_t m, 
                           int64_t stride_ak, int64_t stride_bk, int64_t stride_bn, int64_t stride_cm,
                           int64_t stride_cn, int32_t dtype, int32_t block_m, int32_t block_n, int32_t block_k,
                           int32_t group_size_m, int32_t num_warps, int32_t num_stages, int32_t splits,
-                          int32_t grid_size, void* workspace, int64_t workspace_bytes, int32_t b_stream, void* stream) {
+                          int32_t grid_size, void* workspace, int64_t workspace_bytes, int32_t b_stream, void* stream,
+                          bool transposed_ok = false) {
   const KernelEntry* e = nullptr;
   int rc = check_common(dtype, MOEGEMM_PRECISION_IEEE, group_size_m, &e, block_m, block_n, block_k, num_warps,
                         num_stages);
   if (rc != MOEGEMM_OK) return rc;
   if (!a || !b || !c) return fail(MOEGEMM_ERR_INVALID, "matrix pointers must be non-null");
   if (m <= 0 || n <= 0 || k <= 0) return fail(MOEGEMM_ERR_INVALID, "shape must be positive (m=%d n=%d k=%d)", m, n, k);
-  if (!vector_layout_ok(a, b, c, m, n, k, stride_am, stride_ak, stride_bk, stride_bn, stride_cm, stride_cn, dtype) ||
-      !e->launch_fast)
+  const int layout = fast_layout(a, b, c, m, n, k, stride_am, stride_ak, stride_bk, stride_bn, stride_cm, stride_cn,
+                                 dtype);
+  if (layout < 0 || (layout > 0 && (!transposed_ok || !e->launch_transposed_split[layout - 1])) || !e->launch_fast)
     return fail(MOEGEMM_ERR_INVALID, "split-K needs fp16/bf16 operands in the vector layout");
   const int64_t tiles = cdiv(m, block_m) * cdiv(n, block_n);
   KParams p;
@@ -432,7 +475,7 @@ static int matmul_splitk_impl(const void* a, const void* b, void* c, int32_t m, 
   if (rc != MOEGEMM_OK) return rc;
   const int64_t units = (int64_t)p.total_tiles * p.splits;
   const int grid = grid_size <= 0 || grid_size > units ? (int)units : grid_size;
-  return launch(e, p, grid, true, b_stream, stream);
+  return launch(e, p, grid, layout, b_stream, stream);
 }
 
 int moegemm_matmul_splitk(const void* a, const void* b, void* c, int32_t m, int32_t n, int32_t k, int64_t stride_am,
@@ -443,6 +486,28 @@ int moegemm_matmul_splitk(const void* a, const void* b, void* c, int32_t m, int3
   return matmul_splitk_impl(a, b, c, m, n, k, stride_am, stride_ak, stride_bk, stride_bn, stride_cm, stride_cn, dtype,
                             block_m, block_n, block_k, group_size_m, num_warps, num_stages, splits, grid_size,
                             workspace, workspace_bytes, b_stream, stream);
+}
+
+int moegemm_matmul_splitk_transposed(const void* a, const void* b, void* c, int32_t m, int32_t n, int32_t k,
+                                     int64_t stride_am, int64_t stride_ak, int64_t stride_bk, int64_t stride_bn,
+                                     int64_t stride_cm, int64_t stride_cn, int32_t dtype, int32_t block_m,
+                                     int32_t block_n, int32_t block_k, int32_t group_size_m, int32_t num_warps,
+                                     int32_t num_stages, int32_t splits, int32_t grid_size, void* workspace,
+                                     int64_t workspace_bytes, int32_t b_stream, void* stream) {
+  return matmul_splitk_impl(a, b, c, m, n, k, stride_am, stride_ak, stride_bk, stride_bn, stride_cm, stride_cn, dtype,
+                            block_m, block_n, block_k, group_size_m, num_warps, num_stages, splits, grid_size,
+                            workspace, workspace_bytes, b_stream, stream, true);
+}
+
+int moegemm_kernel_layouts(int dtype, int index) {
+  int count = 0;
+  const KernelEntry* t = table_for(dtype, &count);
+  if (!t || index < 0 || index >= count)
+    return fail(MOEGEMM_ERR_INVALID, "kernel index %d out of range for dtype %d", index, dtype);
+  int mask = t[index].launch_fast ? 1 : 0;
+  for (int layout = 1; layout <= 3; ++layout)
+    if (t[index].launch_transposed[layout - 1]) mask |= 1 << layout;
+  return mask;
 }
 
 int moegemm_matmul_splitk_noalloc(const void* a, const void* b, void* c, int32_t m, int32_t n, int32_t k,
@@ -504,7 +569,7 @@ int moegemm_grouped_gemm_splitk(const int64_t* a_ptrs, const int64_t* b_ptrs, co
   if (rc != MOEGEMM_OK) return rc;
   const int64_t units = (int64_t)p.total_tiles * p.splits;
   const int grid = grid_size <= 0 || grid_size > units ? (int)units : grid_size;
-  return launch(e, p, grid, true, b_stream, stream);
+  return launch(e, p, grid, 0, b_stream, stream);
 }
 
 int moegemm_streamk_workspace_bytes(int32_t tail_tiles, int32_t grid_size, int32_t block_m, int32_t block_n,
@@ -551,7 +616,7 @@ int moegemm_matmul_streamk(const void* a, const void* b, void* c, int32_t m, int
   p.group_m = group_size_m;
   rc = setup_streamk(p, tiles, k, tail_tiles, grid_size, block_m, block_n, block_k, workspace, workspace_bytes);
   if (rc != MOEGEMM_OK) return rc;
-  return launch(e, p, grid_size, true, b_stream, stream);
+  return launch(e, p, grid_size, 0, b_stream, stream);
 }
 
 int moegemm_grouped_gemm_streamk(const int64_t* a_ptrs, const int64_t* b_ptrs, const int64_t* c_ptrs,
@@ -585,7 +650,7 @@ int moegemm_grouped_gemm_streamk(const int64_t* a_ptrs, const int64_t* b_ptrs, c
   p.group_m = group_size_m;
   rc = setup_streamk(p, tiles, k, tail_tiles, grid_size, block_m, block_n, block_k, workspace, workspace_bytes);
   if (rc != MOEGEMM_OK) return rc;
-  return launch(e, p, grid_size, true, b_stream, stream);
+  return launch(e, p, grid_size, 0, b_stream, stream);
 }
 
 int moegemm_kernel_swiglu(int dtype, int index) {
@@ -658,7 +723,7 @@ static int offsets_impl(const void* a, const void* b, void* c, const int32_t* of
     return fail(MOEGEMM_ERR_INVALID, "the SwiGLU epilogue needs the vector layout (LDS-DMA kernel)");
   rc = set_queue(p, queue);
   if (rc != MOEGEMM_OK) return rc;
-  return launch(e, p, grid, vec, b_stream, stream);
+  return launch(e, p, grid, vec ? 0 : kGeneral, b_stream, stream);
 }
 
 int moegemm_grouped_mm_offs(const void* a, const void* b, void* c, const int32_t* offs, int32_t group_count,
@@ -725,8 +790,8 @@ int moegemm_matmul(const void* a, const void* b, void* c, int32_t m, int32_t n, 
   p.tf32 = input_precision == MOEGEMM_PRECISION_TF32;
   p.total_tiles = (int32_t)tiles;
   int grid = grid_size <= 0 ? p.total_tiles : (grid_size < p.total_tiles ? grid_size : p.total_tiles);
-  return launch(e, p, grid, vector_layout_ok(a, b, c, m, n, k, stride_am, stride_ak, stride_bk, stride_bn, stride_cm,
-                                           stride_cn, dtype), b_stream, stream);
+  return launch(e, p, grid, fast_layout(a, b, c, m, n, k, stride_am, stride_ak, stride_bk, stride_bn, stride_cm,
+                                        stride_cn, dtype), b_stream, stream);
 }
 
 }  // extern "C"

@@ -120,9 +120,21 @@ __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <class E, int BM_, int BN_, int BK_, int WM_, int WN_, int STAGES_>
+// LAY: operand layouts (OperandLayout).  A operand panels are K-contiguous (row-major A) or, with
+// kAT, M-contiguous (A is the transposed view of a row-major [K, M] matrix); B panels are
+// N-contiguous (row-major B) or, with kBT, K-contiguous (a linear layer's [N, K] weight).  Whichever
+// operand it is, a K-contiguous panel lives in LDS as [BX][BK] and is read with ds_read_b128, an
+// X-contiguous one as [BK][BX] and is read with the transpose load, so no layout costs an extra
+// pass or a register shuffle: only the copy addresses and the fragment reads differ.  Bound as the
+// row-major tiles are (HBM at few rows, matrix cores otherwise); the general kernel, which took such
+// operands before, was bound by its 2-byte gathers.  Measured (bf16, tuned, before -> after):
+// [16,4096]@[4096,14336] with B stored [N, K] 110 -> 24 us (4.9 TB/s); dC B^T and A^T dC of
+// [1024,4096]@[4096,3584] together 253 -> 63 us (957 TFLOP/s).
+template <class E, int BM_, int BN_, int BK_, int WM_, int WN_, int STAGES_, int LAY_ = 0>
 struct FastTile {
   static_assert(!E::is_f32, "the DMA fast path is for 16-bit operands");
+  static constexpr int LAY = LAY_;
+  static constexpr bool AT = (LAY & kAT) != 0, BT = (LAY & kBT) != 0;
   static constexpr int BM = BM_, BN = BN_, BK = BK_, WM = WM_, WN = WN_, STAGES = STAGES_;
   static constexpr int ES = 2;  // element size in bytes
   static constexpr int NW = WM * WN;
@@ -135,8 +147,8 @@ struct FastTile {
   static constexpr int FM = WTM / MI;
   static constexpr int FN = WTN / MI;
   static constexpr int ACC = MI * MI / 64;
-  static constexpr int CA = BK / 8;  // 16-byte chunks per A row
-  static constexpr int CB = BN / 8;  // 16-byte chunks per B row
+  static constexpr int CA = (AT ? BM : BK) / 8;  // 16-byte chunks per A row in LDS
+  static constexpr int CB = (BT ? BK : BN) / 8;  // 16-byte chunks per B row in LDS
   static constexpr int A_BYTES = BM * BK * 2;
   static constexpr int B_BYTES = BK * BN * 2;
   static constexpr int STAGE_BYTES = A_BYTES + B_BYTES;
@@ -148,9 +160,10 @@ struct FastTile {
   static constexpr int RPA = 64 / CA;             // A rows per issue
   static constexpr int RPB = 64 / CB;             // B rows per issue
   static constexpr int CPW = WTN / 8;             // B chunks per wave column block
-  static constexpr bool SWIGLU_OK = FN % 2 == 0;  // gate and up fragments pair up inside a wave
+  static constexpr bool SWIGLU_OK = FN % 2 == 0 && LAY == 0;  // gate and up fragments pair up inside a wave
   // Staged C epilogue: 16-bit rows of ROWB bytes, whole rows per 1 KiB slot, and the wave's
   // sub-tile fits the slots it owns (XMIN per stage when every wave issues the same copies).
+  static constexpr int FRAG_READS = (AT ? 2 : 1) * FM + (BT ? 1 : 2) * FN;  // LDS reads per K step
   static constexpr int ROWB = WTN * 2;
   static constexpr int ROW_CHUNKS = ROWB / 16;
   static constexpr bool STAGED_OK = IA % NW == 0 && IB % NW == 0 && ROWB >= 32 && 1024 % ROWB == 0 &&
@@ -166,7 +179,7 @@ struct FastTile {
   static_assert(STAGES >= 2, "need at least double buffering");
   static_assert(A_BYTES % 1024 == 0 && B_BYTES % 1024 == 0, "stages must be whole 1 KiB DMA issues");
   static_assert(CA <= 64 && CB <= 64 && 64 % CA == 0 && 64 % CB == 0, "rows must tile a 1 KiB issue");
-  static_assert(CB >= 4, "transpose reads need at least 32 columns");
+  static_assert((BT || CB >= 4) && (!AT || CA >= 4), "transpose reads need at least 32 columns");
   static_assert(WTM % MI == 0 && WTN % MI == 0 && BK % MIK == 0, "tile shape");
   static_assert(STAGES * (QA + QB) < 64, "vmcnt budget: every copy in flight must fit the 6-bit counter");
   static_assert(LDS_BYTES <= 160 * 1024, "LDS budget of one CU");
@@ -176,23 +189,32 @@ struct FastTile {
   struct Dma {
     u32x4_t ra, rb;
     uint32_t a_off[QA];  // byte offset at k0 = 0, or kOutOfRange
-    uint32_t a_kch[QA];  // k index of the lane's chunk at k0 = 0
+    uint32_t a_kch[QA];  // k index of the lane's chunk at k0 = 0 (K-contiguous panels)
     uint32_t b_off[QB];
+    uint32_t b_kch[BT ? QB : 1];
     int32_t k;
-    uint32_t ldb_bytes;
+    uint32_t lda_bytes;  // bytes between K rows of an M-contiguous A
+    uint32_t ldb_bytes;  // bytes between rows of B as stored
     uint32_t lds_wave;   // LDS byte address of this wave's first 1 KiB slot in stage 0
     int32_t b_stream;    // B copies non-temporal (ProblemDesc::b_stream)
   };
 
   __device__ static __forceinline__ void setup_dma(Dma& d, const ProblemDesc& pd, int m0, int n0, const char* smem) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint32_t lda_bytes = (uint32_t)pd.sam * 2u;
-    d.ldb_bytes = (uint32_t)pd.sbk * 2u;
+    const uint32_t lda_bytes = (uint32_t)(AT ? pd.sak : pd.sam) * 2u;
+    d.ldb_bytes = (uint32_t)(BT ? pd.sbn : pd.sbk) * 2u;
     d.k = pd.k;
     d.b_stream = pd.b_stream;
-    const int rows = min(BM, pd.m - m0);
-    d.ra = make_rsrc(pd.a + (int64_t)m0 * lda_bytes, (uint32_t)rows * lda_bytes);
-    if (pd.swiglu)
+    if constexpr (AT) {
+      d.lda_bytes = lda_bytes;
+      d.ra = make_rsrc(pd.a + (int64_t)m0 * 2, (uint32_t)pd.k * lda_bytes - (uint32_t)m0 * 2u);
+    } else {
+      const int rows = min(BM, pd.m - m0);
+      d.ra = make_rsrc(pd.a + (int64_t)m0 * lda_bytes, (uint32_t)rows * lda_bytes);
+    }
+    if constexpr (BT)
+      d.rb = make_rsrc(pd.b + (int64_t)n0 * d.ldb_bytes, (uint32_t)min(BN, pd.n - n0) * d.ldb_bytes);
+    else if (pd.swiglu)
       d.rb = make_rsrc(pd.b, (uint32_t)pd.k * d.ldb_bytes);
     else
       d.rb = make_rsrc(pd.b + (int64_t)n0 * 2, (uint32_t)pd.k * d.ldb_bytes - (uint32_t)n0 * 2u);
@@ -202,15 +224,26 @@ struct FastTile {
       const int j = wave + q * NW;
       const int r = j * RPA + lane / CA;
       const int pc = lane % CA;
-      const int c = pc ^ swz_a(r, CA);
-      d.a_kch[q] = (uint32_t)(c * 8);
-      d.a_off[q] = (uint32_t)r * lda_bytes + (uint32_t)c * 16u;
+      if constexpr (AT) {
+        const int c = pc ^ swz_b(r, CA);
+        d.a_off[q] = (m0 + c * 8 < pd.m) ? (uint32_t)r * lda_bytes + (uint32_t)c * 16u : kOutOfRange;
+      } else {
+        const int c = pc ^ swz_a(r, CA);
+        d.a_kch[q] = (uint32_t)(c * 8);
+        d.a_off[q] = (uint32_t)r * lda_bytes + (uint32_t)c * 16u;
+      }
     }
 #pragma unroll
     for (int q = 0; q < QB; ++q) {
       const int j = wave + q * NW;
       const int r = j * RPB + lane / CB;
       const int pc = lane % CB;
+      if constexpr (BT) {
+        const int c = pc ^ swz_a(r, CB);
+        d.b_kch[q] = (uint32_t)(c * 8);
+        d.b_off[q] = (uint32_t)r * d.ldb_bytes + (uint32_t)c * 16u;
+        continue;
+      }
       const int c = pc ^ swz_b(r, CB);
       if (pd.swiglu) {
         // Logical chunk c of the tile: the first half of the row holds the gate columns of output
@@ -237,11 +270,15 @@ struct FastTile {
     for (int q = 0; q < QA; ++q) {
       const int j = wave + q * NW;
       if (IA % NW == 0 || j < IA) {
-        const uint32_t off = ((int)d.a_kch[q] + k0 < d.k) ? d.a_off[q] + (uint32_t)k0 * 2u : kOutOfRange;
+        uint32_t off;
+        if constexpr (AT)
+          off = d.a_off[q] == kOutOfRange ? kOutOfRange : d.a_off[q] + (uint32_t)k0 * d.lda_bytes;
+        else
+          off = ((int)d.a_kch[q] + k0 < d.k) ? d.a_off[q] + (uint32_t)k0 * 2u : kOutOfRange;
         dma_copy16(d.ra, off, base + (uint32_t)(q * NW * 1024));
       }
     }
-    const uint32_t kstep = (uint32_t)k0 * d.ldb_bytes;
+    const uint32_t kstep = BT ? (uint32_t)k0 : (uint32_t)k0 * d.ldb_bytes;
     if constexpr (NTB >= 0)
       issue_b<NTB == 1>(d, base, kstep, wave);
     else if (d.b_stream)
@@ -250,13 +287,18 @@ struct FastTile {
       issue_b<false>(d, base, kstep, wave);
   }
 
+  // `kstep`: the slice's first k (K-contiguous B), or the byte offset of its first row.
   template <bool NT>
   __device__ static __forceinline__ void issue_b(const Dma& d, uint32_t base, uint32_t kstep, int wave) {
 #pragma unroll
     for (int q = 0; q < QB; ++q) {
       const int j = wave + q * NW;
       if (IB % NW == 0 || j < IB) {
-        const uint32_t off = d.b_off[q] == kOutOfRange ? kOutOfRange : d.b_off[q] + kstep;
+        uint32_t off;
+        if constexpr (BT)
+          off = (int)(d.b_kch[q] + kstep) < d.k ? d.b_off[q] + kstep * 2u : kOutOfRange;
+        else
+          off = d.b_off[q] == kOutOfRange ? kOutOfRange : d.b_off[q] + kstep;
         if constexpr (NT)
           dma_copy16_nt(d.rb, off, base + (uint32_t)(A_BYTES + q * NW * 1024));
         else
@@ -273,34 +315,51 @@ struct FastTile {
     return wave_n * WTN + fn * MI;
   }
 
+  // This lane's fragment of K step kk for panel rows x0 .. x0 + MI - 1, from a K-contiguous panel
+  // ([BX][BK], `chunks` 16-byte chunks per row) ...
+  __device__ static __forceinline__ i16x8_t frag_rows(const char* lds, int chunks, int x0, int kk) {
+    const int lane = threadIdx.x & 63;
+    const int row = x0 + (lane % MI);
+    const int c = (kk * MIK) / 8 + lane / MI;
+    const int pc = c ^ swz_a(row, chunks);
+    return *reinterpret_cast<const i16x8_t*>(lds + (row * chunks + pc) * 16);
+  }
+  // ... or from an X-contiguous one ([BK][BX]), K-packed by the transpose load.
+  __device__ static __forceinline__ i16x8_t frag_transposed(const char* lds, int chunks, int x0, int kk) {
+    const int lane = threadIdx.x & 63;
+    const int g = lane >> 4, s = lane & 15;
+    int row, col;
+    if constexpr (MI == 32) {
+      row = kk * MIK + 8 * (g >> 1) + (s >> 2);
+      col = x0 + 16 * (g & 1) + 4 * (s & 3);
+    } else {
+      row = kk * MIK + 8 * g + (s >> 2);
+      col = x0 + 4 * (s & 3);
+    }
+    const int pc = (col >> 3) ^ swz_b(row, chunks);
+    const char* p0 = lds + (row * chunks + pc) * 16 + (col & 7) * 2;
+    const char* p1 = p0 + 4 * chunks * 16;
+    i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(p0));
+    i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(p1));
+    return i16x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  }
+
   __device__ static __forceinline__ void load_frags(i16x8_t (&af)[FM], i16x8_t (&bf)[FN], const char* lds_a,
                                                     const char* lds_b, int kk, int wave_m, int wave_n,
                                                     bool swiglu = false) {
-    const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int fm = 0; fm < FM; ++fm) {
-      const int row = wave_m * WTM + fm * MI + (lane % MI);
-      const int c = (kk * MIK) / 8 + lane / MI;
-      const int pc = c ^ swz_a(row, CA);
-      af[fm] = *reinterpret_cast<const i16x8_t*>(lds_a + (row * CA + pc) * 16);
+      if constexpr (AT)
+        af[fm] = frag_transposed(lds_a, CA, wave_m * WTM + fm * MI, kk);
+      else
+        af[fm] = frag_rows(lds_a, CA, wave_m * WTM + fm * MI, kk);
     }
 #pragma unroll
     for (int fn = 0; fn < FN; ++fn) {
-      const int g = lane >> 4, s = lane & 15;
-      int row, col;
-      if constexpr (MI == 32) {
-        row = kk * MIK + 8 * (g >> 1) + (s >> 2);
-        col = b_frag_col(fn, wave_n, swiglu) + 16 * (g & 1) + 4 * (s & 3);
-      } else {
-        row = kk * MIK + 8 * g + (s >> 2);
-        col = b_frag_col(fn, wave_n, swiglu) + 4 * (s & 3);
-      }
-      const int pc = (col >> 3) ^ swz_b(row, CB);
-      const char* p0 = lds_b + (row * CB + pc) * 16 + (col & 7) * 2;
-      const char* p1 = p0 + 4 * CB * 16;
-      i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(p0));
-      i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(p1));
-      bf[fn] = i16x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      if constexpr (BT)
+        bf[fn] = frag_rows(lds_b, CB, wave_n * WTN + fn * MI, kk);
+      else
+        bf[fn] = frag_transposed(lds_b, CB, b_frag_col(fn, wave_n, swiglu), kk);
     }
   }
 
@@ -702,7 +761,7 @@ struct FastTile {
                                                   Hook&& before_store) {
     static_assert(KK % 2 == 0, "fragment double buffer alternates by K step");
     constexpr int HALF = FM / 2 > 0 ? FM / 2 : 1;  // fragment rows issued before the mid-slice barrier
-    constexpr int NDS = FM + 2 * FN;                 // LDS reads per K step
+    constexpr int NDS = FRAG_READS;                  // LDS reads per K step
     constexpr int NVM = QA + QB;                      // DMA issues per slice (upper bound per wave)
     const int wave = threadIdx.x >> 6;
     const int wave_m = wave / WN, wave_n = wave % WN;
@@ -902,7 +961,7 @@ struct FastTile {
     static_assert(KK % 2 == 0, "fragment double buffer alternates by K step");
     constexpr int S = STAGES;
     constexpr int HALF = FM / 2 > 0 ? FM / 2 : 1;
-    constexpr int NDS = FM + 2 * FN;
+    constexpr int NDS = FRAG_READS;
     constexpr int NVM = QA + QB;
     const int wave = threadIdx.x >> 6;
     const int wave_m = wave / WN, wave_n = wave % WN;
@@ -1032,7 +1091,7 @@ struct FastTile {
     static_assert(CHAIN_OK, "the chained schedule is for two-stage and four-stage tiles");
     static_assert(KK % 2 == 0, "fragment double buffer alternates by K step");
     constexpr int HALF = FM / 2 > 0 ? FM / 2 : 1;
-    constexpr int NDS = FM + 2 * FN;
+    constexpr int NDS = FRAG_READS;
     constexpr int NVM = QA + QB;
     const int wave = threadIdx.x >> 6;
     const int wave_m = wave / WN, wave_n = wave % WN;

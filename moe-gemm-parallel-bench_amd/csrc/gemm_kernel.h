@@ -49,6 +49,8 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
 enum DType : int { DT_F16 = 0, DT_BF16 = 1, DT_F32 = 2 };
+// Operand layouts of the LDS-DMA tiles (bits): 0 is row-major A and B.
+enum OperandLayout : int { kAT = 1, kBT = 2 };  // A M-contiguous (transposed view); B K-contiguous
 enum Mode : int { MODE_SINGLE = 0, MODE_HOMOGENEOUS = 1, MODE_GENERIC = 2, MODE_OFFSETS = 3 };
 
 // Kernel arguments, passed by value.  Strides are in elements.

@@ -39,9 +39,9 @@ __device__ __forceinline__ void phase_barrier() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-template <class E, int BK_, int STAGES_>
-struct PingPongTile : FastTile<E, 256, 256, BK_, 2, 4, STAGES_> {
-  using Base = FastTile<E, 256, 256, BK_, 2, 4, STAGES_>;
+template <class E, int BK_, int STAGES_, int LAY_ = 0>
+struct PingPongTile : FastTile<E, 256, 256, BK_, 2, 4, STAGES_, LAY_> {
+  using Base = FastTile<E, 256, 256, BK_, 2, 4, STAGES_, LAY_>;
   using typename Base::acc_t;
   using typename Base::Dma;
   static constexpr int BM = Base::BM, BN = Base::BN, BK = Base::BK, STAGES = Base::STAGES;

@@ -1,0 +1,5 @@
+// Compiled bf16 kernels for transposed operands: K-contiguous B.
+#include "registry.h"
+namespace moegemm {
+MOEGEMM_MENU_BT(MOEGEMM_INST16_TR, EBf16)
+}  // namespace moegemm

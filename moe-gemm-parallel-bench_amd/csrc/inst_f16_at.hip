@@ -1,0 +1,5 @@
+// Compiled f16 kernels for transposed operands: M-contiguous A.
+#include "registry.h"
+namespace moegemm {
+MOEGEMM_MENU_AT(MOEGEMM_INST16_TR, EF16)
+}  // namespace moegemm

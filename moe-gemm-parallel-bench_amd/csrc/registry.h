@@ -24,6 +24,9 @@ struct KernelEntry {
   LaunchFn launch_general;
   LaunchFn launch_fast_split;  // the fast path's split-K kernel (null without a fast path)
   LaunchFn launch_fast_streamk;  // the fast path's stream-K kernel (null without a fast path)
+  // The fast path for transposed operands, by OperandLayout - 1 (null: not compiled for this tile).
+  LaunchFn launch_transposed[3];
+  LaunchFn launch_transposed_split[3];
 };
 
 template <class T, bool SPLIT = false, bool STREAMK = false>
@@ -36,13 +39,13 @@ hipError_t launch_tile(const KParams& p, int grid, hipStream_t stream) {
 // menu into explicit kernel instantiations (device and host passes) and into the host table.
 // The 8-wave 256x256 tiles with at least three stages run the ping-pong schedule
 // (gemm_pingpong.h); every other 16-bit vector-layout tile runs FastTile's schedule.
-template <class E, int BM, int BN, int BK, int WM, int WN, int S>
+template <class E, int BM, int BN, int BK, int WM, int WN, int S, int LAY = 0>
 struct FastTileFor {
   using type = typename std::conditional<BM == 256 && BN == 256 && WM == 2 && WN == 4 && S >= 3,
-                                         PingPongTile<E, BK, S>, FastTile<E, BM, BN, BK, WM, WN, S>>::type;
+                                         PingPongTile<E, BK, S, LAY>, FastTile<E, BM, BN, BK, WM, WN, S, LAY>>::type;
 };
-template <class E, int BM, int BN, int BK, int WM, int WN, int S>
-using FastTileT = typename FastTileFor<E, BM, BN, BK, WM, WN, S>::type;
+template <class E, int BM, int BN, int BK, int WM, int WN, int S, int LAY = 0>
+using FastTileT = typename FastTileFor<E, BM, BN, BK, WM, WN, S, LAY>::type;
 #define MOEGEMM_FAST(E, BM, BN, BK, WM, WN, S) FastTileT<E, BM, BN, BK, WM, WN, S>
 // The general kernel has no stage count; the wrapper keeps one instantiation per menu entry even
 // when two entries differ only in the fast path's stages.
@@ -65,6 +68,43 @@ struct GemmTileEntry : GemmTile<E, BM, BN, BK, WM, WN> {};
 #define MOEGEMM_EXTERN16_SK(E, BM, BN, BK, WM, WN, S)                                                          \
   extern template hipError_t launch_tile<MOEGEMM_FAST(E, BM, BN, BK, WM, WN, S), true, true>(const KParams&, int, \
                                                                                              hipStream_t);
+
+// Transposed operands (OperandLayout): the tiles a caller's shapes need there, one table for the
+// K-contiguous B of linear weights (prefill and decode tiles) and one for an M-contiguous A
+// (weight gradients: long M and N, so only large and middle tiles), alone or with a K-contiguous
+// B.  A tile outside these tables runs its general kernel on such operands.
+#define MOEGEMM_MENU_BT(X, E)                                                                            \
+  X(E, 256, 256, 32, 2, 4, 4, 2) X(E, 128, 256, 64, 2, 4, 3, 2) X(E, 128, 128, 64, 2, 2, 4, 2)           \
+  X(E, 64, 256, 64, 1, 4, 3, 2) X(E, 64, 128, 64, 2, 2, 4, 2) X(E, 64, 64, 64, 2, 2, 4, 2)               \
+  X(E, 32, 128, 64, 1, 4, 4, 2) X(E, 32, 128, 128, 1, 4, 3, 2) X(E, 16, 256, 64, 1, 4, 4, 2)             \
+  X(E, 16, 128, 128, 1, 4, 4, 2) X(E, 16, 64, 128, 1, 4, 4, 2) X(E, 16, 64, 128, 1, 4, 7, 2)
+#define MOEGEMM_MENU_AT(X, E)                                                                            \
+  X(E, 256, 256, 32, 2, 4, 4, 1) X(E, 128, 256, 64, 2, 4, 3, 1) X(E, 128, 128, 64, 2, 2, 4, 1)           \
+  X(E, 64, 128, 64, 2, 2, 4, 1) X(E, 64, 64, 64, 2, 2, 4, 1)                                             \
+  X(E, 256, 256, 32, 2, 4, 4, 3) X(E, 128, 256, 64, 2, 4, 3, 3) X(E, 128, 128, 64, 2, 2, 4, 3)           \
+  X(E, 64, 128, 64, 2, 2, 4, 3) X(E, 64, 64, 64, 2, 2, 4, 3)
+#define MOEGEMM_INST16_TR(E, BM, BN, BK, WM, WN, S, LAY)                                                     \
+  template __global__ void grouped_gemm_kernel<FastTileT<E, BM, BN, BK, WM, WN, S, LAY>, false>(KParams);    \
+  template __global__ void grouped_gemm_kernel<FastTileT<E, BM, BN, BK, WM, WN, S, LAY>, true>(KParams);     \
+  template hipError_t launch_tile<FastTileT<E, BM, BN, BK, WM, WN, S, LAY>, false>(const KParams&, int, hipStream_t); \
+  template hipError_t launch_tile<FastTileT<E, BM, BN, BK, WM, WN, S, LAY>, true>(const KParams&, int, hipStream_t);
+#define MOEGEMM_EXTERN16_TR(E, BM, BN, BK, WM, WN, S, LAY)                                                   \
+  extern template hipError_t launch_tile<FastTileT<E, BM, BN, BK, WM, WN, S, LAY>, false>(const KParams&, int, \
+                                                                                          hipStream_t);      \
+  extern template hipError_t launch_tile<FastTileT<E, BM, BN, BK, WM, WN, S, LAY>, true>(const KParams&, int, \
+                                                                                         hipStream_t);
+#define MOEGEMM_MATCH_TR(E, BM, BN, BK, WM, WN, S, LAY) \
+  || (bm == BM && bn == BN && bk == BK && wm == WM && wn == WN && s == S && lay == LAY)
+constexpr bool transposed_compiled(int bm, int bn, int bk, int wm, int wn, int s, int lay) {
+  return false MOEGEMM_MENU_BT(MOEGEMM_MATCH_TR, E) MOEGEMM_MENU_AT(MOEGEMM_MATCH_TR, E);
+}
+template <class E, int BM, int BN, int BK, int WM, int WN, int S, int LAY, bool SPLIT>
+constexpr LaunchFn transposed_launch() {
+  if constexpr (transposed_compiled(BM, BN, BK, WM, WN, S, LAY))
+    return &launch_tile<FastTileT<E, BM, BN, BK, WM, WN, S, LAY>, SPLIT>;
+  else
+    return nullptr;
+}
 #define MOEGEMM_ENTRY16(E, BM, BN, BK, WM, WN, S)                                             \
   KernelEntry{E::dtype, BM, BN, BK, (WM) * (WN), S, WM, WN,                                   \
               MOEGEMM_FAST(E, BM, BN, BK, WM, WN, S)::LDS_BYTES,                              \
@@ -72,14 +112,21 @@ struct GemmTileEntry : GemmTile<E, BM, BN, BK, WM, WN> {};
               &launch_tile<MOEGEMM_FAST(E, BM, BN, BK, WM, WN, S)>,                          \
               &launch_tile<MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S)>,                           \
               &launch_tile<MOEGEMM_FAST(E, BM, BN, BK, WM, WN, S), true>,                    \
-              &launch_tile<MOEGEMM_FAST(E, BM, BN, BK, WM, WN, S), true, true>},
+              &launch_tile<MOEGEMM_FAST(E, BM, BN, BK, WM, WN, S), true, true>,              \
+              {transposed_launch<E, BM, BN, BK, WM, WN, S, 1, false>(),                       \
+               transposed_launch<E, BM, BN, BK, WM, WN, S, 2, false>(),                       \
+               transposed_launch<E, BM, BN, BK, WM, WN, S, 3, false>()},                      \
+              {transposed_launch<E, BM, BN, BK, WM, WN, S, 1, true>(),                        \
+               transposed_launch<E, BM, BN, BK, WM, WN, S, 2, true>(),                        \
+               transposed_launch<E, BM, BN, BK, WM, WN, S, 3, true>()}},
 
 #define MOEGEMM_INST32(E, BM, BN, BK, WM, WN, S) \
   template __global__ void grouped_gemm_kernel<MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S), false>(KParams);
 #define MOEGEMM_ENTRY32(E, BM, BN, BK, WM, WN, S)                                             \
   KernelEntry{E::dtype, BM, BN, BK, (WM) * (WN), S, WM, WN,                                   \
               MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S)::LDS_BYTES, 0, nullptr,                      \
-              &launch_tile<MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S)>, nullptr, nullptr},
+              &launch_tile<MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S)>, nullptr, nullptr,            \
+              {nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}},
 
 // 16-bit menu (bf16 and f16 share it): large-M MFMA-bound tiles down to skinny-M streaming tiles.
 // STAGES is sized to the 160 KiB LDS of a CU; the 2-stage narrow tiles at the end fit two

@@ -61,6 +61,12 @@ SIGNATURES = {
         [_vp, _vp, _vp, _i32, _i32, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i32,
          _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _i64, _i32, _vp],
     ),
+    "moegemm_matmul_splitk_transposed": (
+        ctypes.c_int,
+        [_vp, _vp, _vp, _i32, _i32, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i32,
+         _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _i64, _i32, _vp],
+    ),
+    "moegemm_kernel_layouts": (ctypes.c_int, [ctypes.c_int, ctypes.c_int]),
     "moegemm_matmul_splitk_noalloc": (
         ctypes.c_int,
         [_vp, _vp, _vp, _i32, _i32, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i32,
@@ -179,6 +185,58 @@ def swiglu_tiles(dtype_code: int) -> frozenset:
     return frozenset(keys)
 
 
+# Operand layouts of the LDS-DMA kernels: 0 row-major, else these bits; GENERAL runs the general kernel.
+GENERAL = -1
+A_TRANSPOSED = 1
+B_TRANSPOSED = 2
+# vector_layout argument of the grouped launches per layout (MOEGEMM_LAYOUT_* for transposed operands).
+LAYOUT_FLAGS = {GENERAL: 0, 0: 1, 1: 0x10001, 2: 0x20001, 3: 0x30001}
+
+
+@lru_cache(maxsize=None)
+def layout_tiles(dtype_code: int, layout: int) -> frozenset:
+    """Tile keys whose LDS-DMA kernel is compiled for an operand layout."""
+    lib = library()
+    keys = set()
+    for index, row in enumerate(compiled_kernels(dtype_code)):
+        mask = lib.moegemm_kernel_layouts(dtype_code, index)
+        if mask < 0:
+            check(mask)
+        if mask >> layout & 1:
+            keys.add(tuple(row[:5]))
+    return frozenset(keys)
+
+
+_COPIED_PAST_K = 1024  # K rows past the matrix that a tile's zero slices may address
+
+
+def _operand_layout(tensor, x_dim: int) -> int:
+    """0 when one operand's rows run along K, 1 when they run along its M or N dimension ``x_dim``
+    (either way in aligned 16-byte chunks within the kernels' 32-bit offsets), else -1."""
+    extent, k = tensor.shape[x_dim], tensor.shape[1 - x_dim]
+    sx, sk = tensor.stride(x_dim), tensor.stride(1 - x_dim)
+    if tensor.data_ptr() % 16:
+        return -1
+    if sk == 1 and sx % 8 == 0 and sx >= k and k % 8 == 0 and PANEL_ROWS * sx * 2 < _TWO_GIB:
+        return 0
+    if sx == 1 and sk % 8 == 0 and sk >= extent and extent % 8 == 0 and (k + _COPIED_PAST_K) * sk * 2 < _TWO_GIB:
+        return 1
+    return -1
+
+
+def transposed_layout(a, b, c) -> int:
+    """Layout of 16-bit operands of which at least one is transposed (1, 2 or 3), else GENERAL: the
+    library's rule (api.hip fast_layout) after its row-major one."""
+    n = b.shape[1]
+    scm, scn = c.stride()
+    if scn != 1 or n % 8 or scm % 4 or scm < n or c.data_ptr() % 8 or PANEL_ROWS * scm * 2 >= _TWO_GIB:
+        return GENERAL
+    la, lb = _operand_layout(a, 0), _operand_layout(b, 1)
+    if la < 0 or lb < 0:
+        return GENERAL
+    return (A_TRANSPOSED if la == 1 else 0) | (B_TRANSPOSED if lb == 0 else 0) or GENERAL
+
+
 def splitk_workspace_bytes(tiles: int, splits: int, block_m: int, block_n: int) -> int:
     out = _i64(0)
     check(library().moegemm_splitk_workspace_bytes(tiles, splits, block_m, block_n, ctypes.byref(out)))
@@ -233,6 +291,14 @@ def _refuse_allocation_under_capture(what: str) -> None:
     if torch.cuda.is_available() and torch.cuda.is_current_stream_capturing():
         raise RuntimeError(f"the {what} for this stream does not exist yet and cannot be created during graph "
                            "capture; make the first call on this stream outside capture")
+
+
+def splitk_workspace_ready(device, stream_handle: int, nbytes: int) -> bool:
+    """Whether ``splitk_workspace`` can serve this call: held already, or not under graph capture."""
+    import torch
+
+    held = _SPLITK_WORKSPACES.get((torch.device(device).index or 0, int(stream_handle)))
+    return bool(held and held[-1].numel() >= nbytes) or not torch.cuda.is_current_stream_capturing()
 
 
 def splitk_workspace(device, stream_handle: int, nbytes: int):

@@ -36,6 +36,7 @@ from .matmul import (
     estimate_seconds,
     last_matmul_config,
     launch_matmul,
+    layout_config,
     matmul_candidate_configs,
     select_config,
 )
@@ -76,6 +77,7 @@ class GroupedWorkspace:
     # (whole tiles in exact rounds, then a stream-K tail).
     tile_schedule: str = "static"
     b_stream: int = 0  # 1: the last launch issued its B copies non-temporal
+    default_config: KernelConfig | None = None  # what select_config gave when no config was named
     swiglu_b_stream: int = 0  # the same for the last launch_gate_up_swiglu call
 
     @property
@@ -132,6 +134,7 @@ def grouped_candidate_configs(
     problem_count: int = 1,
     sm_count: int = 0,
     dtype=None,
+    tiles=None,
 ) -> tuple[KernelConfig, ...]:
     """Workload-aware tile and persistent-grid candidates (at most 36).
 
@@ -142,7 +145,8 @@ def grouped_candidate_configs(
     problem spans several M tiles (otherwise traversal order is the same).  Each kept config gets
     cta_multiplier 1, plus 2 (and 4 for skinny tiles) only when the group has more tiles than one
     grid's worth, so no two candidates launch the same grid.  A single problem dispatches to the
-    single-GEMM path, whose candidates carry cta_multiplier 1 only.
+    single-GEMM path, whose candidates carry cta_multiplier 1 only.  ``tiles`` (tile keys; all
+    compiled ones when None) bounds the choice.
     """
     if min(max_m, max_n, max_k, problem_count) <= 0:
         raise ValueError("grouped candidate dimensions and problem_count must be positive")
@@ -162,16 +166,17 @@ def grouped_candidate_configs(
     # faster than the best 16-row tile on DSV3 EP W2 at M_e = 8, though it pads more rows.
     decode = max_m <= 16
     m_cap = max(32 if decode else 16, 2 ** math.ceil(math.log2(max_m)))
-    pool = [cfg for cfg in config_pool(dtype) if cfg.block_m <= m_cap] or list(config_pool(dtype))
+    compiled = [cfg for cfg in config_pool(dtype) if tiles is None or cfg.tile_key in tiles]
+    pool = [cfg for cfg in compiled if cfg.block_m <= m_cap] or compiled
     by_tile: dict[tuple[int, int], list[KernelConfig]] = {}
     for cfg in pool:
         by_tile.setdefault((cfg.block_m, cfg.block_n), []).append(cfg)
     score = {tile: min(estimate_seconds(shapes, cfg, element_size, units, f32) for cfg in cfgs)
              for tile, cfgs in by_tile.items()}
-    tiles = sorted(by_tile, key=lambda t: (score[t], -t[0] * t[1]))
+    ranked = sorted(by_tile, key=lambda t: (score[t], -t[0] * t[1]))
     candidates: list[KernelConfig] = []
     limit = 36
-    for tile in tiles:
+    for tile in ranked:
         several_m_tiles = math.ceil(max_m / tile[0]) > 1
         variants = [cfg for cfg in by_tile[tile] if cfg.group_size_m in ((1, 8) if several_m_tiles else (8,))]
         tile_count = problem_count * math.ceil(max_m / tile[0]) * math.ceil(max_n / tile[1])
@@ -188,7 +193,7 @@ def grouped_candidate_configs(
         if len({(c.block_m, c.block_n) for c in candidates}) >= max(1, base_limit // 3) + (2 if decode else 0):
             break
     fallback = select_config(max_m, max_n, max_k, dtype)
-    if not any(c.tile_key == fallback.tile_key for c in candidates) and len(candidates) < limit:
+    if tiles is None and not any(c.tile_key == fallback.tile_key for c in candidates) and len(candidates) < limit:
         candidates.append(fallback)
     return tuple(dict.fromkeys(candidates))
 
@@ -232,7 +237,8 @@ def workspace_from_tensors(arrays_a, arrays_b, arrays_c, config: KernelConfig | 
         if tensor.device != device or tensor.dtype != dtype:
             raise ValueError("every grouped tensor must share one device and dtype")
     first_m, first_k, first_n = normalized[0]
-    config = config or select_config(first_m, first_n, first_k, dtype)
+    default_config = None if config else select_config(first_m, first_n, first_k, dtype)
+    config = config or default_config
 
     def pointer_table(arrays):
         return torch.tensor([t.data_ptr() for t in arrays], device=device, dtype=torch.int64)
@@ -255,11 +261,13 @@ def workspace_from_tensors(arrays_a, arrays_b, arrays_c, config: KernelConfig | 
     homogeneous = all(s == normalized[0] for s in normalized) and all(
         t.is_contiguous() for t in (*arrays_a, *arrays_b, *arrays_c)
     )
-    return GroupedWorkspace(
+    workspace = GroupedWorkspace(
         list(arrays_a), list(arrays_b), list(arrays_c), a_ptrs, b_ptrs, c_ptrs, dims, strides,
         normalized, config, _shape_signature(normalized), device_signature, sm_count, storage_bytes,
         homogeneous,
     )
+    workspace.default_config = default_config
+    return workspace
 
 
 def build_grouped_workspace(
@@ -327,17 +335,29 @@ def _problem_vector_ok(a, b, c) -> bool:
     )
 
 
-def _vector_layout(workspace: GroupedWorkspace, dtype_code: int) -> bool:
-    """True when every problem meets the fast kernel's layout; cached per set of tensor objects."""
+def _problem_layout(a, b, c) -> int:
+    return 0 if _problem_vector_ok(a, b, c) else _native.transposed_layout(a, b, c)
+
+
+def _group_layout(workspace: GroupedWorkspace, dtype_code: int) -> int:
+    """The one LDS-DMA layout every problem meets (0 row-major, 1 to 3 transposed), or GENERAL;
+    cached per set of tensor objects."""
     if dtype_code == _native.DTYPE_F32:
-        return False
+        return _native.GENERAL
     key = (tuple(map(id, workspace.a)), tuple(map(id, workspace.b)), tuple(map(id, workspace.c)))
     cached = getattr(workspace, "_layout_cache", None)
     if cached is not None and cached[0] == key:
         return cached[1]
-    value = all(_problem_vector_ok(a, b, c) for a, b, c in zip(workspace.a, workspace.b, workspace.c))
+    value = _problem_layout(workspace.a[0], workspace.b[0], workspace.c[0])
+    if value != _native.GENERAL and any(_problem_layout(a, b, c) != value for a, b, c in workspace.problem_tensors()):
+        value = _native.GENERAL
     workspace._layout_cache = (key, value)
     return value
+
+
+def _vector_layout(workspace: GroupedWorkspace, dtype_code: int) -> bool:
+    """True when every problem meets the fast kernel's row-major layout."""
+    return _group_layout(workspace, dtype_code) == 0
 
 
 def _check_workspace(workspace: GroupedWorkspace) -> int:
@@ -387,7 +407,7 @@ def streamk_tail_for(workspace: GroupedWorkspace, cfg: KernelConfig, dtype_code:
 
 
 def _launch_grouped_fixed(workspace: GroupedWorkspace, cfg: KernelConfig, dtype_code: int, precision: int,
-                          split_k=None, schedule: str = "static", b_stream: int = 0) -> int:
+                          split_k=None, schedule: str = "static", b_stream: int = 0, layout=None) -> int:
     """One launch; returns the K splits used.  ``schedule`` "stealing" draws the tiles from the
     work-stealing queues (unsplit launches only); ``b_stream`` 1 issues the LDS-DMA kernels' B copies
     non-temporal."""
@@ -408,8 +428,9 @@ def _launch_grouped_fixed(workspace: GroupedWorkspace, cfg: KernelConfig, dtype_
             _native.check(status)
             return 1
         schedule = "static"  # no partial last round: the static launch is the same work
-    vector = _vector_layout(workspace, dtype_code)
-    splits = _grouped_splits(workspace, cfg, dtype_code, split_k, vector)
+    if layout is None:
+        layout = _group_layout(workspace, dtype_code)
+    splits = _grouped_splits(workspace, cfg, dtype_code, split_k, layout == 0)
     if schedule == "stealing" and splits > 1:
         raise ValueError("the work-stealing schedule runs unsplit launches only (split_k must be 1)")
     if splits > 1:
@@ -436,7 +457,7 @@ def _launch_grouped_fixed(workspace: GroupedWorkspace, cfg: KernelConfig, dtype_
         workspace.problem_count, m, n, k, 1 if workspace.homogeneous else 0,
         workspace.tile_count_for(cfg), dtype_code, precision,
         cfg.block_m, cfg.block_n, cfg.block_k, cfg.group_size_m, cfg.num_warps, cfg.num_stages,
-        _grid_size(workspace, cfg), 1 if vector else 0,
+        _grid_size(workspace, cfg), _native.LAYOUT_FLAGS[layout],
     )
     if schedule == "stealing":
         queue = _native.tile_queue(workspace.a[0].device, stream)
@@ -453,8 +474,8 @@ _GROUPED_AUTOTUNE_CACHE: dict[tuple, tuple] = {}
 
 
 def _grouped_tuning_key(workspace: GroupedWorkspace, scheduler: str, dtype_code: int, precision: int, split_k,
-                        tile_schedule, b_stream=None) -> tuple:
-    return (scheduler, workspace.problem_count, workspace.max_m, workspace.max_n, workspace.max_k,
+                        tile_schedule, b_stream=None, layout=0) -> tuple:
+    return (scheduler, layout, workspace.problem_count, workspace.max_m, workspace.max_n, workspace.max_k,
             workspace.shape_signature, workspace.device_signature, workspace.sm_count, dtype_code, precision,
             split_k, tile_schedule, b_stream)
 
@@ -506,15 +527,19 @@ def launch_grouped(
     dtype_code = _check_workspace(workspace)
     precision = _native.precision_code(input_precision, dtype_code)
     scheduler = "homogeneous_persistent" if workspace.homogeneous else "generic_persistent"
+    layout = _group_layout(workspace, dtype_code)
     if autotune:
-        key = _grouped_tuning_key(workspace, scheduler, dtype_code, precision, split_k, tile_schedule, b_stream)
+        # Transposed operands run other kernels than row-major ones of the same shapes.
+        key = _grouped_tuning_key(workspace, scheduler, dtype_code, precision, split_k, tile_schedule, b_stream,
+                                  max(layout, 0))
         tuned = _GROUPED_AUTOTUNE_CACHE.get(key)
         if tuned is None:
             candidates = grouped_candidate_configs(
                 workspace.max_m, workspace.max_n, workspace.max_k,
                 problem_count=workspace.problem_count, sm_count=workspace.sm_count, dtype=workspace.a[0].dtype,
+                tiles=_native.layout_tiles(dtype_code, layout) if layout > 0 else None,
             )
-            splittable = workspace.homogeneous and _vector_layout(workspace, dtype_code)
+            splittable = workspace.homogeneous and layout == 0
             options = with_schedule_options(
                 with_split_options(candidates, workspace.tile_count_for, workspace.max_k, workspace.sm_count,
                                    split_k, splittable),
@@ -524,7 +549,7 @@ def launch_grouped(
             options = [(cfg, split, schedule, b_stream or 0) for cfg, split, schedule in options]
             # The B copy policy is timed on the finalists where it is not pinned and the LDS-DMA kernels run.
             twin = ((lambda o: (o[0], o[1], o[2], 1))
-                    if b_stream is None and _vector_layout(workspace, dtype_code) else None)
+                    if b_stream is None and layout >= 0 else None)
             tuned = _tune(options, lambda o: _launch_grouped_fixed(workspace, o[0], dtype_code, precision, *o[1:]),
                           twin=twin)
             _GROUPED_AUTOTUNE_CACHE[key] = tuned
@@ -534,7 +559,10 @@ def launch_grouped(
         stream_b = b_stream or 0
         if schedule in ("stealing", "streamk") and split_k is None:
             split_k = 1
-    workspace.split_k = _launch_grouped_fixed(workspace, cfg, dtype_code, precision, split_k, schedule, stream_b)
+        if config is None and cfg is workspace.default_config:
+            cfg = layout_config(cfg, dtype_code, layout, workspace.a[0].dtype)
+    workspace.split_k = _launch_grouped_fixed(workspace, cfg, dtype_code, precision, split_k, schedule, stream_b,
+                                              layout)
     workspace.config = cfg
     workspace.scheduler = scheduler
     workspace.b_stream = stream_b

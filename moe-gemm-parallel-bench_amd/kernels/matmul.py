@@ -89,13 +89,14 @@ _MATMUL_CONFIG_POOL: tuple[KernelConfig, ...] = config_pool()
 _MATMUL_CONFIG_POOL_F32: tuple[KernelConfig, ...] = config_pool("fp32")
 
 
-def _snap(block_m: int, block_n: int, block_k: int, dtype=None, group: int = 8) -> KernelConfig:
-    """The compiled tile nearest to a wanted (block_m, block_n, block_k), in log2 distance."""
+def _snap(block_m: int, block_n: int, block_k: int, dtype=None, group: int = 8, tiles=None) -> KernelConfig:
+    """The compiled tile nearest to a wanted (block_m, block_n, block_k), in log2 distance, among the
+    tile keys ``tiles`` (all when None)."""
     def distance(entry):
         bm, bn, bk, _, _ = entry
         return (abs(math.log2(bm / block_m)) + abs(math.log2(bn / block_n)), abs(math.log2(bk / block_k)))
 
-    bm, bn, bk, warps, stages = min(_menu(dtype), key=distance)
+    bm, bn, bk, warps, stages = min((t for t in _menu(dtype) if tiles is None or t in tiles), key=distance)
     return KernelConfig(bm, bn, bk, group, warps, stages)
 
 
@@ -198,12 +199,23 @@ def estimate_seconds(
     return max(compute, memory)
 
 
+def layout_config(cfg: KernelConfig, dtype_code: int, layout: int, dtype=None) -> KernelConfig:
+    """``cfg``, or the nearest tile compiled for transposed operands of this layout."""
+    if layout <= 0:
+        return cfg
+    tiles = _native.layout_tiles(dtype_code, layout)
+    if cfg.tile_key in tiles:
+        return cfg
+    return _snap(cfg.block_m, cfg.block_n, cfg.block_k, dtype, cfg.group_size_m, tiles)
+
+
 def matmul_candidate_configs(m: int, n: int, k: int, limit: int = 10, *, dtype=None,
-                             sm_count: int = 256) -> tuple[KernelConfig, ...]:
-    """Bounded candidate set for one [m, k] @ [k, n] shape, best predicted first."""
+                             sm_count: int = 256, tiles=None) -> tuple[KernelConfig, ...]:
+    """Bounded candidate set for one [m, k] @ [k, n] shape, best predicted first, drawn from the
+    tile keys ``tiles`` (all compiled tiles when None)."""
     f32 = _is_f32(dtype)
     element_size = 4 if f32 else 2
-    pool = config_pool(dtype)
+    pool = tuple(cfg for cfg in config_pool(dtype) if tiles is None or cfg.tile_key in tiles)
     # Shape family: drop tiles whose M or N edge is more than twice the (rounded-up) extent.
     family = [
         cfg for cfg in pool
@@ -211,7 +223,7 @@ def matmul_candidate_configs(m: int, n: int, k: int, limit: int = 10, *, dtype=N
         and cfg.block_n <= max(64, 2 ** math.ceil(math.log2(max(n, 1))))
     ] or list(pool)
     fallback = select_config(m, n, k, dtype)
-    if fallback not in family:
+    if fallback not in family and tiles is None:
         family.append(fallback)
     # The model ignores L2 reuse, so GROUP_M only breaks ties: with several M tiles the widest group
     # goes first (the M tiles that share a B panel run together; measured 10 % faster on
@@ -289,6 +301,15 @@ def _vector_ok(a, b, c) -> bool:
     )
 
 
+def _operand_layout(a, b, c) -> int:
+    """Layout of the LDS-DMA kernels these operands meet: 0 row-major, 1 to 3 transposed, GENERAL."""
+    import torch
+
+    if a.dtype not in (torch.float16, torch.bfloat16):
+        return _native.GENERAL
+    return 0 if _vector_ok(a, b, c) else _native.transposed_layout(a, b, c)
+
+
 def splitk_count(tiles: int, k: int, block_k: int, sm_count: int) -> int:
     """K splits for a launch with ``tiles`` output tiles: 1 unless the tiles leave over half the CUs
     idle; otherwise enough splits to give every CU a unit, each at least 4 K slices, at most 16."""
@@ -362,7 +383,7 @@ def _launch_fixed_splitk(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, s
     nbytes = _native.splitk_workspace_bytes(tiles, splits, cfg.block_m, cfg.block_n)
     stream = _native.current_stream_handle(a.device)
     workspace = _native.splitk_workspace(a.device, stream, nbytes)
-    status = _native.library().moegemm_matmul_splitk(
+    status = _native.library().moegemm_matmul_splitk_transposed(
         a.data_ptr(), b.data_ptr(), c.data_ptr(), m, n, k,
         a.stride(0), a.stride(1), b.stride(0), b.stride(1), c.stride(0), c.stride(1), dtype_code,
         cfg.block_m, cfg.block_n, cfg.block_k, cfg.group_size_m, cfg.num_warps, cfg.num_stages, splits,
@@ -386,10 +407,16 @@ def _launch_fixed(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, precisio
             return 1
         split_k = 1
     splits = 1
-    if _vector_ok(a, b, c):
+    layout = _operand_layout(a, b, c)
+    if layout == 0 or (layout > 0 and cfg.tile_key in _native.layout_tiles(dtype_code, layout)):
         tiles = -(-m // cfg.block_m) * -(-n // cfg.block_n)
         splits = split_k if split_k is not None else splitk_count(tiles, k, cfg.block_k,
                                                                   _device_signature(a.device) % 1000)
+        # Transposed operands take the unsplit launch where a workspace cannot be made (graph capture).
+        if splits > 1 and layout > 0 and not _native.splitk_workspace_ready(
+                a.device, _native.current_stream_handle(a.device),
+                _native.splitk_workspace_bytes(tiles, splits, cfg.block_m, cfg.block_n)):
+            splits = 1
     if splits > 1:
         _launch_fixed_splitk(a, b, c, m, n, k, cfg, dtype_code, splits, b_stream)
         return splits
@@ -434,7 +461,7 @@ def launch_matmul(
     if b_stream not in (None, 0, 1):
         raise ValueError(f"b_stream must be None, 0 or 1, got {b_stream!r}")
     if not autotune:
-        cfg = config or select_config(m, n, k, a.dtype)
+        cfg = config or layout_config(select_config(m, n, k, a.dtype), dtype_code, _operand_layout(a, b, c), a.dtype)
         _LAST_SPLIT[0] = _launch_fixed(a, b, c, m, n, k, cfg, dtype_code, precision, split_k, b_stream or 0)
         return
     key = (
@@ -444,14 +471,16 @@ def launch_matmul(
     best = _AUTOTUNE_CACHE.get(key)
     if best is None:
         sm_count = _device_signature(a.device) % 1000
-        configs = matmul_candidate_configs(m, n, k, dtype=a.dtype, sm_count=sm_count)
+        layout = _operand_layout(a, b, c)
+        tiles = _native.layout_tiles(dtype_code, layout) if layout > 0 else None
+        configs = matmul_candidate_configs(m, n, k, dtype=a.dtype, sm_count=sm_count, tiles=tiles)
         options = with_split_options(configs, lambda cfg: -(-m // cfg.block_m) * -(-n // cfg.block_n), k,
-                                     sm_count, split_k, _vector_ok(a, b, c))
+                                     sm_count, split_k, layout >= 0)
         if split_k is None:  # a stream-K tail where the tiles leave a partial last round
             options += [(cfg, STREAMK) for cfg in configs if _streamk_tail(a, b, c, m, n, k, cfg)]
         options = [(cfg, split, b_stream or 0) for cfg, split in options]
         # The B copy policy is timed on the finalists where it is not pinned and the LDS-DMA kernels run.
-        twin = (lambda o: (o[0], o[1], 1)) if b_stream is None and _vector_ok(a, b, c) else None
+        twin = (lambda o: (o[0], o[1], 1)) if b_stream is None and layout >= 0 else None
         best = _tune(options, lambda o: _launch_fixed(a, b, c, m, n, k, o[0], dtype_code, precision, o[1], o[2]),
                      twin=twin)
         _AUTOTUNE_CACHE[key] = best

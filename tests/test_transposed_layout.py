@@ -1,0 +1,134 @@
+"""Operand layouts of the LDS-DMA kernels: the Python rule against the library's, and the kernels on
+transposed operands (linear weights [N, K], backward products) against exact integer products."""
+
+from __future__ import annotations
+
+import random
+
+import pytest
+import torch
+
+from kernels import _native
+
+CODES = {torch.float16: _native.DTYPE_F16, torch.bfloat16: _native.DTYPE_BF16}
+
+
+def test_layout_rule_matches_the_library():
+    """The split-K entry checks layouts before its workspace, so operands it accepts fail on the
+    missing workspace instead, and nothing is launched."""
+    from kernels.matmul import _operand_layout
+
+    rng = random.Random(5)
+    storage = torch.empty(1 << 20, dtype=torch.bfloat16)
+    seen = set()
+    for _ in range(4000):
+        m, n, k = (rng.choice((8, 40, 64, 77, 136)) for _ in range(3))
+        k += 128  # two K ranges of the tile below, so the workspace is needed
+        views = []
+        for rows, cols in ((m, k), (k, n), (m, n)):
+            swap = rng.random() < (0.5 if cols != n or rows != m else 0.05)
+            extent = rows if swap else cols
+            pitch = extent + rng.choice((0, 0, 8, -extent % 8, 1, 4))
+            inner = 2 if rng.random() < 0.05 else 1
+            strides = (inner, pitch) if swap else (pitch, inner)
+            views.append(storage.as_strided((rows, cols), strides, rng.choice((0, 0, 8, 4, 1))))
+        a, b, c = views
+        layout = _operand_layout(a, b, c)
+        status = _native.library().moegemm_matmul_splitk_transposed(
+            a.data_ptr(), b.data_ptr(), c.data_ptr(), m, n, k, *a.stride(), *b.stride(), *c.stride(),
+            _native.DTYPE_BF16, 64, 64, 64, 8, 4, 4, 2, 0, None, 0, 0, None)
+        assert status == _native.ERR_INVALID
+        accepted = "workspace" in _native.last_error()
+        assert accepted != ("vector layout" in _native.last_error())
+        assert accepted == (layout >= 0), (layout, a.stride(), b.stride(), c.stride(), m, n, k)
+        # What the row-major entry refused before stays refused there.
+        status = _native.library().moegemm_matmul_splitk(
+            a.data_ptr(), b.data_ptr(), c.data_ptr(), m, n, k, *a.stride(), *b.stride(), *c.stride(),
+            _native.DTYPE_BF16, 64, 64, 64, 8, 4, 4, 2, 0, None, 0, 0, None)
+        assert ("workspace" in _native.last_error()) == (layout == 0)
+        seen.add(layout)
+    assert seen == {-1, 0, 1, 2, 3}
+
+
+def test_compiled_layouts_are_reported():
+    assert _native.layout_tiles(_native.DTYPE_F32, 0) == frozenset()
+    for code in CODES.values():
+        every = {tuple(row[:5]) for row in _native.compiled_kernels(code)}
+        assert _native.layout_tiles(code, 0) == every
+        for layout in (1, 2, 3):
+            assert _native.layout_tiles(code, layout) and _native.layout_tiles(code, layout) <= every
+    assert _native.library().moegemm_kernel_layouts(_native.DTYPE_BF16, 10_000) < 0
+
+
+def _operand(rows, cols, transposed, pad, dtype, gen):
+    """Integers in {-1, 0, 1} as a row-major or transposed view whose padding and neighbourhood hold
+    NaN: a copy that took anything past the operand's extents would show."""
+    shape = (cols, rows) if transposed else (rows, cols)
+    storage = torch.full((shape[0] + 16, shape[1] + pad), float("nan"), device="cuda", dtype=dtype)
+    values = torch.randint(-1, 2, shape, generator=gen, device="cuda", dtype=torch.int32).to(dtype)
+    view = storage[:shape[0], :shape[1]]
+    view.copy_(values)
+    return view.t() if transposed else view
+
+
+def _cases():
+    # (m, k, n): one chunk; partial tiles in every direction; several tiles, K past the stages and
+    # no multiple of the slice; M = 1 and odd M (rows along K), odd K (both operands along M and N).
+    for layout in (1, 2, 3):
+        for shape in ((8, 8, 8), (40, 72, 136), (264, 328, 520), (512, 1032, 256)):
+            yield layout, shape
+    yield from ((2, (1, 136, 24)), (2, (77, 264, 72)), (1, (72, 77, 136)), (1, (264, 1, 264)), (1, (8, 641, 8)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", list(CODES), ids=str)
+@pytest.mark.parametrize("layout,shape", list(_cases()))
+def test_transposed_operands_every_tile(layout, shape, dtype):
+    if not torch.cuda.is_available():
+        pytest.skip("ROCm GPU unavailable")
+    from kernels.matmul import KernelConfig, _operand_layout, last_matmul_split, launch_matmul
+
+    m, k, n = shape
+    gen = torch.Generator(device="cuda").manual_seed(m + k + n)
+    a = _operand(m, k, bool(layout & 1), 8, dtype, gen)
+    b = _operand(k, n, bool(layout & 2), 16, dtype, gen)
+    expected = (a.double() @ b.double()).to(dtype)  # exact in fp32, so rounded once either way
+    for tile in sorted(_native.layout_tiles(CODES[dtype], layout)):
+        for splits in (1, 3):
+            print(f"transposed layout={layout} shape={shape} tile={tile} splits={splits}", flush=True)
+            guard = torch.full((m + 2, n + 8), float("nan"), device="cuda", dtype=dtype)
+            c = guard[1:m + 1, :n]
+            assert _operand_layout(a, b, c) == layout
+            launch_matmul(a, b, c, KernelConfig(*tile[:3], 2, *tile[3:]), autotune=False, split_k=splits,
+                          b_stream=splits & 1)
+            torch.cuda.synchronize()
+            assert last_matmul_split() == splits
+            assert torch.equal(c, expected), (tile, splits)
+            assert torch.isnan(guard[:, n:]).all() and torch.isnan(guard[0]).all() and torch.isnan(guard[-1]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", [1, 2, 3])
+@pytest.mark.parametrize("schedule", ["static", "stealing"])
+def test_transposed_groups(layout, schedule):
+    """Unequal problems of one layout take its kernels; a group that mixes layouts stays general."""
+    if not torch.cuda.is_available():
+        pytest.skip("ROCm GPU unavailable")
+    from kernels.grouped_gemm import _group_layout, launch_grouped, workspace_from_tensors
+
+    gen = torch.Generator(device="cuda").manual_seed(layout)
+    shapes = [(72, 136, 264), (8, 264, 520), (264, 72, 136), (136, 520, 8)]
+    for mixed in (False, True):
+        a, b, c = [], [], []
+        for i, (m, k, n) in enumerate(shapes):
+            lay = 0 if mixed and i == 1 else layout
+            a.append(_operand(m, k, bool(lay & 1), 8, torch.bfloat16, gen))
+            b.append(_operand(k, n, bool(lay & 2), 8, torch.bfloat16, gen))
+            c.append(torch.full((m, n), float("nan"), device="cuda", dtype=torch.bfloat16))
+        ws = workspace_from_tensors(a, b, c)
+        assert _group_layout(ws, _native.DTYPE_BF16) == (-1 if mixed else layout)
+        print(f"transposed group layout={layout} schedule={schedule} mixed={mixed}", flush=True)
+        launch_grouped(ws, autotune=False, tile_schedule=schedule)
+        torch.cuda.synchronize()
+        for x, y, z in zip(a, b, c):
+            assert torch.equal(z, (x.double() @ y.double()).to(z.dtype))
