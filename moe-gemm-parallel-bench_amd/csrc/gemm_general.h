@@ -1,0 +1,481 @@
+// General tile of the grouped GEMM: fp32 operands, and 16-bit operands outside the LDS-DMA layouts
+// (gfx950).
+//
+// Operands whose inner dimension is contiguous, at any alignment and of any extent of at least 8,
+// run here; the rest (other strides, tiny extents) runs GemmTile's element-wise staging.
+//
+//  * Staging.  Every thread owns fixed 8-element chunks of each K slice: 16 bytes (16-bit types) or
+//    two 16-byte loads (fp32), at whatever alignment the row has (gfx950 global loads need none).
+//    One to four slices are in flight in registers while another is computed from LDS.  No load is
+//    predicated: a chunk that would pass the end of its row is loaded from the row's last 8
+//    elements, a row past the matrix from its last row, and a slice past K from the last slice, so
+//    every address stays inside the operand and the loads of a slice are the same instructions in
+//    every case.  What must read as zero (k past K) is shifted or cleared when the chunk is written
+//    to LDS, under uniform branches that only edge slices take.  Values past M or N feed only
+//    outputs that are not stored.
+//  * Layouts.  A panel whose rows run along K lives in LDS as [BX][BK], one whose rows run along M
+//    or N as [BK][BX]; fragments are read as in FastTile (gemm_fast.h).  The loop is compiled for
+//    each of the four combinations and chosen per problem, so transposed views cost nothing extra.
+//  * fp32 on the bf16 matrix cores.  v_mfma_f32_16x16x4_f32 runs at 1/16 of the bf16 rate.  An fp32
+//    value is the exact sum of three bf16 values x0 + x1 + x2 (x0 = bf16(x), x1 = bf16(x - x0),
+//    x2 = x - x0 - x1: 8 + 8 + 8 significand bits), so a product needs nine bf16 products, which
+//    are exact in the fp32 accumulation.  The six largest are computed; the three dropped ones
+//    (x1 y2, x2 y1, x2 y2) are below 2^-25 of the product, less than the rounding of one fp32
+//    addition.  TF32 operands (11 significand bits) are the exact sum of two bf16 values, and all
+//    four products are computed.  The accumulator is rounded once per 16 (32) products instead of
+//    once per product, so results are closer to the exact product than the fp32 instruction's.
+//    Chunks are split on their way into LDS, once per workgroup, into one LDS panel per part.
+//    Relative error against 64 bits, normal operands, fp32 instruction -> parts: 1.45e-7 -> 1.10e-7
+//    at K = 64, 1.51e-6 -> 1.34e-6 at K = 7168; TF32 1.34e-7 -> 0.88e-7 and 1.51e-6 -> 1.06e-6.
+//    Below K = 8 the fp32 instruction is closer and runs.
+//  * Bound and measured.  Large fp32 tiles are bound by the matrix cores and by the split's vector
+//    instructions (about 7.5 an element in IEEE mode, 7 in TF32), so the eight-wave 256x128 tile, which
+//    splits each element for twice the MFMAs of a 64-wide tile, leads: 4 x [2048,4096]@[4096,4096] runs
+//    at 190 TFLOP/s (1140 of bf16 MFMA work), TF32 at 255; the fp32 instruction's nominal peak is 157.
+//    8 x [512,2048]@[2048,1536] 458 -> 185 us; TF32 [1024,4096]@[4096,3584] 669 -> 131 us; fp16
+//    [777,2881]@[2881,1443] 148 -> 38 us (element-wise gathers before); bf16
+//    [4001,4003]@[4003,4005] runs at 814 TFLOP/s.
+//  * Range.  The split is exact and its products neither overflow nor lose their small parts while
+//    every non-zero operand lies in [2^-96, 2^60).  Each thread keeps the extremes of what it
+//    loaded; a tile that met a value outside (infinities and NaN included) is computed again by GemmTile, with the fp32
+//    instruction.
+#pragma once
+
+#include "gemm_kernel.h"
+
+namespace moegemm {
+
+typedef uint32_t u32x4_a2_t __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x4_a4_t __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x2_a2_t __attribute__((ext_vector_type(2), aligned(2)));
+
+// PARTS: bf16 panels per operand (3 = fp32 operands, 2 = TF32 operands, 1 = 16-bit operands).
+template <class E, int BM_, int BN_, int BK_, int WM_, int WN_, int PARTS_>
+struct GeneralTile {
+  using Plain = GemmTile<E, BM_, BN_, BK_, WM_, WN_>;
+  static constexpr int BM = BM_, BN = BN_, BK = BK_, WM = WM_, WN = WN_, PARTS = PARTS_;
+  static constexpr bool F32 = E::is_f32;
+  static constexpr int ES = sizeof(typename E::raw);
+  static constexpr int NW = WM * WN;
+  static constexpr int NT = NW * 64;
+  static constexpr int WTM = BM / WM, WTN = BN / WN;
+  static constexpr int MI = (WTM >= 32 && WTN >= 32) ? 32 : 16;
+  static constexpr int MIK = MI == 32 ? 16 : 32;
+  static constexpr int KK = BK / MIK;
+  static constexpr int FM = WTM / MI, FN = WTN / MI;
+  static constexpr int ACC = MI * MI / 64;
+  static constexpr int PRODUCTS = PARTS == 3 ? 6 : PARTS * PARTS;  // MFMAs per fragment pair and K step
+  static constexpr int VL = ES / 2;  // 16-byte loads per 8-element chunk
+  static constexpr int A_CHUNKS = BM * BK / 8, B_CHUNKS = BK * BN / 8;
+  static constexpr int A_PT = (A_CHUNKS + NT - 1) / NT, B_PT = (B_CHUNKS + NT - 1) / NT;
+  // Slices in flight in registers: one where a slice's MFMAs outlast a load, else two or, where a
+  // slice is small, four.
+  static constexpr int SLICE_REGS = (A_PT + B_PT) * VL * 4;
+  static constexpr int DEPTH = KK * FM * FN * PRODUCTS * (MI == 32 ? 2 : 1) >= 48 ? 1 : SLICE_REGS <= 16 ? 4 : 2;
+  static constexpr int UNROLL = DEPTH > 2 ? DEPTH : 2;  // steps per loop: LDS buffer and register set are static
+  static constexpr int A_BYTES = A_CHUNKS * 16, B_BYTES = B_CHUNKS * 16;  // one part
+  static constexpr int STAGE_BYTES = PARTS * (A_BYTES + B_BYTES);
+  static constexpr int PREFIX = Plain::PREFIX;
+  static constexpr int PREFIX_OFFSET = 2 * STAGE_BYTES > Plain::PREFIX_OFFSET ? 2 * STAGE_BYTES : Plain::PREFIX_OFFSET;
+  static constexpr int LDS_BYTES = PREFIX_OFFSET + (PREFIX + 1) * 4 + NT * 4;
+  // Tiles of four waves whose LDS fits twice run two workgroups a CU: 256 registers a wave.
+  static constexpr int WAVES_PER_EU = 2 * LDS_BYTES <= 160 * 1024 || NW == 8 ? 2 : 1;
+  static constexpr bool CHAIN_OK = false;
+  static constexpr bool CHAIN_STEALING = false;
+
+  static_assert(F32 ? PARTS >= 2 : PARTS == 1, "16-bit operands are one part, fp32 operands two or three");
+  static_assert(BK % MIK == 0 && WTM % MI == 0 && WTN % MI == 0, "tile shape");
+  static_assert(LDS_BYTES <= 160 * 1024, "LDS budget of one CU");
+
+  using acc_t = typename std::conditional<ACC == 16, f32x16_t, f32x4_t>::type;
+  using vec_t = typename std::conditional<F32, u32x4_a4_t, u32x4_a2_t>::type;
+
+  // One operand's chunks of this thread.  XC: rows run along the operand's M or N dimension x.
+  // Global addresses are a uniform base plus a 32-bit offset (the caller checked the pitch).
+  template <bool XC, int BX, int PT>
+  struct Operand {
+    static constexpr int CPR = XC ? BX / 8 : BK / 8;  // chunks per LDS row
+    static constexpr int CHUNKS = BX * BK / 8;
+    // Chunk i lies i * NT / CPR rows below chunk 0 in the same LDS column; where that keeps the row's
+    // swizzle, the chunks share one LDS address.
+    static constexpr int RSTEP = NT / CPR;
+    static constexpr bool SHARED = NT % CPR == 0 && RSTEP % (XC ? 16 : 32) == 0 && CHUNKS % NT == 0;
+    const char* base;    // row x0 (K-contiguous) or column x0 (XC) of the matrix; uniform
+    uint32_t off[PT];    // K-contiguous: offset of the chunk's row, inside the matrix; XC: of its column
+    int32_t col;         // first chunk's position along the LDS row, in elements
+    uint32_t pitch;      // bytes between K rows (XC)
+    uint32_t lds[SHARED ? 1 : PT];
+    int32_t k, x_over;   // x_over: elements of the tile's partial x chunk past the matrix (XC), 0 if none
+    int32_t x_limit;     // matrix extent along x, relative to the tile
+
+    __device__ static __forceinline__ void place(int i, int& r, int& c) {
+      int cl = (int)threadIdx.x + i * NT;
+      if (CHUNKS % NT != 0) cl = min(cl, CHUNKS - 1);
+      r = cl / CPR;
+      c = cl % CPR;
+    }
+
+    __device__ __forceinline__ void setup(const char* p, int64_t sx, int64_t sk, int x0, int extent, int32_t k_) {
+      k = k_;
+      x_limit = extent - x0;
+      x_over = XC && x_limit < BX ? (8 - (x_limit & 7)) & 7 : 0;
+      pitch = XC ? (uint32_t)(sk * ES) : 0;
+      // The last 8 columns may start before x0: the base steps back with them.
+      const int back = XC ? max(0, 8 - x_limit) : 0;
+      base = p + (XC ? (int64_t)(x0 - back) * ES : (int64_t)x0 * sx * ES);
+#pragma unroll
+      for (int i = 0; i < PT; ++i) {
+        int r, c;
+        place(i, r, c);
+        if (i == 0) col = c * 8;
+        off[i] = XC ? (uint32_t)(min(c * 8, x_limit - 8) + back) * ES
+                    : (uint32_t)min(r, x_limit - 1) * (uint32_t)(sx * ES);
+        if (!SHARED || i == 0) lds[i] = (uint32_t)(r * CPR + (c ^ (XC ? swz_b(r, CPR) : swz_a(r, CPR)))) * 16u;
+      }
+    }
+
+    // Loads of the slice that starts at k0 < k.
+    __device__ __forceinline__ void load(u32x4_t (&out)[PT][VL], int k0) const {
+      const char* from = XC ? base + (int64_t)k0 * pitch : base;
+#pragma unroll
+      for (int i = 0; i < PT; ++i) {
+        int r, c;
+        place(i, r, c);
+        const uint32_t at = XC ? off[i] + (uint32_t)min(r, k - 1 - k0) * pitch
+                               : off[i] + (uint32_t)min(k0 + (SHARED ? col : c * 8), k - 8) * (uint32_t)ES;
+#pragma unroll
+        for (int v = 0; v < VL; ++v) out[i][v] = *MOEGEMM_GLOBAL(const vec_t, from + (uint64_t)at + v * 16);
+      }
+    }
+
+    // Writes the chunks to the slice's LDS panel (PARTS of them).  EDGE false: the slice lies inside K
+    // and the tile has no partial x chunk.
+    template <bool EDGE>
+    __device__ __forceinline__ void store(u32x4_t (&in)[PT][VL], int k0, char* panel, uint32_t (&range)[2]) const {
+      const bool edge = EDGE && (k0 + BK > k || x_over != 0);  // uniform
+#pragma unroll
+      for (int i = 0; i < PT; ++i) {
+        if (edge) {
+          int r, c;
+          place(i, r, c);
+          const int over = XC ? x_over : (8 - (k & 7)) & 7;
+          const int past = XC ? c * 8 + 8 - x_limit : k0 + c * 8 + 8 - k;
+          if (past > 0 && past < 8) shift_down(in[i], over);
+          const bool clear = XC ? k0 + r >= k : past >= 8;
+          if (clear) {
+#pragma unroll
+            for (int v = 0; v < VL; ++v) in[i][v] = u32x4_t{0u, 0u, 0u, 0u};
+          }
+        }
+        u32x4_t part[PARTS];
+        split(in[i], part, range);
+        char* dst = panel + (SHARED ? lds[0] : lds[SHARED ? 0 : i]) + (SHARED ? i * RSTEP * CPR * 16 : 0);
+        if (CHUNKS % NT == 0 || (int)threadIdx.x + i * NT < CHUNKS) {
+#pragma unroll
+          for (int q = 0; q < PARTS; ++q) *reinterpret_cast<u32x4_t*>(dst + q * (BX * BK * 2)) = part[q];
+        }
+      }
+    }
+  };
+
+  // Moves a chunk's elements down by `over` (uniform, 1 to 7), zeros in at the top.
+  __device__ static __forceinline__ void shift_down(u32x4_t (&v)[VL], int over) {
+    uint32_t w[4 * VL];
+#pragma unroll
+    for (int i = 0; i < 4 * VL; ++i) w[i] = v[i / 4][i % 4];
+    const int words = F32 ? over : over >> 1;
+#pragma unroll
+    for (int bit = 4 * VL / 2; bit >= 1; bit >>= 1)
+      if (words & bit) {
+#pragma unroll
+        for (int i = 0; i < 4 * VL; ++i) w[i] = i + bit < 4 * VL ? w[(i + bit) % (4 * VL)] : 0u;
+      }
+    if (!F32 && (over & 1)) {
+#pragma unroll
+      for (int i = 0; i < 4 * VL; ++i) w[i] = (w[i] >> 16) | (i + 1 < 4 * VL ? w[(i + 1) % (4 * VL)] << 16 : 0u);
+    }
+#pragma unroll
+    for (int i = 0; i < 4 * VL; ++i) v[i / 4][i % 4] = w[i];
+  }
+
+  __device__ static __forceinline__ uint32_t pack_bf16(float x, float y) {
+    uint32_t h;  // one instruction; the compiler converts the halves one by one and merges them
+    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(h) : "v"(x), "v"(y));
+    return h;
+  }
+
+  // The chunk's bf16 parts.  range[0]: the largest |x| seen (as float bits; a NaN stays), range[1]: the
+  // smallest non-zero |x| (as twice its bits, less one: zero wraps to the top).
+  __device__ static __forceinline__ void split(const u32x4_t (&in)[VL], u32x4_t (&part)[PARTS], uint32_t (&range)[2]) {
+    if constexpr (!F32) {
+      part[0] = in[0];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        uint32_t u0 = in[(2 * i) / 4][(2 * i) % 4], u1 = in[(2 * i + 1) / 4][(2 * i + 1) % 4];
+        asm("v_maximum3_f32 %0, %0, |%1|, |%2|" : "+v"(range[0]) : "v"(u0), "v"(u1));
+        range[1] = min(min(range[1], (u0 << 1) - 1u), (u1 << 1) - 1u);
+        if constexpr (PARTS == 2) {  // TF32: 10-bit mantissa, ties away (NaN leaves by its range)
+          u0 = (u0 + 0x1000u) & 0xffffe000u;
+          u1 = (u1 + 0x1000u) & 0xffffe000u;
+        }
+        float x = __builtin_bit_cast(float, u0), y = __builtin_bit_cast(float, u1);
+#pragma unroll
+        for (int q = 0; q < PARTS; ++q) {
+          const uint32_t h = pack_bf16(x, y);
+          part[q][i] = h;
+          x -= __builtin_bit_cast(float, h << 16);
+          y -= __builtin_bit_cast(float, h & 0xffff0000u);
+        }
+      }
+    }
+  }
+  // Bits of 2^60, and twice those of 2^-96 less one.
+  static constexpr uint32_t kTooLarge = (127u + 60u) << 23;
+  static constexpr uint32_t kTooSmall = ((127u - 96u) << 24) - 1u;
+
+  // Fragments of one operand (as FastTile's frag_rows / frag_transposed): per-lane LDS offsets of the
+  // wave's first rows, to which fragment and K step add constants (the swizzles do not see them).
+  template <bool XC, int BX, int NF>
+  struct Frags {
+    static constexpr int CPR = XC ? BX / 8 : BK / 8;
+    // Fragments 16 rows apart differ in a swizzle bit when a K-contiguous row has 8 chunks.
+    static constexpr int ROWS = !XC && MI == 16 && CPR == 8 ? NF : 1;
+    uint32_t off[XC ? NF : KK * ROWS];
+
+    __device__ __forceinline__ void setup(int x0) {
+      const int lane = threadIdx.x & 63;
+      if constexpr (!XC) {
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+          for (int f = 0; f < ROWS; ++f) {
+            const int row = x0 + f * MI + (lane % MI);
+            off[kk * ROWS + f] = (uint32_t)(row * CPR + (((kk * MIK) / 8 + lane / MI) ^ swz_a(row, CPR))) * 16u;
+          }
+      } else {
+        const int g = lane >> 4, s = lane & 15;
+        const int row = MI == 32 ? 8 * (g >> 1) + (s >> 2) : 8 * g + (s >> 2);
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+          const int col = x0 + f * MI + (MI == 32 ? 16 * (g & 1) + 4 * (s & 3) : 4 * (s & 3));
+          off[f] = (uint32_t)((row * CPR + ((col >> 3) ^ swz_b(row, CPR))) * 16 + (col & 7) * 2);
+        }
+      }
+    }
+    __device__ __forceinline__ i16x8_t get(const char* panel, int f, int kk) const {
+      if constexpr (!XC) {
+        const char* p = panel + off[kk * ROWS + (ROWS > 1 ? f : 0)] + (ROWS > 1 ? 0 : f * MI * CPR * 16);
+        return *reinterpret_cast<const i16x8_t*>(p);
+      } else {
+        const char* p0 = panel + off[f] + kk * MIK * CPR * 16;
+        const char* p1 = p0 + 4 * CPR * 16;
+        i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(p0));
+        i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(p1));
+        return i16x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      }
+    }
+  };
+
+  __device__ static __forceinline__ acc_t mfma(i16x8_t b, i16x8_t a, acc_t c) {
+    if constexpr (E::dtype == DT_F16) {
+      if constexpr (MI == 32)
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, b), __builtin_bit_cast(f16x8_t, a), c, 0, 0, 0);
+      else
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, b), __builtin_bit_cast(f16x8_t, a), c, 0, 0, 0);
+    } else {
+      if constexpr (MI == 32)
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, b), __builtin_bit_cast(bf16x8_t, a), c, 0, 0, 0);
+      else
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, b), __builtin_bit_cast(bf16x8_t, a), c, 0, 0, 0);
+    }
+  }
+
+  // Fragment registers of one K step; four-wave tiles read all of a slice's fragments ahead of its MFMAs
+  // where they fit (a lone wave on its SIMD has nothing else to hide the LDS latency of each K step).
+  static constexpr int STEP_REGS = PARTS * (FM + FN) * 4;
+  static constexpr bool READ_AHEAD =
+      NW <= 4 && KK * STEP_REGS + FM * FN * ACC + DEPTH * SLICE_REGS <= (WAVES_PER_EU == 1 ? 320 : 160);
+
+  template <class FA, class FB>
+  __device__ static __forceinline__ void compute(acc_t (&acc)[FM][FN], const char* lds, const FA& fa, const FB& fb) {
+    i16x8_t af[KK][PARTS][FM], bf[KK][PARTS][FN];
+    auto read = [&](int kk) {
+#pragma unroll
+      for (int q = 0; q < PARTS; ++q) {
+#pragma unroll
+        for (int fm = 0; fm < FM; ++fm) af[kk][q][fm] = fa.get(lds + q * A_BYTES, fm, kk);
+#pragma unroll
+        for (int fn = 0; fn < FN; ++fn) bf[kk][q][fn] = fb.get(lds + PARTS * A_BYTES + q * B_BYTES, fn, kk);
+      }
+    };
+    if constexpr (READ_AHEAD) {
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) read(kk);
+      __builtin_amdgcn_sched_barrier(0x0216);  // vector, scalar, global memory and LDS writes may cross
+    }
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) {
+      if constexpr (!READ_AHEAD) read(kk);
+      // Products in falling order of the parts' sum: the small ones are added first.
+#pragma unroll
+      for (int sum = PARTS == 3 ? 2 : 2 * (PARTS - 1); sum >= 0; --sum)
+#pragma unroll
+        for (int qa = 0; qa < PARTS; ++qa) {
+          const int qb = sum - qa;
+          if (qb < 0 || qb >= PARTS) continue;
+#pragma unroll
+          for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+            for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = mfma(bf[kk][qb][fn], af[kk][qa][fm], acc[fm][fn]);
+        }
+    }
+  }
+
+  // C: four consecutive columns a lane (see GemmTile::store_tile), stored at any alignment.
+  __device__ static __forceinline__ void store_tile(const acc_t (&acc)[FM][FN], const ProblemDesc& pd, int m0, int n0,
+                                                    int wave_m, int wave_n) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int fm = 0; fm < FM; ++fm) {
+      const int gm = m0 + wave_m * WTM + fm * MI + (lane % MI);
+      if (gm >= pd.m) continue;
+      char* crow = pd.c + (int64_t)gm * pd.scm * ES;
+#pragma unroll
+      for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+        for (int q = 0; q < ACC / 4; ++q) {
+          const int gn = n0 + wave_n * WTN + fn * MI + ((MI == 32) ? (q * 8 + (lane >> 5) * 4) : ((lane >> 4) * 4));
+          const f32x4_t v = {acc[fm][fn][q * 4 + 0], acc[fm][fn][q * 4 + 1], acc[fm][fn][q * 4 + 2],
+                             acc[fm][fn][q * 4 + 3]};
+          if (pd.scn == 1 && gn + 4 <= pd.n) {
+            if constexpr (F32)
+              *MOEGEMM_GLOBAL(u32x4_a4_t, crow + (int64_t)gn * 4) = __builtin_bit_cast(u32x4_t, v);
+            else
+              *MOEGEMM_GLOBAL(u32x2_a2_t, crow + (int64_t)gn * 2) = pack4<E>(v);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (gn + e < pd.n) store1<E>(crow + (int64_t)(gn + e) * pd.scn * ES, v[e]);
+          }
+        }
+    }
+  }
+
+  // The tile with both operands in 8-element chunks; false when it must be computed by Plain.
+  template <bool AT, bool BT, class Hook>
+  __device__ static __forceinline__ bool chunk_tile(const ProblemDesc& pd, int tm, int tn, char* smem,
+                                                    Hook&& before_store) {
+    const int wave = threadIdx.x >> 6;
+    const int wave_m = wave / WN, wave_n = wave % WN;
+    const int m0 = tm * BM, n0 = tn * BN;
+    Operand<AT, BM, A_PT> a;
+    Operand<!BT, BN, B_PT> b;
+    a.setup(pd.a, pd.sam, pd.sak, m0, pd.m, pd.k);
+    b.setup(pd.b, pd.sbn, pd.sbk, n0, pd.n, pd.k);
+    Frags<AT, BM, FM> fa;
+    Frags<!BT, BN, FN> fb;
+    fa.setup(wave_m * WTM);
+    fb.setup(wave_n * WTN);
+    acc_t acc[FM][FN];
+#pragma unroll
+    for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+      for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+        for (int i = 0; i < ACC; ++i) acc[fm][fn][i] = 0.0f;
+    uint32_t range[2] = {0u, 0xffffffffu};
+
+    const int last = (pd.k + BK - 1) / BK - 1;  // last K slice
+    u32x4_t ra[DEPTH][A_PT][VL], rb[DEPTH][B_PT][VL];
+    // Register set of slice kt: kt % DEPTH; LDS buffer: kt % 2.  J: kt modulo UNROLL.
+    auto load = [&](auto j, int kt) {
+      constexpr int S = decltype(j)::value % DEPTH;
+      const int k0 = min(kt, last) * BK;
+      a.load(ra[S], k0);
+      b.load(rb[S], k0);
+    };
+    auto store = [&](auto j, auto edge, int kt) {
+      constexpr int S = decltype(j)::value % DEPTH;
+      constexpr bool EDGE = decltype(edge)::value;
+      char* lds = smem + (decltype(j)::value % 2) * STAGE_BYTES;
+      a.template store<EDGE>(ra[S], kt * BK, lds, range);
+      b.template store<EDGE>(rb[S], kt * BK, lds + PARTS * A_BYTES, range);
+    };
+    // Slice kt is computed from its LDS buffer while slice kt + 1 (in registers) goes to the other
+    // one and slices up to kt + DEPTH are in flight.  Steps whose stored slice is no edge are one
+    // basic block, so the split's vector instructions can issue between the MFMAs.
+    auto step = [&](auto j, auto edge, int kt) {
+      constexpr int J = decltype(j)::value;
+      using ahead = std::integral_constant<int, (J + DEPTH) % UNROLL>;
+      using next = std::integral_constant<int, (J + 1) % UNROLL>;
+      load(ahead{}, kt + DEPTH);
+      compute(acc, smem + (J % 2) * STAGE_BYTES, fa, fb);
+      store(next{}, edge, kt + 1);
+      __syncthreads();
+    };
+    // Steps kt .. kt + UNROLL - 1, those before `end`.
+    auto steps = [&](auto edge, int kt, int end) {
+      step(std::integral_constant<int, 0>{}, edge, kt);
+      if (!decltype(edge)::value || kt + 1 < end) step(std::integral_constant<int, 1>{}, edge, kt + 1);
+      if constexpr (UNROLL == 4) {
+        if (!decltype(edge)::value || kt + 2 < end) step(std::integral_constant<int, 2>{}, edge, kt + 2);
+        if (!decltype(edge)::value || kt + 3 < end) step(std::integral_constant<int, 3>{}, edge, kt + 3);
+      }
+    };
+    load(std::integral_constant<int, 0>{}, 0);
+    if constexpr (DEPTH >= 2) load(std::integral_constant<int, 1>{}, 1);
+    if constexpr (DEPTH == 4) {
+      load(std::integral_constant<int, 2>{}, 2);
+      load(std::integral_constant<int, 3>{}, 3);
+    }
+    store(std::integral_constant<int, 0>{}, std::true_type{}, 0);
+    __syncthreads();
+    int kt = 0;
+    if (a.x_over == 0 && b.x_over == 0) {
+      const int inner = pd.k / BK;  // whole slices
+      for (; kt + UNROLL < inner; kt += UNROLL) steps(std::false_type{}, kt, 0);
+    }
+    for (; kt < last; kt += UNROLL) steps(std::true_type{}, kt, last);
+    compute(acc, smem + (last & 1) * STAGE_BYTES, fa, fb);
+    if constexpr (F32) {
+      // Also the barrier between this tile's LDS reads and the next tile's writes.
+      if (__syncthreads_or(range[0] >= kTooLarge || range[1] < kTooSmall)) return false;
+    } else {
+      __syncthreads();
+    }
+    before_store();
+    store_tile(acc, pd, m0, n0, wave_m, wave_n);
+    return true;
+  }
+
+  template <int EPI, class Hook>
+  __device__ static __forceinline__ void run_tile(const ProblemDesc& pd, int tm, int tn, char* smem, bool tf32,
+                                                  Hook&& before_store) {
+    static_assert(EPI == EPI_C, "the general kernel has no split-K epilogue");
+    if (pd.swiglu || pd.splits > 1) return;  // LDS-DMA tiles only (the host enforces it)
+    // 32-bit offsets span a tile's rows (K-contiguous) or a slice's (XC).
+    constexpr int64_t kPitchLimit = (int64_t(1) << 32) / (BM > BN ? BM : BN) / 2;
+    const bool a_rows = pd.sak == 1 && pd.k >= 8 && pd.sam * ES < kPitchLimit && (int64_t)pd.k * ES < (1ll << 31);
+    const bool deep = !F32 || pd.k >= 8;  // shorter fp32 sums are closer with the fp32 instruction
+    const bool a_cols = deep && BM >= 32 && pd.sam == 1 && pd.m >= 8 && pd.sak * ES < kPitchLimit;
+    const bool b_rows = pd.sbk == 1 && pd.k >= 8 && pd.sbn * ES < kPitchLimit && (int64_t)pd.k * ES < (1ll << 31);
+    const bool b_cols = deep && pd.sbn == 1 && pd.n >= 8 && pd.sbk * ES < kPitchLimit;
+    bool done = false;
+    if (a_rows && b_cols) {
+      done = chunk_tile<false, false>(pd, tm, tn, smem, before_store);
+    } else if (a_rows && b_rows) {
+      done = chunk_tile<false, true>(pd, tm, tn, smem, before_store);
+    } else if (a_cols && (b_cols || b_rows)) {
+      if constexpr (BM >= 32) {
+        if (b_cols)
+          done = chunk_tile<true, false>(pd, tm, tn, smem, before_store);
+        else
+          done = chunk_tile<true, true>(pd, tm, tn, smem, before_store);
+      }
+    }
+    if (!done) Plain::template run_tile<EPI_C>(pd, tm, tn, smem, tf32, before_store);
+  }
+};
+
+}  // namespace moegemm

@@ -413,9 +413,11 @@ struct GemmTile {
   __device__ static __forceinline__ void compute_stage(acc_t (&acc)[FM][FN], const char* lds_a, const char* lds_b,
                                                        int wave_m, int wave_n) {
     const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int kk = 0; kk < BK / MIK; ++kk) {
-      if constexpr (F32) {
+    if constexpr (F32) {
+      // Unrolled by two only: fully unrolled, the eight steps' fragments took more registers than the
+      // whole of GeneralTile's loop, which shares a kernel with this one.
+#pragma unroll 2
+      for (int kk = 0; kk < BK / MIK; ++kk) {
         // v_mfma_f32_16x16x4_f32, swapped: first operand B^T (row n = lane%16, k = lane/16),
         // second operand A^T (col m = lane%16, k = lane/16).
         float af[FM], bf[FN];
@@ -439,7 +441,12 @@ struct GemmTile {
 #pragma unroll
           for (int fn = 0; fn < FN; ++fn)
             acc[fm][fn] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[fn], af[fm], acc[fm][fn], 0, 0, 0);
-      } else {
+      }
+      return;
+    }
+#pragma unroll
+    for (int kk = 0; kk < BK / MIK; ++kk) {
+      if constexpr (!F32) {
         i16x8_t af[FM], bf[FN];
 #pragma unroll
         for (int fm = 0; fm < FM; ++fm) {

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include "gemm_fast.h"
+#include "gemm_general.h"
 #include "gemm_kernel.h"
 #include "gemm_pingpong.h"
 
@@ -49,14 +50,27 @@ using FastTileT = typename FastTileFor<E, BM, BN, BK, WM, WN, S, LAY>::type;
 #define MOEGEMM_FAST(E, BM, BN, BK, WM, WN, S) FastTileT<E, BM, BN, BK, WM, WN, S>
 // The general kernel has no stage count; the wrapper keeps one instantiation per menu entry even
 // when two entries differ only in the fast path's stages.
-template <class E, int BM, int BN, int BK, int WM, int WN, int S>
-struct GemmTileEntry : GemmTile<E, BM, BN, BK, WM, WN> {};
-#define MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S) GemmTileEntry<E, BM, BN, BK, WM, WN, S>
+template <class E, int BM, int BN, int BK, int WM, int WN, int S, int PARTS>
+struct GeneralTileEntry : GeneralTile<E, BM, BN, BK, WM, WN, PARTS> {};
+#define MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S) GeneralTileEntry<E, BM, BN, BK, WM, WN, S, 1>
+#define MOEGEMM_GEN32(E, BM, BN, BK, WM, WN, S) GeneralTileEntry<E, BM, BN, BK, WM, WN, S, 3>
+#define MOEGEMM_GEN_TF32(E, BM, BN, BK, WM, WN, S) GeneralTileEntry<E, BM, BN, BK, WM, WN, S, 2>
+
+// fp32 launches: the input precision picks the kernel (three bf16 parts per operand, or TF32's two).
+template <class IEEE, class TF32>
+hipError_t launch_f32(const KParams& p, int grid, hipStream_t stream) {
+  return p.tf32 ? launch_tile<TF32>(p, grid, stream) : launch_tile<IEEE>(p, grid, stream);
+}
 
 #define MOEGEMM_INST16(E, BM, BN, BK, WM, WN, S)                                                     \
   template __global__ void grouped_gemm_kernel<MOEGEMM_FAST(E, BM, BN, BK, WM, WN, S), false>(KParams); \
-  template __global__ void grouped_gemm_kernel<MOEGEMM_FAST(E, BM, BN, BK, WM, WN, S), true>(KParams);  \
-  template __global__ void grouped_gemm_kernel<MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S), false>(KParams);
+  template __global__ void grouped_gemm_kernel<MOEGEMM_FAST(E, BM, BN, BK, WM, WN, S), true>(KParams);
+// The general kernels, in translation units of their own (inst_*_gen.hip) like the stream-K ones.
+#define MOEGEMM_INST16_GEN(E, BM, BN, BK, WM, WN, S)                                                         \
+  template __global__ void grouped_gemm_kernel<MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S), false>(KParams);       \
+  template hipError_t launch_tile<MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S)>(const KParams&, int, hipStream_t);
+#define MOEGEMM_EXTERN16_GEN(E, BM, BN, BK, WM, WN, S) \
+  extern template hipError_t launch_tile<MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S)>(const KParams&, int, hipStream_t);
 // The stream-K kernels live in translation units of their own (inst_*_sk.hip): compiled next to
 // the other kernels of a tile, their presence in the module changed the register allocation of
 // those kernels (18 of 54 moved, one from 8 to 72 bytes of scratch).  Each such unit instantiates
@@ -121,12 +135,13 @@ constexpr LaunchFn transposed_launch() {
                transposed_launch<E, BM, BN, BK, WM, WN, S, 3, true>()}},
 
 #define MOEGEMM_INST32(E, BM, BN, BK, WM, WN, S) \
-  template __global__ void grouped_gemm_kernel<MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S), false>(KParams);
+  template __global__ void grouped_gemm_kernel<MOEGEMM_GEN32(E, BM, BN, BK, WM, WN, S), false>(KParams); \
+  template __global__ void grouped_gemm_kernel<MOEGEMM_GEN_TF32(E, BM, BN, BK, WM, WN, S), false>(KParams);
 #define MOEGEMM_ENTRY32(E, BM, BN, BK, WM, WN, S)                                             \
   KernelEntry{E::dtype, BM, BN, BK, (WM) * (WN), S, WM, WN,                                   \
-              MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S)::LDS_BYTES, 0, nullptr,                      \
-              &launch_tile<MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S)>, nullptr, nullptr,            \
-              {nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}},
+              MOEGEMM_GEN32(E, BM, BN, BK, WM, WN, S)::LDS_BYTES, 0, nullptr,                    \
+              &launch_f32<MOEGEMM_GEN32(E, BM, BN, BK, WM, WN, S), MOEGEMM_GEN_TF32(E, BM, BN, BK, WM, WN, S)>, \
+              nullptr, nullptr, {nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}},
 
 // 16-bit menu (bf16 and f16 share it): large-M MFMA-bound tiles down to skinny-M streaming tiles.
 // STAGES is sized to the 160 KiB LDS of a CU; the 2-stage narrow tiles at the end fit two
@@ -145,9 +160,9 @@ constexpr LaunchFn transposed_launch() {
   X(E, 16, 128, 64, 1, 4, 2) X(E, 16, 512, 64, 1, 4, 2) X(E, 64, 512, 64, 1, 4, 2)        \
   X(E, 32, 512, 32, 1, 4, 4)
 
-// fp32 menu (general kernel, v_mfma_f32_16x16x4_f32); STAGES is the register-staged double buffer.
+// fp32 menu (general kernel); STAGES is the register-staged double buffer.
 #define MOEGEMM_MENU_F32(X, E)                                                               \
-  X(E, 128, 128, 32, 2, 2, 2) X(E, 64, 64, 32, 2, 2, 2) X(E, 32, 64, 32, 1, 4, 2)            \
+  X(E, 256, 128, 32, 4, 2, 2) X(E, 128, 128, 32, 2, 4, 2) X(E, 128, 128, 32, 2, 2, 2) X(E, 64, 64, 32, 2, 2, 2) X(E, 32, 64, 32, 1, 4, 2)            \
   X(E, 16, 64, 32, 1, 4, 2) X(E, 32, 32, 32, 1, 2, 2)
 
 extern const KernelEntry kEntriesBf16[];

@@ -58,7 +58,7 @@ _MENU_16BIT: tuple[tuple[int, int, int, int, int], ...] = (
     (32, 512, 32, 4, 4),
 )
 _MENU_F32: tuple[tuple[int, int, int, int, int], ...] = (
-    (128, 128, 32, 4, 2), (64, 64, 32, 4, 2), (32, 64, 32, 4, 2),
+    (256, 128, 32, 8, 2), (128, 128, 32, 8, 2), (128, 128, 32, 4, 2), (64, 64, 32, 4, 2), (32, 64, 32, 4, 2),
     (16, 64, 32, 4, 2), (32, 32, 32, 2, 2),
 )
 _GROUP_SIZES = (1, 4, 8)

@@ -1,0 +1,119 @@
+"""The general tile (fp32 products from bf16 parts, 16-bit operands at any alignment) on the GPU."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = (torch.float32, torch.bfloat16, torch.float16)
+
+
+@pytest.fixture(autouse=True)
+def _gpu_only():
+    if not torch.cuda.is_available():
+        pytest.skip("ROCm GPU unavailable")
+
+
+def _tiles(dtype):
+    from kernels.matmul import KernelConfig, _menu
+
+    return [KernelConfig(bm, bn, bk, 2, warps, stages) for bm, bn, bk, warps, stages in _menu(dtype)]
+
+
+def _view(rows, cols, transposed, offset, pad, dtype, gen):
+    """Integers in {-2 .. 2} as a view at an odd offset and pitch, surrounded by NaN."""
+    shape = (cols, rows) if transposed else (rows, cols)
+    pitch = shape[1] + pad
+    storage = torch.full((offset + shape[0] * pitch + 64,), float("nan"), device="cuda", dtype=dtype)
+    view = storage[offset:offset + shape[0] * pitch].view(shape[0], pitch)[:, :shape[1]]
+    view.copy_(torch.randint(-2, 3, shape, generator=gen, device="cuda", dtype=torch.int32))
+    return view.t() if transposed else view
+
+
+# (m, k, n): below one chunk, one chunk, odd remainders of chunk, slice and tile, several slices.
+SHAPES = ((1, 1, 1), (3, 7, 5), (8, 8, 8), (9, 15, 17), (33, 65, 31), (70, 129, 67), (257, 323, 261), (16, 1001, 130))
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("transposed", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_every_tile_any_alignment(shape, transposed, dtype):
+    from kernels.matmul import launch_matmul
+
+    m, k, n = shape
+    gen = torch.Generator(device="cuda").manual_seed(m * k + n)
+    a = _view(m, k, transposed[0], 1, 3, dtype, gen)
+    b = _view(k, n, transposed[1], 3, 1, dtype, gen)
+    expected = (a.double() @ b.double()).to(dtype)  # exact in fp32, so rounded once either way
+    for cfg in _tiles(dtype):
+        print(f"general tile {cfg.tile_key} shape={shape} transposed={transposed} {dtype}", flush=True)
+        guard = torch.full((m + 2, n + 5), float("nan"), device="cuda", dtype=dtype)
+        c = guard[1:m + 1, 3:n + 3]
+        launch_matmul(a, b, c, cfg, "tf32", autotune=False)  # these integers are TF32 values
+        if dtype == torch.float32:
+            torch.cuda.synchronize()
+            assert torch.equal(c, expected), (cfg, "tf32")
+            c.fill_(float("nan"))
+            launch_matmul(a, b, c, cfg, autotune=False)
+        torch.cuda.synchronize()
+        assert torch.equal(c, expected), cfg
+        assert int(torch.isnan(guard).sum()) == guard.numel() - m * n
+
+
+@pytest.mark.parametrize("precision", ["ieee", "tf32"])
+@pytest.mark.parametrize("k", [8, 33, 256, 4096])
+@pytest.mark.parametrize("scale", [1.0, 2.0**-45, 2.0**50])
+def test_fp32_error_is_the_rounding_of_its_sums(precision, k, scale):
+    """Against 64 bits: K fp32 additions of a random walk leave about sqrt(K / 2) x 2^-25 of the result's
+    norm; the parts' products are rounded into the sum at most as often, so twice that bounds them,
+    plus the dropped products of parts (2^-25) and the store's rounding (2^-25)."""
+    from kernels.matmul import launch_matmul
+
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    a = torch.randn((130, k), device="cuda", generator=gen) * scale
+    b = torch.randn((k, 129), device="cuda", generator=gen) * scale
+    x, y = a, b
+    if precision == "tf32":
+        x, y = (((t.view(torch.int32) + 0x1000) & -0x2000).view(torch.float32) for t in (a, b))
+    expected = x.double() @ y.double()
+    bound = (2 * (k / 2) ** 0.5 + 2) * 2.0**-25
+    for cfg in _tiles(torch.float32):
+        c = torch.empty((130, 129), device="cuda")
+        print(f"fp32 error {cfg.tile_key} {precision} k={k} scale={scale}", flush=True)
+        launch_matmul(a, b, c, cfg, precision, autotune=False)
+        torch.cuda.synchronize()
+        error = float((c.double() - expected).norm() / expected.norm())
+        assert error <= bound, (cfg, error, bound)
+
+
+@pytest.mark.parametrize("precision", ["ieee", "tf32"])
+def test_fp32_values_outside_the_split_range(precision):
+    """Infinities, NaN, values near the largest and denormal ones: what a plain fp32 product gives."""
+    from kernels.matmul import launch_matmul
+
+    m, k, n = 150, 72, 140
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    base_a = torch.randint(-2, 3, (m, k), generator=gen, device="cuda").float()
+    base_b = torch.randint(1, 3, (k, n), generator=gen, device="cuda").float()
+    nan_bits = torch.tensor([-1, 0x7fffffff], dtype=torch.int32).view(torch.float32)
+    cases = [(float("inf"), 1.0), (float("-inf"), 1.0), (float("nan"), 1.0), (float(2.0**120), 1.0),
+             (float(2.0**-120), 2.0**-100), (2.0**-140, 2.0**100), (nan_bits[0], 1.0), (nan_bits[1], 1.0)]
+    for value, scale in cases:
+        a, b = base_a.clone(), base_b * scale
+        a[37, 11] = value
+        a[140, 70] = value
+        reference = a.cpu().double() @ b.cpu().double()
+        for cfg in _tiles(torch.float32):
+            c = torch.empty((m, n), device="cuda")
+            print(f"fp32 range {value} {cfg.tile_key} {precision}", flush=True)
+            launch_matmul(a, b, c, cfg, precision, autotune=False)
+            torch.cuda.synchronize()
+            got = c.cpu().double()
+            assert torch.equal(torch.isnan(got), torch.isnan(reference)), (value, cfg)
+            finite = torch.isfinite(reference)
+            assert torch.equal(got[~finite & ~torch.isnan(reference)], reference[~finite & ~torch.isnan(reference)])
+            # 72 products per sum: each fp32 rounding is within 2^-24 of the absolute values' sum.
+            bound = 72 * 2.0**-24 * (a.cpu().double().abs() @ b.cpu().double().abs())
+            assert ((got - reference).abs() <= bound)[finite].all(), (value, cfg)
