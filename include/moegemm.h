@@ -162,17 +162,16 @@ int moegemm_matmul_splitk(const void* a, const void* b, void* c, int32_t m, int3
                           int32_t block_m, int32_t block_n, int32_t block_k, int32_t group_size_m,
                           int32_t num_warps, int32_t num_stages, int32_t splits, int32_t grid_size,
                           void* workspace, int64_t workspace_bytes, int32_t b_stream, void* stream);
-/* moegemm_matmul_splitk for every operand layout the LDS-DMA kernels take: row-major operands as
- * above, and transposed ones (the layouts of MOEGEMM_LAYOUT_*, found from the strides) on the tiles
- * compiled for them (moegemm_kernel_layouts).  It serves launch_matmul (reference
- * kernels/matmul.py:332-392) on transposed views: a linear layer's [N, K] weight, and the products
- * of a backward pass. */
-int moegemm_matmul_splitk_transposed(const void* a, const void* b, void* c, int32_t m, int32_t n, int32_t k,
-                                     int64_t stride_am, int64_t stride_ak, int64_t stride_bk, int64_t stride_bn,
-                                     int64_t stride_cm, int64_t stride_cn, int32_t dtype, int32_t block_m,
-                                     int32_t block_n, int32_t block_k, int32_t group_size_m, int32_t num_warps,
-                                     int32_t num_stages, int32_t splits, int32_t grid_size, void* workspace,
-                                     int64_t workspace_bytes, int32_t b_stream, void* stream);
+/* moegemm_matmul_splitk for operands of every layout and dtype: row-major 16-bit operands as above,
+ * transposed ones on the tiles compiled for them, and everything else (fp32, any strides and
+ * alignment) on the general tiles with a split-K kernel (moegemm_kernel_layouts).  It serves
+ * launch_matmul (reference kernels/matmul.py:332-392) where few output tiles leave most CUs idle. */
+int moegemm_matmul_splitk_any(const void* a, const void* b, void* c, int32_t m, int32_t n, int32_t k,
+                              int64_t stride_am, int64_t stride_ak, int64_t stride_bk, int64_t stride_bn,
+                              int64_t stride_cm, int64_t stride_cn, int32_t dtype, int32_t input_precision,
+                              int32_t block_m, int32_t block_n, int32_t block_k, int32_t group_size_m,
+                              int32_t num_warps, int32_t num_stages, int32_t splits, int32_t grid_size,
+                              void* workspace, int64_t workspace_bytes, int32_t b_stream, void* stream);
 /*
  * moegemm_matmul_splitk without the workspace argument: the partials and tile counters live in a
  * static device array of MOEGEMM_NOALLOC_SCRATCH_BYTES inside the library (one per GPU, held until
@@ -204,6 +203,15 @@ int moegemm_grouped_gemm_splitk(const int64_t* a_ptrs, const int64_t* b_ptrs, co
                                 int32_t group_size_m, int32_t num_warps, int32_t num_stages,
                                 int32_t splits, int32_t grid_size, int32_t vector_layout,
                                 void* workspace, int64_t workspace_bytes, int32_t b_stream, void* stream);
+
+/* moegemm_grouped_gemm_splitk for every dtype: vector_layout 0 (and fp32) runs the general tiles with
+ * a split-K kernel (reference kernels/grouped_gemm.py:321-397, whose programs take whole tiles). */
+int moegemm_grouped_gemm_splitk_any(const int64_t* a_ptrs, const int64_t* b_ptrs, const int64_t* c_ptrs,
+                                    int32_t problem_count, int32_t m, int32_t n, int32_t k, int32_t dtype,
+                                    int32_t input_precision, int32_t block_m, int32_t block_n, int32_t block_k,
+                                    int32_t group_size_m, int32_t num_warps, int32_t num_stages, int32_t splits,
+                                    int32_t grid_size, int32_t vector_layout, void* workspace,
+                                    int64_t workspace_bytes, int32_t b_stream, void* stream);
 
 /*
  * Stream-K tail in one launch, for launches whose tile count leaves the last round of a persistent
@@ -245,7 +253,8 @@ int moegemm_grouped_gemm_streamk(const int64_t* a_ptrs, const int64_t* b_ptrs, c
 int moegemm_kernel_swiglu(int dtype, int index);
 
 /* Operand layouts compiled kernel `index` of `dtype` runs on the LDS-DMA path, as a bit mask: bit 0
- * row-major, bit 1 A transposed, bit 2 B transposed, bit 3 both; < 0 on a bad index.  No counterpart
+ * row-major, bit 1 A transposed, bit 2 B transposed, bit 3 both; bit 4: its general tile has a
+ * split-K kernel (the *_splitk_any entry points); < 0 on a bad index.  No counterpart
  * in the reference (its Triton kernels take strides). */
 int moegemm_kernel_layouts(int dtype, int index);
 

@@ -85,7 +85,8 @@ int launch(const KernelEntry* e, KParams& p, int grid, int layout, int32_t b_str
       return fail(MOEGEMM_ERR_INVALID, "stream-K needs fp16/bf16 operands in the vector layout");
     fn = e->launch_fast_streamk;
   } else if (p.splits > 1) {  // split-K units: the fast path's split kernel (the callers checked the layout)
-    fn = layout == 0 ? e->launch_fast_split : layout > 0 ? e->launch_transposed_split[layout - 1] : nullptr;
+    fn = layout == 0 ? e->launch_fast_split
+                     : layout > 0 ? e->launch_transposed_split[layout - 1] : e->launch_general_split;
     if (!fn) return fail(MOEGEMM_ERR_INVALID, "split-K needs fp16/bf16 operands in the vector layout");
   }
   hipError_t err = fn(p, grid, reinterpret_cast<hipStream_t>(stream));
@@ -442,17 +443,20 @@ static int matmul_splitk_impl(const void* a, const void* b, void* c, int32_t m, 
                           int64_t stride_cn, int32_t dtype, int32_t block_m, int32_t block_n, int32_t block_k,
                           int32_t group_size_m, int32_t num_warps, int32_t num_stages, int32_t splits,
                           int32_t grid_size, void* workspace, int64_t workspace_bytes, int32_t b_stream, void* stream,
-                          bool transposed_ok = false) {
+                          bool any_layout = false,
+                          int32_t input_precision = MOEGEMM_PRECISION_IEEE) {
   const KernelEntry* e = nullptr;
-  int rc = check_common(dtype, MOEGEMM_PRECISION_IEEE, group_size_m, &e, block_m, block_n, block_k, num_warps,
+  int rc = check_common(dtype, input_precision, group_size_m, &e, block_m, block_n, block_k, num_warps,
                         num_stages);
   if (rc != MOEGEMM_OK) return rc;
   if (!a || !b || !c) return fail(MOEGEMM_ERR_INVALID, "matrix pointers must be non-null");
   if (m <= 0 || n <= 0 || k <= 0) return fail(MOEGEMM_ERR_INVALID, "shape must be positive (m=%d n=%d k=%d)", m, n, k);
-  const int layout = fast_layout(a, b, c, m, n, k, stride_am, stride_ak, stride_bk, stride_bn, stride_cm, stride_cn,
-                                 dtype);
-  if (layout < 0 || (layout > 0 && (!transposed_ok || !e->launch_transposed_split[layout - 1])) || !e->launch_fast)
+  int layout = fast_layout(a, b, c, m, n, k, stride_am, stride_ak, stride_bk, stride_bn, stride_cm, stride_cn, dtype);
+  if (layout > 0 && !e->launch_transposed_split[layout - 1]) layout = kGeneral;
+  if (!any_layout && layout != 0)
     return fail(MOEGEMM_ERR_INVALID, "split-K needs fp16/bf16 operands in the vector layout");
+  if (layout == kGeneral && !e->launch_general_split)
+    return fail(MOEGEMM_ERR_INVALID, "this tile has no split-K kernel outside the vector layout");
   const int64_t tiles = cdiv(m, block_m) * cdiv(n, block_n);
   KParams p;
   std::memset(&p, 0, sizeof(p));
@@ -471,6 +475,7 @@ static int matmul_splitk_impl(const void* a, const void* b, void* c, int32_t m, 
   p.scn = stride_cn;
   p.G = 1;
   p.group_m = group_size_m;
+  p.tf32 = input_precision == MOEGEMM_PRECISION_TF32;
   rc = setup_splits(p, tiles, k, splits, block_m, block_n, block_k, workspace, workspace_bytes);
   if (rc != MOEGEMM_OK) return rc;
   const int64_t units = (int64_t)p.total_tiles * p.splits;
@@ -488,15 +493,15 @@ int moegemm_matmul_splitk(const void* a, const void* b, void* c, int32_t m, int3
                             workspace, workspace_bytes, b_stream, stream);
 }
 
-int moegemm_matmul_splitk_transposed(const void* a, const void* b, void* c, int32_t m, int32_t n, int32_t k,
-                                     int64_t stride_am, int64_t stride_ak, int64_t stride_bk, int64_t stride_bn,
-                                     int64_t stride_cm, int64_t stride_cn, int32_t dtype, int32_t block_m,
-                                     int32_t block_n, int32_t block_k, int32_t group_size_m, int32_t num_warps,
-                                     int32_t num_stages, int32_t splits, int32_t grid_size, void* workspace,
-                                     int64_t workspace_bytes, int32_t b_stream, void* stream) {
+int moegemm_matmul_splitk_any(const void* a, const void* b, void* c, int32_t m, int32_t n, int32_t k,
+                              int64_t stride_am, int64_t stride_ak, int64_t stride_bk, int64_t stride_bn,
+                              int64_t stride_cm, int64_t stride_cn, int32_t dtype, int32_t input_precision,
+                              int32_t block_m, int32_t block_n, int32_t block_k, int32_t group_size_m,
+                              int32_t num_warps, int32_t num_stages, int32_t splits, int32_t grid_size,
+                              void* workspace, int64_t workspace_bytes, int32_t b_stream, void* stream) {
   return matmul_splitk_impl(a, b, c, m, n, k, stride_am, stride_ak, stride_bk, stride_bn, stride_cm, stride_cn, dtype,
                             block_m, block_n, block_k, group_size_m, num_warps, num_stages, splits, grid_size,
-                            workspace, workspace_bytes, b_stream, stream, true);
+                            workspace, workspace_bytes, b_stream, stream, true, input_precision);
 }
 
 int moegemm_kernel_layouts(int dtype, int index) {
@@ -507,6 +512,7 @@ int moegemm_kernel_layouts(int dtype, int index) {
   int mask = t[index].launch_fast ? 1 : 0;
   for (int layout = 1; layout <= 3; ++layout)
     if (t[index].launch_transposed[layout - 1]) mask |= 1 << layout;
+  if (t[index].launch_general_split) mask |= 1 << 4;
   return mask;
 }
 
@@ -537,22 +543,25 @@ int moegemm_matmul_splitk_noalloc(const void* a, const void* b, void* c, int32_t
                             MOEGEMM_NOALLOC_SCRATCH_BYTES, b_stream, stream);
 }
 
-int moegemm_grouped_gemm_splitk(const int64_t* a_ptrs, const int64_t* b_ptrs, const int64_t* c_ptrs,
+static int grouped_splitk_impl(const int64_t* a_ptrs, const int64_t* b_ptrs, const int64_t* c_ptrs,
                                 int32_t problem_count, int32_t m, int32_t n, int32_t k, int32_t dtype,
                                 int32_t block_m, int32_t block_n, int32_t block_k, int32_t group_size_m,
                                 int32_t num_warps, int32_t num_stages, int32_t splits, int32_t grid_size,
                                 int32_t vector_layout, void* workspace, int64_t workspace_bytes,
-                                int32_t b_stream, void* stream) {
+                                int32_t b_stream, void* stream, bool any_layout, int32_t input_precision) {
   const KernelEntry* e = nullptr;
-  int rc = check_common(dtype, MOEGEMM_PRECISION_IEEE, group_size_m, &e, block_m, block_n, block_k, num_warps,
+  int rc = check_common(dtype, input_precision, group_size_m, &e, block_m, block_n, block_k, num_warps,
                         num_stages);
   if (rc != MOEGEMM_OK) return rc;
   if (problem_count <= 0) return fail(MOEGEMM_ERR_INVALID, "problem_count must be positive (got %d)", problem_count);
   if (!a_ptrs || !b_ptrs || !c_ptrs) return fail(MOEGEMM_ERR_INVALID, "pointer tables must be non-null");
   if (m <= 0 || n <= 0 || k <= 0)
     return fail(MOEGEMM_ERR_INVALID, "homogeneous shape must be positive (m=%d n=%d k=%d)", m, n, k);
-  if (!vector_layout || !e->launch_fast)
+  const int layout = vector_layout && e->launch_fast ? 0 : kGeneral;
+  if (layout == kGeneral && !any_layout)
     return fail(MOEGEMM_ERR_INVALID, "split-K needs fp16/bf16 operands in the vector layout");
+  if (layout == kGeneral && !e->launch_general_split)
+    return fail(MOEGEMM_ERR_INVALID, "this tile has no split-K kernel outside the vector layout");
   const int64_t tiles = (int64_t)problem_count * cdiv(m, block_m) * cdiv(n, block_n);
   KParams p;
   std::memset(&p, 0, sizeof(p));
@@ -565,11 +574,34 @@ int moegemm_grouped_gemm_splitk(const int64_t* a_ptrs, const int64_t* b_ptrs, co
   p.N = n;
   p.K = k;
   p.group_m = group_size_m;
+  p.tf32 = input_precision == MOEGEMM_PRECISION_TF32;
   rc = setup_splits(p, tiles, k, splits, block_m, block_n, block_k, workspace, workspace_bytes);
   if (rc != MOEGEMM_OK) return rc;
   const int64_t units = (int64_t)p.total_tiles * p.splits;
   const int grid = grid_size <= 0 || grid_size > units ? (int)units : grid_size;
-  return launch(e, p, grid, 0, b_stream, stream);
+  return launch(e, p, grid, layout, b_stream, stream);
+}
+
+int moegemm_grouped_gemm_splitk(const int64_t* a_ptrs, const int64_t* b_ptrs, const int64_t* c_ptrs,
+                                int32_t problem_count, int32_t m, int32_t n, int32_t k, int32_t dtype,
+                                int32_t block_m, int32_t block_n, int32_t block_k, int32_t group_size_m,
+                                int32_t num_warps, int32_t num_stages, int32_t splits, int32_t grid_size,
+                                int32_t vector_layout, void* workspace, int64_t workspace_bytes,
+                                int32_t b_stream, void* stream) {
+  return grouped_splitk_impl(a_ptrs, b_ptrs, c_ptrs, problem_count, m, n, k, dtype, block_m, block_n, block_k,
+                             group_size_m, num_warps, num_stages, splits, grid_size, vector_layout, workspace,
+                             workspace_bytes, b_stream, stream, false, MOEGEMM_PRECISION_IEEE);
+}
+
+int moegemm_grouped_gemm_splitk_any(const int64_t* a_ptrs, const int64_t* b_ptrs, const int64_t* c_ptrs,
+                                    int32_t problem_count, int32_t m, int32_t n, int32_t k, int32_t dtype,
+                                    int32_t input_precision, int32_t block_m, int32_t block_n, int32_t block_k,
+                                    int32_t group_size_m, int32_t num_warps, int32_t num_stages, int32_t splits,
+                                    int32_t grid_size, int32_t vector_layout, void* workspace,
+                                    int64_t workspace_bytes, int32_t b_stream, void* stream) {
+  return grouped_splitk_impl(a_ptrs, b_ptrs, c_ptrs, problem_count, m, n, k, dtype, block_m, block_n, block_k,
+                             group_size_m, num_warps, num_stages, splits, grid_size, vector_layout, workspace,
+                             workspace_bytes, b_stream, stream, true, input_precision);
 }
 
 int moegemm_streamk_workspace_bytes(int32_t tail_tiles, int32_t grid_size, int32_t block_m, int32_t block_n,

@@ -852,6 +852,7 @@ struct FastTile {
   static constexpr bool CHAIN_OK = (STAGES == 2 && FM * FN * ACC <= 128 && BM * BN <= 32768) || CHAIN_DEEP;
   static constexpr int CHAIN_MIN_SLICES = CHAIN_DEEP ? STAGES : 1;
   static constexpr int CHAIN_MAX_SLICES = CHAIN_DEEP ? 8 : FM * FN * ACC <= 64 ? (1 << 30) : 8;
+  static constexpr bool ABSOLUTE_K = false;
   static constexpr bool CHAIN_STEALING = STAGES == 2;  // the two-stage loop also runs the stealing schedule
   static constexpr int CH_ROWS_FIT = STAGED_OK ? (XMIN * 1024 / ROWB) / MI * MI : MI;
   static constexpr int CH_ROWS = CH_ROWS_FIT < WTM ? CH_ROWS_FIT : WTM;  // staged rows per round

@@ -35,12 +35,18 @@
 //    8 x [512,2048]@[2048,1536] 458 -> 185 us; TF32 [1024,4096]@[4096,3584] 669 -> 131 us; fp16
 //    [777,2881]@[2881,1443] 148 -> 38 us (element-wise gathers before); bf16
 //    [4001,4003]@[4003,4005] runs at 814 TFLOP/s.
+//  * Split-K.  Few tiles leave the chip idle, and a lone workgroup on a CU runs at the latency of its
+//    steps, so a tile's K slices can be shared by several workgroups (fp32 [64,4096]@[4096,1024]:
+//    66 us whole, 21 us in eight; the reduction costs about 5 us, so large groups stay whole): each stores its fp32 partial, and the last to arrive sums them in split order
+//    (deterministic) and stores C.  Counters, partial layout and coherence are FastTile's
+//    (gemm_fast.h, split_store); nobody waits for another unit.
 //  * Range.  The split is exact and its products neither overflow nor lose their small parts while
 //    every non-zero operand lies in [2^-96, 2^60).  Each thread keeps the extremes of what it
 //    loaded; a tile that met a value outside (infinities and NaN included) is computed again by GemmTile, with the fp32
 //    instruction.
 #pragma once
 
+#include "gemm_fast.h"
 #include "gemm_kernel.h"
 
 namespace moegemm {
@@ -82,6 +88,7 @@ struct GeneralTile {
   static constexpr int WAVES_PER_EU = 2 * LDS_BYTES <= 160 * 1024 || NW == 8 ? 2 : 1;
   static constexpr bool CHAIN_OK = false;
   static constexpr bool CHAIN_STEALING = false;
+  static constexpr bool ABSOLUTE_K = true;
 
   static_assert(F32 ? PARTS >= 2 : PARTS == 1, "16-bit operands are one part, fp32 operands two or three");
   static_assert(BK % MIK == 0 && WTM % MI == 0 && WTN % MI == 0, "tile shape");
@@ -362,8 +369,82 @@ struct GeneralTile {
     }
   }
 
+  // Split-K: stores the unit's partial (unless `bad`: a value outside the split's range was met) and
+  // arrives at the tile's counter (arrivals in bits 0-15, bad units above).  The last unit to arrive
+  // re-arms the counter and sums the partials into acc, in split order.  Returns what is left to
+  // this workgroup: 0 nothing, 1 store acc, 2 compute the whole tile with the fp32 instruction.
+  static constexpr int CHUNKS = FM * FN * (ACC / 4);  // 16-byte accumulator chunks per lane
+  __device__ static __forceinline__ int reduce_splits(acc_t (&acc)[FM][FN], const ProblemDesc& pd, bool bad) {
+    __shared__ int s_left;
+    constexpr int kBytes = BM * BN * 4;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane_off = (wave * CHUNKS * 64 + (int)(threadIdx.x & 63)) * 16;
+    auto partial = [&](int split) {
+      return __builtin_amdgcn_make_buffer_rsrc(pd.partials + ((int64_t)pd.slot0 + split) * (BM * BN), (short)0, kBytes,
+                                               (int)kBufferFlags);
+    };
+    if (!bad) {
+      const auto mine = partial(pd.split);
+#pragma unroll
+      for (int c = 0; c < CHUNKS; ++c) {
+        const acc_t& t = acc[c / (ACC / 4) / FN][c / (ACC / 4) % FN];
+        const int q = c % (ACC / 4);
+        const f32x4_t v = {t[q * 4 + 0], t[q * 4 + 1], t[q * 4 + 2], t[q * 4 + 3]};
+        __builtin_amdgcn_raw_buffer_store_b128(v, mine, lane_off + c * 1024, 0, kDeviceCoherent);
+      }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int32_t* word = pd.counters + pd.tile;
+      const int old = atomicAdd(word, bad ? 0x10001 : 1);
+      int left = 0;
+      if ((old & 0xffff) == pd.splits - 1) {
+        atomicExch(word, 0);
+        left = bad || (old >> 16) ? 2 : 1;
+      }
+      s_left = left;
+    }
+    __syncthreads();
+    const int left = uniform(s_left);
+    if (left != 1) return left;
+    constexpr int GC = CHUNKS < 4 ? CHUNKS : 4, WAYS = 4;  // chunks and partials read at a time
+#pragma unroll
+    for (int c0 = 0; c0 < CHUNKS; c0 += GC) {
+      f32x4_t sum[GC];
+#pragma unroll
+      for (int i = 0; i < GC; ++i) sum[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int s0 = 0; s0 < pd.splits; s0 += WAYS) {
+        f32x4_t v[WAYS][GC];
+#pragma unroll
+        for (int w = 0; w < WAYS; ++w) {
+          const auto from = partial(min(s0 + w, pd.splits - 1));
+#pragma unroll
+          for (int i = 0; i < GC; ++i)
+            v[w][i] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                      from, lane_off + (c0 + i) * 1024, 0, kDeviceCoherent));
+        }
+#pragma unroll
+        for (int w = 0; w < WAYS; ++w)
+          if (s0 + w < pd.splits) {
+#pragma unroll
+            for (int i = 0; i < GC; ++i)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) sum[i][e] += v[w][i][e];
+          }
+      }
+#pragma unroll
+      for (int i = 0; i < GC; ++i) {
+        const int c = c0 + i;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[c / (ACC / 4) / FN][c / (ACC / 4) % FN][c % (ACC / 4) * 4 + e] = sum[i][e];
+      }
+    }
+    return 1;
+  }
+
   // The tile with both operands in 8-element chunks; false when it must be computed by Plain.
-  template <bool AT, bool BT, class Hook>
+  template <bool AT, bool BT, int EPI, class Hook>
   __device__ static __forceinline__ bool chunk_tile(const ProblemDesc& pd, int tm, int tn, char* smem,
                                                     Hook&& before_store) {
     const int wave = threadIdx.x >> 6;
@@ -386,12 +467,14 @@ struct GeneralTile {
         for (int i = 0; i < ACC; ++i) acc[fm][fn][i] = 0.0f;
     uint32_t range[2] = {0u, 0xffffffffu};
 
-    const int last = (pd.k + BK - 1) / BK - 1;  // last K slice
+    // K slices first .. first + last, from k_first on; a unit's range starts at a whole slice.
+    const int k_first = EPI == EPI_SPLIT ? pd.k_begin : 0, k_end = EPI == EPI_SPLIT ? pd.k_end : pd.k;
+    const int last = (k_end - k_first + BK - 1) / BK - 1;
     u32x4_t ra[DEPTH][A_PT][VL], rb[DEPTH][B_PT][VL];
     // Register set of slice kt: kt % DEPTH; LDS buffer: kt % 2.  J: kt modulo UNROLL.
     auto load = [&](auto j, int kt) {
       constexpr int S = decltype(j)::value % DEPTH;
-      const int k0 = min(kt, last) * BK;
+      const int k0 = k_first + min(kt, last) * BK;
       a.load(ra[S], k0);
       b.load(rb[S], k0);
     };
@@ -399,8 +482,8 @@ struct GeneralTile {
       constexpr int S = decltype(j)::value % DEPTH;
       constexpr bool EDGE = decltype(edge)::value;
       char* lds = smem + (decltype(j)::value % 2) * STAGE_BYTES;
-      a.template store<EDGE>(ra[S], kt * BK, lds, range);
-      b.template store<EDGE>(rb[S], kt * BK, lds + PARTS * A_BYTES, range);
+      a.template store<EDGE>(ra[S], k_first + kt * BK, lds, range);
+      b.template store<EDGE>(rb[S], k_first + kt * BK, lds + PARTS * A_BYTES, range);
     };
     // Slice kt is computed from its LDS buffer while slice kt + 1 (in registers) goes to the other
     // one and slices up to kt + DEPTH are in flight.  Steps whose stored slice is no edge are one
@@ -433,16 +516,21 @@ struct GeneralTile {
     __syncthreads();
     int kt = 0;
     if (a.x_over == 0 && b.x_over == 0) {
-      const int inner = pd.k / BK;  // whole slices
+      const int inner = (k_end - k_first) / BK;  // whole slices
       for (; kt + UNROLL < inner; kt += UNROLL) steps(std::false_type{}, kt, 0);
     }
     for (; kt < last; kt += UNROLL) steps(std::true_type{}, kt, last);
     compute(acc, smem + (last & 1) * STAGE_BYTES, fa, fb);
-    if constexpr (F32) {
-      // Also the barrier between this tile's LDS reads and the next tile's writes.
-      if (__syncthreads_or(range[0] >= kTooLarge || range[1] < kTooSmall)) return false;
-    } else {
+    bool bad = false;
+    if constexpr (F32)  // also the barrier between this tile's LDS reads and the next tile's writes
+      bad = __syncthreads_or(range[0] >= kTooLarge || range[1] < kTooSmall) != 0;
+    else
       __syncthreads();
+    if constexpr (EPI == EPI_SPLIT) {
+      const int left = reduce_splits(acc, pd, bad);
+      if (left != 1) return left == 0;
+    } else {
+      if (bad) return false;
     }
     before_store();
     store_tile(acc, pd, m0, n0, wave_m, wave_n);
@@ -452,8 +540,8 @@ struct GeneralTile {
   template <int EPI, class Hook>
   __device__ static __forceinline__ void run_tile(const ProblemDesc& pd, int tm, int tn, char* smem, bool tf32,
                                                   Hook&& before_store) {
-    static_assert(EPI == EPI_C, "the general kernel has no split-K epilogue");
-    if (pd.swiglu || pd.splits > 1) return;  // LDS-DMA tiles only (the host enforces it)
+    static_assert(EPI == EPI_C || EPI == EPI_SPLIT, "the general kernel has no stream-K tail");
+    if (pd.swiglu || (EPI == EPI_C && pd.splits > 1)) return;  // the host launches neither
     // 32-bit offsets span a tile's rows (K-contiguous) or a slice's (XC).
     constexpr int64_t kPitchLimit = (int64_t(1) << 32) / (BM > BN ? BM : BN) / 2;
     const bool a_rows = pd.sak == 1 && pd.k >= 8 && pd.sam * ES < kPitchLimit && (int64_t)pd.k * ES < (1ll << 31);
@@ -462,19 +550,27 @@ struct GeneralTile {
     const bool b_rows = pd.sbk == 1 && pd.k >= 8 && pd.sbn * ES < kPitchLimit && (int64_t)pd.k * ES < (1ll << 31);
     const bool b_cols = deep && pd.sbn == 1 && pd.n >= 8 && pd.sbk * ES < kPitchLimit;
     bool done = false;
+    if constexpr (EPI == EPI_SPLIT) {
+      // Operands Plain must stage: unit 0 of each tile computes it whole.
+      if (!((a_rows || (BM >= 32 && a_cols)) && (b_rows || b_cols)) && pd.split != 0) return;
+    }
     if (a_rows && b_cols) {
-      done = chunk_tile<false, false>(pd, tm, tn, smem, before_store);
+      done = chunk_tile<false, false, EPI>(pd, tm, tn, smem, before_store);
     } else if (a_rows && b_rows) {
-      done = chunk_tile<false, true>(pd, tm, tn, smem, before_store);
+      done = chunk_tile<false, true, EPI>(pd, tm, tn, smem, before_store);
     } else if (a_cols && (b_cols || b_rows)) {
       if constexpr (BM >= 32) {
         if (b_cols)
-          done = chunk_tile<true, false>(pd, tm, tn, smem, before_store);
+          done = chunk_tile<true, false, EPI>(pd, tm, tn, smem, before_store);
         else
-          done = chunk_tile<true, true>(pd, tm, tn, smem, before_store);
+          done = chunk_tile<true, true, EPI>(pd, tm, tn, smem, before_store);
       }
     }
-    if (!done) Plain::template run_tile<EPI_C>(pd, tm, tn, smem, tf32, before_store);
+    if (!done) {
+      ProblemDesc whole = pd;
+      whole.splits = 1;
+      Plain::template run_tile<EPI_C>(whole, tm, tn, smem, tf32, before_store);
+    }
   }
 };
 

@@ -112,6 +112,7 @@ struct ProblemDesc {
   int32_t* counters;
   int32_t slot0;       // partial slot of the tile's unit 0; unit s writes slot slot0 + s
   int32_t b_stream;    // KParams::b_stream
+  int32_t k_begin, k_end;  // split-K units of ABSOLUTE_K tiles: the unit's K range (a, b, k unshifted)
 };
 
 
@@ -301,6 +302,7 @@ struct GemmTile {
   static constexpr int WAVES_PER_EU = 1;
   static constexpr bool CHAIN_OK = false;  // no cross-tile copy chaining (LDS-DMA tiles only)
   static constexpr bool CHAIN_STEALING = false;
+  static constexpr bool ABSOLUTE_K = false;
 
   static_assert(BM % WM == 0 && BN % WN == 0, "tile must split evenly over waves");
   static_assert(WTM % MI == 0 && WTN % MI == 0, "wave tile must be a multiple of the MFMA tile");
@@ -1076,9 +1078,14 @@ grouped_gemm_kernel(KParams p) {
     pd.counters = p.counters;
     if (splits > 1) {  // this unit's K range: shift A's columns and B's rows, shorten K
       const int k_begin = pd.split * p.k_chunk;
-      pd.a += (int64_t)k_begin * pd.sak * T::ES;
-      pd.b += (int64_t)k_begin * pd.sbk * T::ES;
-      pd.k = min(p.k_chunk, pd.k - k_begin);
+      if constexpr (T::ABSOLUTE_K) {
+        pd.k_begin = uniform(k_begin);
+        pd.k_end = uniform(min(k_begin + p.k_chunk, pd.k));
+      } else {
+        pd.a += (int64_t)k_begin * pd.sak * T::ES;
+        pd.b += (int64_t)k_begin * pd.sbk * T::ES;
+        pd.k = min(p.k_chunk, pd.k - k_begin);
+      }
     }
     make_uniform(pd);
     int ticket = -1;  // the next unit's ticket: drawn before the C stores, resolved after the tile

@@ -1,0 +1,5 @@
+// Compiled f16 split-K kernels of the general tile.
+#include "registry.h"
+namespace moegemm {
+MOEGEMM_MENU_GEN_SPLIT(MOEGEMM_INST16_GENSPLIT, EF16)
+}  // namespace moegemm

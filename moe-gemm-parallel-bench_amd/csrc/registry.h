@@ -28,6 +28,7 @@ struct KernelEntry {
   // The fast path for transposed operands, by OperandLayout - 1 (null: not compiled for this tile).
   LaunchFn launch_transposed[3];
   LaunchFn launch_transposed_split[3];
+  LaunchFn launch_general_split;  // the general tile's split-K kernel (null: not compiled for this tile)
 };
 
 template <class T, bool SPLIT = false, bool STREAMK = false>
@@ -57,9 +58,9 @@ struct GeneralTileEntry : GeneralTile<E, BM, BN, BK, WM, WN, PARTS> {};
 #define MOEGEMM_GEN_TF32(E, BM, BN, BK, WM, WN, S) GeneralTileEntry<E, BM, BN, BK, WM, WN, S, 2>
 
 // fp32 launches: the input precision picks the kernel (three bf16 parts per operand, or TF32's two).
-template <class IEEE, class TF32>
+template <class IEEE, class TF32, bool SPLIT>
 hipError_t launch_f32(const KParams& p, int grid, hipStream_t stream) {
-  return p.tf32 ? launch_tile<TF32>(p, grid, stream) : launch_tile<IEEE>(p, grid, stream);
+  return p.tf32 ? launch_tile<TF32, SPLIT>(p, grid, stream) : launch_tile<IEEE, SPLIT>(p, grid, stream);
 }
 
 #define MOEGEMM_INST16(E, BM, BN, BK, WM, WN, S)                                                     \
@@ -69,6 +70,28 @@ hipError_t launch_f32(const KParams& p, int grid, hipStream_t stream) {
 #define MOEGEMM_INST16_GEN(E, BM, BN, BK, WM, WN, S)                                                         \
   template __global__ void grouped_gemm_kernel<MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S), false>(KParams);       \
   template hipError_t launch_tile<MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S)>(const KParams&, int, hipStream_t);
+// General tiles with a split-K kernel: one per size class, for the tuner to spread few tiles.
+#define MOEGEMM_MENU_GEN_SPLIT(X, E)                                                                    \
+  X(E, 256, 256, 32, 2, 4, 4) X(E, 128, 128, 64, 2, 2, 4) X(E, 128, 64, 64, 2, 2, 4)                    \
+  X(E, 64, 128, 64, 2, 2, 4) X(E, 64, 64, 64, 2, 2, 4) X(E, 32, 128, 64, 1, 4, 4)                       \
+  X(E, 16, 64, 128, 1, 4, 4)
+#define MOEGEMM_INST16_GENSPLIT(E, BM, BN, BK, WM, WN, S)                                               \
+  template __global__ void grouped_gemm_kernel<MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S), true>(KParams);   \
+  template hipError_t launch_tile<MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S), true>(const KParams&, int, hipStream_t);
+#define MOEGEMM_EXTERN16_GENSPLIT(E, BM, BN, BK, WM, WN, S) \
+  extern template hipError_t launch_tile<MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S), true>(const KParams&, int, hipStream_t);
+#define MOEGEMM_MATCH_GENSPLIT(E, BM, BN, BK, WM, WN, S) \
+  || (bm == BM && bn == BN && bk == BK && wm == WM && wn == WN && s == S)
+constexpr bool general_split_compiled(int bm, int bn, int bk, int wm, int wn, int s) {
+  return false MOEGEMM_MENU_GEN_SPLIT(MOEGEMM_MATCH_GENSPLIT, E);
+}
+template <class E, int BM, int BN, int BK, int WM, int WN, int S>
+constexpr LaunchFn general_split_launch() {
+  if constexpr (general_split_compiled(BM, BN, BK, WM, WN, S))
+    return &launch_tile<MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S), true>;
+  else
+    return nullptr;
+}
 #define MOEGEMM_EXTERN16_GEN(E, BM, BN, BK, WM, WN, S) \
   extern template hipError_t launch_tile<MOEGEMM_GEN(E, BM, BN, BK, WM, WN, S)>(const KParams&, int, hipStream_t);
 // The stream-K kernels live in translation units of their own (inst_*_sk.hip): compiled next to
@@ -132,16 +155,26 @@ constexpr LaunchFn transposed_launch() {
                transposed_launch<E, BM, BN, BK, WM, WN, S, 3, false>()},                      \
               {transposed_launch<E, BM, BN, BK, WM, WN, S, 1, true>(),                        \
                transposed_launch<E, BM, BN, BK, WM, WN, S, 2, true>(),                        \
-               transposed_launch<E, BM, BN, BK, WM, WN, S, 3, true>()}},
+               transposed_launch<E, BM, BN, BK, WM, WN, S, 3, true>()},                       \
+              general_split_launch<E, BM, BN, BK, WM, WN, S>()},
 
 #define MOEGEMM_INST32(E, BM, BN, BK, WM, WN, S) \
   template __global__ void grouped_gemm_kernel<MOEGEMM_GEN32(E, BM, BN, BK, WM, WN, S), false>(KParams); \
   template __global__ void grouped_gemm_kernel<MOEGEMM_GEN_TF32(E, BM, BN, BK, WM, WN, S), false>(KParams);
+#define MOEGEMM_INST32_SPLIT(E, BM, BN, BK, WM, WN, S) \
+  template __global__ void grouped_gemm_kernel<MOEGEMM_GEN32(E, BM, BN, BK, WM, WN, S), true>(KParams); \
+  template __global__ void grouped_gemm_kernel<MOEGEMM_GEN_TF32(E, BM, BN, BK, WM, WN, S), true>(KParams); \
+  template hipError_t launch_f32<MOEGEMM_GEN32(E, BM, BN, BK, WM, WN, S), MOEGEMM_GEN_TF32(E, BM, BN, BK, WM, WN, S), \
+                                 true>(const KParams&, int, hipStream_t);
+#define MOEGEMM_EXTERN32_SPLIT(E, BM, BN, BK, WM, WN, S) \
+  extern template hipError_t launch_f32<MOEGEMM_GEN32(E, BM, BN, BK, WM, WN, S), \
+                                        MOEGEMM_GEN_TF32(E, BM, BN, BK, WM, WN, S), true>(const KParams&, int, hipStream_t);
 #define MOEGEMM_ENTRY32(E, BM, BN, BK, WM, WN, S)                                             \
   KernelEntry{E::dtype, BM, BN, BK, (WM) * (WN), S, WM, WN,                                   \
               MOEGEMM_GEN32(E, BM, BN, BK, WM, WN, S)::LDS_BYTES, 0, nullptr,                    \
-              &launch_f32<MOEGEMM_GEN32(E, BM, BN, BK, WM, WN, S), MOEGEMM_GEN_TF32(E, BM, BN, BK, WM, WN, S)>, \
-              nullptr, nullptr, {nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}},
+              &launch_f32<MOEGEMM_GEN32(E, BM, BN, BK, WM, WN, S), MOEGEMM_GEN_TF32(E, BM, BN, BK, WM, WN, S), false>, \
+              nullptr, nullptr, {nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr},         \
+              &launch_f32<MOEGEMM_GEN32(E, BM, BN, BK, WM, WN, S), MOEGEMM_GEN_TF32(E, BM, BN, BK, WM, WN, S), true>},
 
 // 16-bit menu (bf16 and f16 share it): large-M MFMA-bound tiles down to skinny-M streaming tiles.
 // STAGES is sized to the 160 KiB LDS of a CU; the 2-stage narrow tiles at the end fit two

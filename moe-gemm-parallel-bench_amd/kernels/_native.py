@@ -61,10 +61,15 @@ SIGNATURES = {
         [_vp, _vp, _vp, _i32, _i32, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i32,
          _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _i64, _i32, _vp],
     ),
-    "moegemm_matmul_splitk_transposed": (
+    "moegemm_matmul_splitk_any": (
         ctypes.c_int,
-        [_vp, _vp, _vp, _i32, _i32, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i32,
+        [_vp, _vp, _vp, _i32, _i32, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i32, _i32,
          _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _i64, _i32, _vp],
+    ),
+    "moegemm_grouped_gemm_splitk_any": (
+        ctypes.c_int,
+        [_vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32,
+         _i32, _i32, _i32, _vp, _i64, _i32, _vp],
     ),
     "moegemm_kernel_layouts": (ctypes.c_int, [ctypes.c_int, ctypes.c_int]),
     "moegemm_matmul_splitk_noalloc": (
@@ -193,9 +198,13 @@ B_TRANSPOSED = 2
 LAYOUT_FLAGS = {GENERAL: 0, 0: 1, 1: 0x10001, 2: 0x20001, 3: 0x30001}
 
 
+GENERAL_SPLIT = 4  # moegemm_kernel_layouts' bit for a general tile with a split-K kernel
+
+
 @lru_cache(maxsize=None)
 def layout_tiles(dtype_code: int, layout: int) -> frozenset:
-    """Tile keys whose LDS-DMA kernel is compiled for an operand layout."""
+    """Tile keys whose LDS-DMA kernel is compiled for an operand layout (``GENERAL_SPLIT``: whose
+    general tile has a split-K kernel)."""
     lib = library()
     keys = set()
     for index, row in enumerate(compiled_kernels(dtype_code)):
@@ -205,6 +214,11 @@ def layout_tiles(dtype_code: int, layout: int) -> frozenset:
         if mask >> layout & 1:
             keys.add(tuple(row[:5]))
     return frozenset(keys)
+
+
+def split_tiles(dtype_code: int, layout: int) -> frozenset:
+    """Tile keys that can split K over operands of this layout."""
+    return layout_tiles(dtype_code, GENERAL_SPLIT if layout == GENERAL else layout)
 
 
 _COPIED_PAST_K = 1024  # K rows past the matrix that a tile's zero slices may address

@@ -369,14 +369,19 @@ def _check_workspace(workspace: GroupedWorkspace) -> int:
     return _native.dtype_code(a0.dtype)
 
 
-def _grouped_splits(workspace: GroupedWorkspace, cfg: KernelConfig, dtype_code: int, split_k, vector=None) -> int:
-    if vector is None:
-        vector = _vector_layout(workspace, dtype_code)
-    if not workspace.homogeneous or not vector:
+def _grouped_splits(workspace: GroupedWorkspace, cfg: KernelConfig, dtype_code: int, split_k, layout=None) -> int:
+    if layout is None:
+        layout = _group_layout(workspace, dtype_code)
+    if not workspace.homogeneous or (layout != 0 and cfg.tile_key not in _native.split_tiles(dtype_code, layout)):
         return 1
-    if split_k is not None:
-        return split_k
-    return splitk_count(workspace.tile_count_for(cfg), workspace.max_k, cfg.block_k, workspace.sm_count)
+    tiles = workspace.tile_count_for(cfg)
+    splits = split_k if split_k is not None else splitk_count(tiles, workspace.max_k, cfg.block_k, workspace.sm_count)
+    # General tiles take the unsplit launch where a workspace cannot be made (graph capture).
+    if splits > 1 and layout != 0 and not _native.splitk_workspace_ready(
+            workspace.a[0].device, _native.current_stream_handle(workspace.a[0].device),
+            _native.splitk_workspace_bytes(tiles, splits, cfg.block_m, cfg.block_n)):
+        splits = 1
+    return splits
 
 
 def with_schedule_options(options, tile_schedule: str | None, streamk_ok=None) -> list:
@@ -430,7 +435,7 @@ def _launch_grouped_fixed(workspace: GroupedWorkspace, cfg: KernelConfig, dtype_
         schedule = "static"  # no partial last round: the static launch is the same work
     if layout is None:
         layout = _group_layout(workspace, dtype_code)
-    splits = _grouped_splits(workspace, cfg, dtype_code, split_k, layout == 0)
+    splits = _grouped_splits(workspace, cfg, dtype_code, split_k, layout)
     if schedule == "stealing" and splits > 1:
         raise ValueError("the work-stealing schedule runs unsplit launches only (split_k must be 1)")
     if splits > 1:
@@ -439,11 +444,11 @@ def _launch_grouped_fixed(workspace: GroupedWorkspace, cfg: KernelConfig, dtype_
         stream = _native.current_stream_handle(workspace.a[0].device)
         scratch = _native.splitk_workspace(workspace.a[0].device, stream,
                                            _native.splitk_workspace_bytes(tiles, splits, cfg.block_m, cfg.block_n))
-        status = _native.library().moegemm_grouped_gemm_splitk(
+        status = _native.library().moegemm_grouped_gemm_splitk_any(
             workspace.a_ptrs.data_ptr(), workspace.b_ptrs.data_ptr(), workspace.c_ptrs.data_ptr(),
-            workspace.problem_count, m, n, k, dtype_code,
+            workspace.problem_count, m, n, k, dtype_code, precision,
             cfg.block_m, cfg.block_n, cfg.block_k, cfg.group_size_m, cfg.num_warps, cfg.num_stages, splits,
-            max(1, min(tiles * splits, workspace.sm_count * cfg.cta_multiplier)), 1,
+            max(1, min(tiles * splits, workspace.sm_count * cfg.cta_multiplier)), _native.LAYOUT_FLAGS[layout],
             scratch.data_ptr(), scratch.numel(), b_stream, stream,
         )
         _native.check(status)
@@ -540,9 +545,11 @@ def launch_grouped(
                 tiles=_native.layout_tiles(dtype_code, layout) if layout > 0 else None,
             )
             splittable = workspace.homogeneous and layout == 0
+            general = (_native.split_tiles(dtype_code, layout)
+                       if workspace.homogeneous and layout == _native.GENERAL else None)
             options = with_schedule_options(
                 with_split_options(candidates, workspace.tile_count_for, workspace.max_k, workspace.sm_count,
-                                   split_k, splittable),
+                                   split_k, splittable, general),
                 tile_schedule,
                 lambda cfg: streamk_tail_for(workspace, cfg, dtype_code) > 0,
             )

@@ -319,19 +319,27 @@ def splitk_count(tiles: int, k: int, block_k: int, sm_count: int) -> int:
     return splits if splits >= 2 else 1
 
 
-def with_split_options(configs, tiles_of, k: int, sm_count: int, split_k, splittable: bool) -> list:
+def with_split_options(configs, tiles_of, k: int, sm_count: int, split_k, splittable: bool, general=None) -> list:
     """(config, split) tuning candidates: each config unsplit and, where ``splitk_count`` would
     split it, also split — so measurement, not the heuristic alone, decides.  An explicit
-    ``split_k`` pins the split of every candidate."""
+    ``split_k`` pins the split of every candidate.  ``general``: tile keys of the general kernels that
+    can split (None for the LDS-DMA kernels).  Those run one slice's latency at a time and most fit a CU
+    twice, so the count that gives every CU two units, and two splits of up to three tiles a CU, are
+    timed too: fp16 [777,2881]@[2881,1443] 38 us unsplit, 31 in three (156 tiles of 64x128); fp32
+    [64,4096]@[4096,1024] 66 -> 21 us; fp32 8 x [16,4096]@[4096,4096] 144 -> 108 us in two."""
     out = []
     for cfg in configs:
         if split_k is not None:
             out.append((cfg, split_k))
             continue
         out.append((cfg, 1))
-        splits = splitk_count(tiles_of(cfg), k, cfg.block_k, sm_count) if splittable else 1
-        if splits > 1:
-            out.append((cfg, splits))
+        tiles = tiles_of(cfg)
+        if general is None:
+            counts = [splitk_count(tiles, k, cfg.block_k, sm_count)] if splittable else []
+        else:
+            most = min(k // (4 * cfg.block_k), 16) if cfg.tile_key in general and tiles <= 3 * sm_count else 1
+            counts = [min(most, sm_count // tiles), min(most, 2 * sm_count // tiles), min(most, 2)]
+        out += [(cfg, splits) for splits in dict.fromkeys(counts) if splits > 1]
     return out
 
 
@@ -378,14 +386,15 @@ def _launch_fixed_streamk(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, 
     _native.check(status)
 
 
-def _launch_fixed_splitk(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, splits: int, b_stream: int = 0) -> None:
+def _launch_fixed_splitk(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, splits: int, b_stream: int = 0,
+                         precision: int = _native.PRECISION_IEEE) -> None:
     tiles = -(-m // cfg.block_m) * -(-n // cfg.block_n)
     nbytes = _native.splitk_workspace_bytes(tiles, splits, cfg.block_m, cfg.block_n)
     stream = _native.current_stream_handle(a.device)
     workspace = _native.splitk_workspace(a.device, stream, nbytes)
-    status = _native.library().moegemm_matmul_splitk_transposed(
+    status = _native.library().moegemm_matmul_splitk_any(
         a.data_ptr(), b.data_ptr(), c.data_ptr(), m, n, k,
-        a.stride(0), a.stride(1), b.stride(0), b.stride(1), c.stride(0), c.stride(1), dtype_code,
+        a.stride(0), a.stride(1), b.stride(0), b.stride(1), c.stride(0), c.stride(1), dtype_code, precision,
         cfg.block_m, cfg.block_n, cfg.block_k, cfg.group_size_m, cfg.num_warps, cfg.num_stages, splits,
         0, workspace.data_ptr(), workspace.numel(), b_stream, stream,
     )
@@ -408,17 +417,18 @@ def _launch_fixed(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, precisio
         split_k = 1
     splits = 1
     layout = _operand_layout(a, b, c)
-    if layout == 0 or (layout > 0 and cfg.tile_key in _native.layout_tiles(dtype_code, layout)):
+    if layout == 0 or cfg.tile_key in _native.split_tiles(dtype_code, layout):
         tiles = -(-m // cfg.block_m) * -(-n // cfg.block_n)
         splits = split_k if split_k is not None else splitk_count(tiles, k, cfg.block_k,
                                                                   _device_signature(a.device) % 1000)
-        # Transposed operands take the unsplit launch where a workspace cannot be made (graph capture).
-        if splits > 1 and layout > 0 and not _native.splitk_workspace_ready(
+        # Other operands than row-major ones take the unsplit launch where a workspace cannot be made
+        # (graph capture).
+        if splits > 1 and layout != 0 and not _native.splitk_workspace_ready(
                 a.device, _native.current_stream_handle(a.device),
                 _native.splitk_workspace_bytes(tiles, splits, cfg.block_m, cfg.block_n)):
             splits = 1
     if splits > 1:
-        _launch_fixed_splitk(a, b, c, m, n, k, cfg, dtype_code, splits, b_stream)
+        _launch_fixed_splitk(a, b, c, m, n, k, cfg, dtype_code, splits, b_stream, precision)
         return splits
     lib = _native.library()
     status = lib.moegemm_matmul(
@@ -474,8 +484,13 @@ def launch_matmul(
         layout = _operand_layout(a, b, c)
         tiles = _native.layout_tiles(dtype_code, layout) if layout > 0 else None
         configs = matmul_candidate_configs(m, n, k, dtype=a.dtype, sm_count=sm_count, tiles=tiles)
+        general = _native.split_tiles(dtype_code, layout) if layout == _native.GENERAL else None
+        if general is not None:  # the tiles that can split K join what the shape family gives
+            configs += tuple(c for c in config_pool(a.dtype)
+                             if c.tile_key in general and c.group_size_m == 8 and c not in configs
+                             and c.block_m <= max(16, 2 * m) and c.block_n <= max(64, 2 * n))
         options = with_split_options(configs, lambda cfg: -(-m // cfg.block_m) * -(-n // cfg.block_n), k,
-                                     sm_count, split_k, layout >= 0)
+                                     sm_count, split_k, layout >= 0, general)
         if split_k is None:  # a stream-K tail where the tiles leave a partial last round
             options += [(cfg, STREAMK) for cfg in configs if _streamk_tail(a, b, c, m, n, k, cfg)]
         options = [(cfg, split, b_stream or 0) for cfg, split in options]

@@ -117,3 +117,87 @@ def test_fp32_values_outside_the_split_range(precision):
             # 72 products per sum: each fp32 rounding is within 2^-24 of the absolute values' sum.
             bound = 72 * 2.0**-24 * (a.cpu().double().abs() @ b.cpu().double().abs())
             assert ((got - reference).abs() <= bound)[finite].all(), (value, cfg)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+@pytest.mark.parametrize("shape", [(3, 300, 5), (70, 1029, 67), (257, 640, 261)])
+def test_split_k_of_the_general_tiles(shape, dtype):
+    """Every split tile and several counts, odd extents (the last range ends inside a chunk)."""
+    from kernels import _native
+    from kernels.matmul import last_matmul_split, launch_matmul
+
+    m, k, n = shape
+    gen = torch.Generator(device="cuda").manual_seed(m + k + n)
+    code = _native.dtype_code(dtype)
+    for transposed in ((False, False), (True, True)):
+        a = _view(m, k, transposed[0], 1, 3, dtype, gen)
+        b = _view(k, n, transposed[1], 3, 1, dtype, gen)
+        expected = (a.double() @ b.double()).to(dtype)
+        for cfg in _tiles(dtype):
+            if cfg.tile_key not in _native.split_tiles(code, _native.GENERAL):
+                continue
+            for splits in (2, 3, 7):
+                print(f"general split {cfg.tile_key} shape={shape} {transposed} {dtype} splits={splits}", flush=True)
+                for precision in ("ieee", "tf32") if dtype == torch.float32 else ("ieee",):
+                    c = torch.full((m, n + 3), float("nan"), device="cuda", dtype=dtype)[:, 1:n + 1]
+                    launch_matmul(a, b, c, cfg, precision, autotune=False, split_k=splits)
+                    torch.cuda.synchronize()
+                    assert last_matmul_split() == splits
+                    assert torch.equal(c, expected), (cfg, splits, precision)
+
+
+def test_split_k_groups_strides_range_and_capture():
+    """A homogeneous fp32 group; operands only Plain can stage (unit 0 computes the tile); a value
+    outside the split range in one unit of a tile; and capture before any workspace exists."""
+    from kernels.grouped_gemm import launch_grouped, workspace_from_tensors
+    from kernels.matmul import KernelConfig, last_matmul_split, launch_matmul
+
+    gen = torch.Generator(device="cuda").manual_seed(4)
+
+    def ints(*shape):
+        return torch.randint(-2, 3, shape, generator=gen, device="cuda").float()
+
+    cfg = KernelConfig(64, 64, 32, 2, 4, 2)
+    a, b = [ints(70, 515) for _ in range(3)], [ints(515, 130) for _ in range(3)]
+    ws = workspace_from_tensors(a, b, [torch.full((70, 130), float("nan"), device="cuda") for _ in range(3)])
+    print("general split group", flush=True)
+    launch_grouped(ws, config=cfg, autotune=False, split_k=4)
+    torch.cuda.synchronize()
+    assert ws.split_k == 4
+    for x, y, z in ws.problem_tensors():
+        assert torch.equal(z, (x.double() @ y.double()).float())
+
+    print("general split, strided operands", flush=True)
+    x, y = ints(70, 1030)[:, ::2], ints(515, 130)
+    c = torch.full((70, 130), float("nan"), device="cuda")
+    launch_matmul(x, y, c, cfg, autotune=False, split_k=4)
+    torch.cuda.synchronize()
+    assert torch.equal(c, (x.double() @ y.double()).float())
+
+    print("general split, infinity", flush=True)
+    x = ints(70, 515)
+    x[5, 300] = float("inf")
+    y = y.abs() + 1
+    for _ in range(2):  # the counters are re-armed
+        c.fill_(float("nan"))
+        launch_matmul(x, y, c, cfg, autotune=False, split_k=4)
+        torch.cuda.synchronize()
+        assert torch.isinf(c[5]).all()
+        rest = [i for i in range(70) if i != 5]
+        assert torch.equal(c[rest], (x[rest].double() @ y.double()).float())
+
+    x = ints(70, 515)
+    expected = (x.double() @ y.double()).float()
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    c.fill_(float("nan"))
+    torch.cuda.synchronize()
+    print("general split under capture", flush=True)
+    with torch.cuda.graph(graph, stream=stream):
+        launch_matmul(x, y, c, cfg, autotune=False, split_k=4)
+    assert last_matmul_split() == 1  # no workspace of this stream yet: the unsplit launch
+    for _ in range(3):
+        c.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c, expected)

@@ -34,9 +34,9 @@ def test_layout_rule_matches_the_library():
             views.append(storage.as_strided((rows, cols), strides, rng.choice((0, 0, 8, 4, 1))))
         a, b, c = views
         layout = _operand_layout(a, b, c)
-        status = _native.library().moegemm_matmul_splitk_transposed(
+        status = _native.library().moegemm_matmul_splitk_any(
             a.data_ptr(), b.data_ptr(), c.data_ptr(), m, n, k, *a.stride(), *b.stride(), *c.stride(),
-            _native.DTYPE_BF16, 64, 64, 64, 8, 4, 4, 2, 0, None, 0, 0, None)
+            _native.DTYPE_BF16, 0, 128, 256, 64, 8, 8, 3, 2, 0, None, 0, 0, None)
         assert status == _native.ERR_INVALID
         accepted = "workspace" in _native.last_error()
         assert accepted != ("vector layout" in _native.last_error())
