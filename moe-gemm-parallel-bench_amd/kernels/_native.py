@@ -372,4 +372,6 @@ def precision_code(input_precision: str, dtype_code_value: int) -> int:
 def current_stream_handle(device) -> int:
     import torch
 
-    return int(torch.cuda.current_stream(device).cuda_stream)
+    # The raw handle: building a torch.cuda.Stream object for it took about 2 us of a 11 us call.
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)

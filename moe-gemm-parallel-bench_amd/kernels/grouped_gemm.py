@@ -39,6 +39,7 @@ from .matmul import (
     layout_config,
     matmul_candidate_configs,
     select_config,
+    select_ragged_config,
 )
 
 _CTA_MULTIPLIERS = (1, 2, 4)
@@ -236,9 +237,14 @@ def workspace_from_tensors(arrays_a, arrays_b, arrays_c, config: KernelConfig | 
     for tensor in (*arrays_a, *arrays_b, *arrays_c):
         if tensor.device != device or tensor.dtype != dtype:
             raise ValueError("every grouped tensor must share one device and dtype")
-    first_m, first_k, first_n = normalized[0]
-    default_config = None if config else select_config(first_m, first_n, first_k, dtype)
-    config = config or default_config
+    default_config = None
+    if config is None:
+        rows, ks, ns = zip(*normalized)
+        if len(normalized) > 1 and len(set(rows)) > 1:  # unequal row counts: what a router gives
+            default_config = select_ragged_config(max(1, sum(rows) // len(rows)), max(ns), max(ks), dtype)
+        else:
+            default_config = select_config(rows[0], ns[0], ks[0], dtype)
+        config = default_config
 
     def pointer_table(arrays):
         return torch.tensor([t.data_ptr() for t in arrays], device=device, dtype=torch.int64)
@@ -518,7 +524,7 @@ def launch_grouped(
         raise ValueError(f"the {tile_schedule} schedule runs unsplit launches only (split_k must be 1)")
     if b_stream not in (None, 0, 1):
         raise ValueError(f"b_stream must be None, 0 or 1, got {b_stream!r}")
-    _require_runtime()
+    _require_runtime(workspace.a[0])
     cfg = config or workspace.config
     if workspace.problem_count == 1:
         launch_matmul(workspace.a[0], workspace.b[0], workspace.c[0], cfg, input_precision, autotune=autotune,

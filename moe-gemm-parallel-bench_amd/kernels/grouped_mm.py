@@ -30,7 +30,15 @@ from itertools import accumulate
 
 from . import _native
 from .grouped_gemm import grouped_candidate_configs
-from .matmul import KernelConfig, _device_signature, _require_runtime, _tune, config_pool, select_config
+from .matmul import (
+    KernelConfig,
+    _device_signature,
+    _require_runtime,
+    _tune,
+    config_pool,
+    select_config,
+    select_ragged_config,
+)
 
 
 def offsets_tile_bound(rows: int, group_count: int, n: int, block_m: int, block_n: int) -> int:
@@ -134,7 +142,7 @@ def grouped_mm(mat_a, mat_b, offs, *, out=None, config: KernelConfig | None = No
     if b_stream not in (None, 0, 1):
         raise ValueError(f"b_stream must be None, 0 or 1, got {b_stream!r}")
     rows, k, n, groups = _validate(mat_a, mat_b, offs, out)
-    _require_runtime()
+    _require_runtime(mat_a)
     if out is None:
         out = torch.empty((rows, n), device=mat_a.device, dtype=mat_a.dtype)
     if rows == 0:
@@ -149,7 +157,7 @@ def grouped_mm(mat_a, mat_b, offs, *, out=None, config: KernelConfig | None = No
                       option[1], option[2])
 
     if config is not None or not autotune:
-        option = (config or select_config(mean_m, n, k, mat_a.dtype), tile_schedule or "static", b_stream or 0)
+        option = (config or select_ragged_config(mean_m, n, k, mat_a.dtype), tile_schedule or "static", b_stream or 0)
     else:
         key = (rows, k, n, groups, tuple(mat_a.stride()), tuple(mat_b.stride()), tuple(out.stride()),
                dtype_code, precision, _device_signature(mat_a.device), tile_schedule, b_stream)
@@ -206,7 +214,7 @@ def grouped_mm_swiglu(mat_a, mat_b, offs, *, out=None, config: KernelConfig | No
               and mat_a.data_ptr() % 16 == 0 and mat_b.data_ptr() % 16 == 0)
     if not vector:
         raise ValueError("the fused SwiGLU epilogue needs 16-byte aligned operands with K a multiple of 8")
-    _require_runtime()
+    _require_runtime(mat_a)
     if out is None:
         out = torch.empty((rows, f), device=mat_a.device, dtype=mat_a.dtype)
     if out.stride(0) % 4 or out.data_ptr() % 8:
@@ -230,7 +238,9 @@ def grouped_mm_swiglu(mat_a, mat_b, offs, *, out=None, config: KernelConfig | No
     if config is not None or not autotune:
         cfg = config
         if cfg is None:
-            cfg = next((c for c in config_pool(mat_a.dtype) if c.tile_key in allowed and c.group_size_m == 8), None)
+            cfg = select_ragged_config(max(1, rows // groups), n, k, mat_a.dtype)
+            if cfg.tile_key not in allowed:  # narrow outputs: the first tile that pairs gate and up
+                cfg = next((c for c in config_pool(mat_a.dtype) if c.tile_key in allowed and c.group_size_m == 8), None)
     else:
         key = (rows, k, n, groups, tuple(mat_a.stride()), tuple(mat_b.stride()), tuple(out.stride()), dtype_code,
                _device_signature(mat_a.device))

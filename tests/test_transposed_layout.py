@@ -132,3 +132,22 @@ def test_transposed_groups(layout, schedule):
         torch.cuda.synchronize()
         for x, y, z in zip(a, b, c):
             assert torch.equal(z, (x.double() @ y.double()).to(z.dtype))
+
+
+def test_untuned_ragged_configs_are_compiled():
+    from kernels.matmul import _menu, select_ragged_config
+
+    for dtype in (torch.bfloat16, torch.float16, torch.float32):
+        for mean in (1, 4, 5, 64, 256, 257, 4096):
+            for n in (1, 64, 128, 129, 1023, 1024, 7168):
+                assert select_ragged_config(mean, n, 512, dtype).tile_key in _menu(dtype)
+
+
+def test_unequal_groups_default_to_the_ragged_rule():
+    from kernels.grouped_gemm import build_grouped_workspace
+    from kernels.matmul import select_config, select_ragged_config
+
+    ragged = build_grouped_workspace([(8, 64, 256), (40, 64, 256), (72, 64, 256)], torch.bfloat16, device="cpu")
+    assert ragged.config == select_ragged_config(40, 256, 64, torch.bfloat16)
+    equal = build_grouped_workspace([(40, 64, 256)] * 3, torch.bfloat16, device="cpu")
+    assert equal.config == select_config(40, 256, 64, torch.bfloat16)
