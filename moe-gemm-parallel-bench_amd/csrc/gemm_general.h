@@ -42,8 +42,8 @@
 //    (gemm_fast.h, split_store); nobody waits for another unit.
 //  * Range.  The split is exact and its products neither overflow nor lose their small parts while
 //    every non-zero operand lies in [2^-96, 2^60).  Each thread keeps the extremes of what it
-//    loaded; a tile that met a value outside (infinities and NaN included) is computed again by GemmTile, with the fp32
-//    instruction.
+//    loaded, and the accumulators show overflow; a tile that left the range (infinities and NaN
+//    included) is computed again by GemmTile, with the fp32 instruction.
 #pragma once
 
 #include "gemm_fast.h"
@@ -211,8 +211,12 @@ struct GeneralTile {
     return h;
   }
 
-  // The chunk's bf16 parts.  range[0]: the largest |x| seen (as float bits; a NaN stays), range[1]: the
-  // smallest non-zero |x| (as twice its bits, less one: zero wraps to the top).
+  // The chunk's bf16 parts.  range[1]: the smallest non-zero |x| seen (as twice its bits, less one: zero
+  // wraps to the top).  range[0], TF32 only: the largest |x| (as float bits; a NaN stays), because
+  // rounding can turn a NaN into a number.  In IEEE mode large values need no watch: whatever
+  // overflows in the parts or their products (infinities and NaN too) leaves an accumulator that is
+  // not finite (all_finite).  The register it saves ended spills in the 256x128 loop: 214 -> 185 us on
+  // 8 x [512,2048]@[2048,1536].
   __device__ static __forceinline__ void split(const u32x4_t (&in)[VL], u32x4_t (&part)[PARTS], uint32_t (&range)[2]) {
     if constexpr (!F32) {
       part[0] = in[0];
@@ -220,7 +224,7 @@ struct GeneralTile {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         uint32_t u0 = in[(2 * i) / 4][(2 * i) % 4], u1 = in[(2 * i + 1) / 4][(2 * i + 1) % 4];
-        asm("v_maximum3_f32 %0, %0, |%1|, |%2|" : "+v"(range[0]) : "v"(u0), "v"(u1));
+        if constexpr (PARTS == 2) asm("v_maximum3_f32 %0, %0, |%1|, |%2|" : "+v"(range[0]) : "v"(u0), "v"(u1));
         range[1] = min(min(range[1], (u0 << 1) - 1u), (u1 << 1) - 1u);
         if constexpr (PARTS == 2) {  // TF32: 10-bit mantissa, ties away (NaN leaves by its range)
           u0 = (u0 + 0x1000u) & 0xffffe000u;
@@ -236,6 +240,16 @@ struct GeneralTile {
         }
       }
     }
+  }
+  __device__ static __forceinline__ bool all_finite(const acc_t (&acc)[FM][FN]) {
+    float worst = 0.0f;  // x - x is zero exactly when x is finite
+#pragma unroll
+    for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+      for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+        for (int i = 0; i < ACC; ++i) worst += acc[fm][fn][i] - acc[fm][fn][i];
+    return worst == 0.0f;
   }
   // Bits of 2^60, and twice those of 2^-96 less one.
   static constexpr uint32_t kTooLarge = (127u + 60u) << 23;
@@ -523,7 +537,7 @@ struct GeneralTile {
     compute(acc, smem + (last & 1) * STAGE_BYTES, fa, fb);
     bool bad = false;
     if constexpr (F32)  // also the barrier between this tile's LDS reads and the next tile's writes
-      bad = __syncthreads_or(range[0] >= kTooLarge || range[1] < kTooSmall) != 0;
+      bad = __syncthreads_or(range[1] < kTooSmall || (PARTS == 2 ? range[0] >= kTooLarge : !all_finite(acc))) != 0;
     else
       __syncthreads();
     if constexpr (EPI == EPI_SPLIT) {
