@@ -307,11 +307,18 @@ def _refuse_allocation_under_capture(what: str) -> None:
                            "capture; make the first call on this stream outside capture")
 
 
-def splitk_workspace_ready(device, stream_handle: int, nbytes: int) -> bool:
-    """Whether ``splitk_workspace`` can serve this call: held already, or not under graph capture."""
+_SPLITK_MAX_SPLITS, _SPLITK_MAX_TILES = 64, 65536  # the split-K launches' limits (moegemm.h)
+
+
+def splitk_serves(device, stream_handle: int, tiles: int, splits: int, block_m: int, block_n: int) -> bool:
+    """Whether a split launch can be made: within the library's limits, and its workspace is held
+    already or can be made (not under graph capture)."""
     import torch
 
+    if splits > _SPLITK_MAX_SPLITS or tiles > _SPLITK_MAX_TILES:
+        return False
     held = _SPLITK_WORKSPACES.get((torch.device(device).index or 0, int(stream_handle)))
+    nbytes = splitk_workspace_bytes(tiles, splits, block_m, block_n)
     return bool(held and held[-1].numel() >= nbytes) or not torch.cuda.is_current_stream_capturing()
 
 

@@ -382,10 +382,11 @@ def _grouped_splits(workspace: GroupedWorkspace, cfg: KernelConfig, dtype_code: 
         return 1
     tiles = workspace.tile_count_for(cfg)
     splits = split_k if split_k is not None else splitk_count(tiles, workspace.max_k, cfg.block_k, workspace.sm_count)
-    # General tiles take the unsplit launch where a workspace cannot be made (graph capture).
-    if splits > 1 and layout != 0 and not _native.splitk_workspace_ready(
-            workspace.a[0].device, _native.current_stream_handle(workspace.a[0].device),
-            _native.splitk_workspace_bytes(tiles, splits, cfg.block_m, cfg.block_n)):
+    # General tiles take the unsplit launch where a split one cannot be made (graph capture before the
+    # workspace exists, or a named split_k past the library's limits).
+    if splits > 1 and layout != 0 and not _native.splitk_serves(
+            workspace.a[0].device, _native.current_stream_handle(workspace.a[0].device), tiles, splits,
+            cfg.block_m, cfg.block_n):
         splits = 1
     return splits
 

@@ -442,11 +442,10 @@ def _launch_fixed(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, precisio
         tiles = -(-m // cfg.block_m) * -(-n // cfg.block_n)
         splits = split_k if split_k is not None else splitk_count(tiles, k, cfg.block_k,
                                                                   _device_signature(a.device) % 1000)
-        # Other operands than row-major ones take the unsplit launch where a workspace cannot be made
-        # (graph capture).
-        if splits > 1 and layout != 0 and not _native.splitk_workspace_ready(
-                a.device, _native.current_stream_handle(a.device),
-                _native.splitk_workspace_bytes(tiles, splits, cfg.block_m, cfg.block_n)):
+        # Other operands than row-major ones take the unsplit launch where a split one cannot be made
+        # (graph capture before the workspace exists, or a named split_k past the library's limits).
+        if splits > 1 and layout != 0 and not _native.splitk_serves(
+                a.device, _native.current_stream_handle(a.device), tiles, splits, cfg.block_m, cfg.block_n):
             splits = 1
     if splits > 1:
         _launch_fixed_splitk(a, b, c, m, n, k, cfg, dtype_code, splits, b_stream, precision)

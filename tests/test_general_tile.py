@@ -201,3 +201,27 @@ def test_split_k_groups_strides_range_and_capture():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(c, expected)
+
+
+@pytest.mark.parametrize("shape,splits", [((70, 515, 67), 65), ((16 * 257, 64, 64 * 256), 2)])
+def test_split_k_past_the_limits_runs_whole(shape, splits):
+    """More splits, or more tiles, than a split launch takes: fp32 calls that name them run unsplit."""
+    from kernels.grouped_gemm import launch_grouped, workspace_from_tensors
+    from kernels.matmul import KernelConfig, last_matmul_split, launch_matmul
+
+    m, k, n = shape
+    cfg = KernelConfig(16, 64, 32, 8, 4, 2)
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    a = torch.randint(-2, 3, (m, k), generator=gen, device="cuda").float()
+    b = torch.randint(-2, 3, (k, n), generator=gen, device="cuda").float()
+    c = [torch.full((m, n), float("nan"), device="cuda") for _ in range(2)]
+    print(f"split past the limits shape={shape} splits={splits}", flush=True)
+    launch_matmul(a, b, c[0], cfg, autotune=False, split_k=splits)
+    assert last_matmul_split() == 1
+    ws = workspace_from_tensors([a, a], [b, b], [torch.empty_like(c[0]), c[1]])
+    launch_grouped(ws, config=cfg, autotune=False, split_k=splits)
+    assert ws.split_k == 1
+    torch.cuda.synchronize()
+    expected = (a.double() @ b.double()).float()
+    for out in (c[0], c[1], ws.c[0]):
+        assert torch.equal(out, expected)
