@@ -38,6 +38,7 @@ from .matmul import (
     launch_matmul,
     layout_config,
     matmul_candidate_configs,
+    ragged_b_stream,
     select_config,
     select_ragged_config,
 )
@@ -79,6 +80,7 @@ class GroupedWorkspace:
     tile_schedule: str = "static"
     b_stream: int = 0  # 1: the last launch issued its B copies non-temporal
     default_config: KernelConfig | None = None  # what select_config gave when no config was named
+    default_b_stream: int = 0  # the B copy policy that goes with it
     swiglu_b_stream: int = 0  # the same for the last launch_gate_up_swiglu call
 
     @property
@@ -237,11 +239,14 @@ def workspace_from_tensors(arrays_a, arrays_b, arrays_c, config: KernelConfig | 
     for tensor in (*arrays_a, *arrays_b, *arrays_c):
         if tensor.device != device or tensor.dtype != dtype:
             raise ValueError("every grouped tensor must share one device and dtype")
-    default_config = None
+    default_config, default_b_stream = None, 0
     if config is None:
         rows, ks, ns = zip(*normalized)
         if len(normalized) > 1 and len(set(rows)) > 1:  # unequal row counts: what a router gives
-            default_config = select_ragged_config(max(1, sum(rows) // len(rows)), max(ns), max(ks), dtype)
+            mean_m = max(1, sum(rows) // len(rows))
+            default_config = select_ragged_config(mean_m, max(ns), max(ks), dtype)
+            if dtype.itemsize == 2:
+                default_b_stream = ragged_b_stream(mean_m, 2 * sum(k * n for k, n in zip(ks, ns)))
         else:
             default_config = select_config(rows[0], ns[0], ks[0], dtype)
         config = default_config
@@ -272,7 +277,7 @@ def workspace_from_tensors(arrays_a, arrays_b, arrays_c, config: KernelConfig | 
         normalized, config, _shape_signature(normalized), device_signature, sm_count, storage_bytes,
         homogeneous,
     )
-    workspace.default_config = default_config
+    workspace.default_config, workspace.default_b_stream = default_config, default_b_stream
     return workspace
 
 
@@ -514,8 +519,9 @@ def launch_grouped(
     count leaves a partial last round, static otherwise); None lets the tuner measure them
     (static without autotuning).  ``workspace.tile_schedule`` records what ran.  ``b_stream``
     (keyword-only, not in the reference's signature): 1 issues the LDS-DMA kernels' B copies
-    non-temporal, 0 as ordinary loads, None lets the tuner measure both on its finalists (0 without
-    autotuning); ``workspace.b_stream`` records what ran.  G == 1 always runs the single GEMM.
+    non-temporal, 0 as ordinary loads, None lets the tuner measure both on its finalists (without
+    autotuning ``ragged_b_stream``'s choice for unequal problems, else 0); ``workspace.b_stream``
+    records what ran.  G == 1 always runs the single GEMM.
     """
     if split_k is not None and split_k < 1:
         raise ValueError("split_k must be None or a positive integer")
@@ -574,6 +580,8 @@ def launch_grouped(
         if schedule in ("stealing", "streamk") and split_k is None:
             split_k = 1
         if config is None and cfg is workspace.default_config:
+            if b_stream is None and layout == 0:
+                stream_b = workspace.default_b_stream
             cfg = layout_config(cfg, dtype_code, layout, workspace.a[0].dtype)
     workspace.split_k = _launch_grouped_fixed(workspace, cfg, dtype_code, precision, split_k, schedule, stream_b,
                                               layout)

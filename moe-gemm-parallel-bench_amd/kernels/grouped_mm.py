@@ -36,6 +36,7 @@ from .matmul import (
     _require_runtime,
     _tune,
     config_pool,
+    ragged_b_stream,
     select_config,
     select_ragged_config,
 )
@@ -133,7 +134,8 @@ def grouped_mm(mat_a, mat_b, offs, *, out=None, config: KernelConfig | None = No
     even split of ``rows`` over the groups.  ``tile_schedule``: "static", "stealing" (per-XCD
     work-stealing tile queues), or None to let the tuner measure both (static otherwise).
     ``b_stream``: 1 issues the LDS-DMA kernels' B copies non-temporal, 0 as ordinary loads, None lets
-    the tuner measure both on its finalists (0 without autotuning).
+    the tuner measure both on its finalists (``ragged_b_stream``'s choice without autotuning, 0 with a
+    ``config``).
     """
     import torch
 
@@ -156,8 +158,12 @@ def grouped_mm(mat_a, mat_b, offs, *, out=None, config: KernelConfig | None = No
         _launch_fixed(mat_a, mat_b, offs, out, rows, k, n, groups, option[0], dtype_code, precision, sm_count,
                       option[1], option[2])
 
-    if config is not None or not autotune:
-        option = (config or select_ragged_config(mean_m, n, k, mat_a.dtype), tile_schedule or "static", b_stream or 0)
+    if config is not None:
+        option = (config, tile_schedule or "static", b_stream or 0)
+    elif not autotune:
+        if b_stream is None:
+            b_stream = ragged_b_stream(mean_m, 2 * groups * k * n) if mat_a.element_size() == 2 else 0
+        option = (select_ragged_config(mean_m, n, k, mat_a.dtype), tile_schedule or "static", b_stream)
     else:
         key = (rows, k, n, groups, tuple(mat_a.stride()), tuple(mat_b.stride()), tuple(out.stride()),
                dtype_code, precision, _device_signature(mat_a.device), tile_schedule, b_stream)
@@ -225,20 +231,23 @@ def grouped_mm_swiglu(mat_a, mat_b, offs, *, out=None, config: KernelConfig | No
     sm_count = _device_signature(mat_a.device) % 1000
     allowed = _native.swiglu_tiles(dtype_code)
 
-    def launch(cfg):
+    def launch(cfg, b_stream=0):
         grid = max(1, min(offsets_tile_bound(rows, groups, n, cfg.block_m, cfg.block_n), sm_count * cfg.cta_multiplier))
         status = _native.library().moegemm_grouped_mm_offs_swiglu(
             mat_a.data_ptr(), mat_b.data_ptr(), out.data_ptr(), offs.data_ptr(), groups, rows, n, k,
             mat_a.stride(0), mat_b.stride(0), mat_b.stride(1), out.stride(0), dtype_code,
             cfg.block_m, cfg.block_n, cfg.block_k, cfg.group_size_m, cfg.num_warps, cfg.num_stages, grid,
-            0, _native.current_stream_handle(mat_a.device),
+            b_stream, _native.current_stream_handle(mat_a.device),
         )
         _native.check(status)
 
+    stream_b = 0
     if config is not None or not autotune:
         cfg = config
         if cfg is None:
-            cfg = select_ragged_config(max(1, rows // groups), n, k, mat_a.dtype)
+            mean_m = max(1, rows // groups)
+            stream_b = ragged_b_stream(mean_m, 2 * groups * k * n)
+            cfg = select_ragged_config(mean_m, n, k, mat_a.dtype)
             if cfg.tile_key not in allowed:  # narrow outputs: the first tile that pairs gate and up
                 cfg = next((c for c in config_pool(mat_a.dtype) if c.tile_key in allowed and c.group_size_m == 8), None)
     else:
@@ -253,7 +262,7 @@ def grouped_mm_swiglu(mat_a, mat_b, offs, *, out=None, config: KernelConfig | No
                 [c for c in config_pool(mat_a.dtype) if c.tile_key in allowed and c.group_size_m == 8][:6]
             cfg = _tune(candidates, launch)
             _SWIGLU_OFFSETS_CACHE[key] = cfg
-    launch(cfg)
+    launch(cfg, stream_b)
     _LAST_SWIGLU_CONFIG[0] = cfg
     return out
 

@@ -144,6 +144,23 @@ def select_ragged_config(mean_m: int, n: int, k: int, dtype=None) -> KernelConfi
     return KernelConfig(256, 256, 32, 8, 8, 4)
 
 
+_MEMORY_SIDE_CACHE = 256 << 20  # bytes
+
+
+def ragged_b_stream(mean_m: int, weight_bytes: int) -> int:
+    """B copy policy of an untuned group of unequal problems: 1 (non-temporal) where B comes from HBM and
+    is read about once.
+
+    Up to 64 rows a problem is mostly one 128-row tile.  Measured on bf16 groups larger than the cache
+    (7 K x N from 2880 x 5760 to 1024 x 7168; expert-sorted, fused SwiGLU and pointer groups): 1 to 32
+    rows run in 0.86 to 0.97 of the time of ordinary copies, 64 rows in 0.95 to 1.02; from 128 rows on,
+    where M tiles share B panels in L2, ordinary copies are up to 26 % faster.  Weights that stay in the
+    256 MiB memory-side cache from call to call are up to 23 % slower non-temporal (16 x [2048,1408]:
+    22 -> 27 us), so the bytes of the experts that hold rows, about 1 - e^-mean of them, must exceed it:
+    at 384 MiB, repeated calls on the same weights run in 0.91 to 0.98."""
+    return int(mean_m <= 64 and weight_bytes * (1 - math.exp(-mean_m)) > _MEMORY_SIDE_CACHE)
+
+
 def diverse_configs(ordered: list[KernelConfig], limit: int) -> list[KernelConfig]:
     """Truncate a best-first list to ``limit`` while covering distinct tile/traversal choices.
 

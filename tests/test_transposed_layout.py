@@ -151,3 +151,53 @@ def test_unequal_groups_default_to_the_ragged_rule():
     assert ragged.config == select_ragged_config(40, 256, 64, torch.bfloat16)
     equal = build_grouped_workspace([(40, 64, 256)] * 3, torch.bfloat16, device="cpu")
     assert equal.config == select_config(40, 256, 64, torch.bfloat16)
+
+
+@pytest.mark.parametrize("mean,mib,expected", [(64, 257, 1), (65, 4096, 0), (4, 256, 0), (1, 384, 0), (1, 512, 1)])
+def test_untuned_b_stream_rule(mean, mib, expected):
+    from kernels.matmul import ragged_b_stream
+
+    assert ragged_b_stream(mean, mib << 20) == expected
+
+
+@pytest.mark.gpu
+def test_untuned_routed_groups_stream_large_weights():
+    """Above the cache's size all three untuned routes run non-temporal copies; a named policy, a named
+    config and small weights keep theirs; the results are the same bytes."""
+    if not torch.cuda.is_available():
+        pytest.skip("ROCm GPU unavailable")
+    from kernels import grouped_mm
+    from kernels.grouped_gemm import launch_grouped, workspace_from_tensors
+    from kernels.grouped_mm import last_grouped_mm_b_stream, last_grouped_mm_config
+
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    rows = [5, 0, 40, 3, 16, 1, 0, 31]
+    g, k, n = len(rows), 4096, 4608  # 288 MiB
+    a = torch.randint(-1, 2, (sum(rows), k), generator=gen, device="cuda").to(torch.bfloat16)
+    b = torch.randint(-1, 2, (g, k, n), generator=gen, device="cuda", dtype=torch.int8).to(torch.bfloat16)
+    offs = torch.tensor(rows, device="cuda").cumsum(0).to(torch.int32)
+    print("untuned b_stream, expert-sorted", flush=True)
+    streamed = grouped_mm(a, b, offs, autotune=False)
+    assert last_grouped_mm_b_stream() == 1
+    plain = grouped_mm(a, b, offs, autotune=False, b_stream=0)
+    assert last_grouped_mm_b_stream() == 0
+    grouped_mm(a, b, offs, config=last_grouped_mm_config())
+    assert last_grouped_mm_b_stream() == 0
+    grouped_mm(a, b[:, :, :4096].contiguous(), offs, autotune=False)  # 256 MiB
+    assert last_grouped_mm_b_stream() == 0
+    first, spans = 0, []
+    for e, count in enumerate(rows):
+        if count:
+            spans.append((e, first, first + count))
+        first += count
+    expected = torch.cat([(a[x:y].double() @ b[e].double()).to(a.dtype) for e, x, y in spans])
+    assert torch.equal(streamed, expected) and torch.equal(plain, expected)
+    print("untuned b_stream, pointer group", flush=True)
+    c = torch.empty_like(expected)
+    spans = spans + [(1, 0, 5), (6, 5, 45)]  # every expert's weights
+    outs = [c[x:y] for _, x, y in spans[:-2]] + [torch.empty_like(c[x:y]) for _, x, y in spans[-2:]]
+    ws = workspace_from_tensors([a[x:y] for _, x, y in spans], [b[e] for e, _, _ in spans], outs)
+    launch_grouped(ws, autotune=False)
+    assert ws.b_stream == 1
+    torch.cuda.synchronize()
+    assert torch.equal(c, expected)
