@@ -239,12 +239,19 @@ def workspace_from_tensors(arrays_a, arrays_b, arrays_c, config: KernelConfig | 
     for tensor in (*arrays_a, *arrays_b, *arrays_c):
         if tensor.device != device or tensor.dtype != dtype:
             raise ValueError("every grouped tensor must share one device and dtype")
+    if device.type == "cuda":
+        props = torch.cuda.get_device_properties(device)
+        sm_count = int(props.multi_processor_count)
+        device_signature = (int(props.major) * 10 + int(props.minor)) * 1000 + sm_count
+    else:
+        sm_count, device_signature = 0, 0
     default_config, default_b_stream = None, 0
     if config is None:
         rows, ks, ns = zip(*normalized)
         if len(normalized) > 1 and len(set(rows)) > 1:  # unequal row counts: what a router gives
             mean_m = max(1, sum(rows) // len(rows))
-            default_config = select_ragged_config(mean_m, max(ns), max(ks), dtype)
+            default_config = select_ragged_config(mean_m, max(ns), max(ks), dtype, groups=len(rows), rows=rows,
+                                                  sm_count=sm_count or 256)
             if dtype.itemsize == 2:
                 default_b_stream = ragged_b_stream(mean_m, 2 * sum(k * n for k, n in zip(ks, ns)))
         else:
@@ -263,12 +270,6 @@ def workspace_from_tensors(arrays_a, arrays_b, arrays_c, config: KernelConfig | 
     )
     tables = [a_ptrs, b_ptrs, c_ptrs, dims, strides]
     storage_bytes = sum(t.numel() * t.element_size() for t in (*arrays_a, *arrays_b, *arrays_c, *tables))
-    if device.type == "cuda":
-        props = torch.cuda.get_device_properties(device)
-        sm_count = int(props.multi_processor_count)
-        device_signature = (int(props.major) * 10 + int(props.minor)) * 1000 + sm_count
-    else:
-        sm_count, device_signature = 0, 0
     homogeneous = all(s == normalized[0] for s in normalized) and all(
         t.is_contiguous() for t in (*arrays_a, *arrays_b, *arrays_c)
     )

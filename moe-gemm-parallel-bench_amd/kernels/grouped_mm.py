@@ -163,7 +163,8 @@ def grouped_mm(mat_a, mat_b, offs, *, out=None, config: KernelConfig | None = No
     elif not autotune:
         if b_stream is None:
             b_stream = ragged_b_stream(mean_m, 2 * groups * k * n) if mat_a.element_size() == 2 else 0
-        option = (select_ragged_config(mean_m, n, k, mat_a.dtype), tile_schedule or "static", b_stream)
+        cfg = select_ragged_config(mean_m, n, k, mat_a.dtype, groups=groups, sm_count=sm_count)
+        option = (cfg, tile_schedule or "static", b_stream)
     else:
         key = (rows, k, n, groups, tuple(mat_a.stride()), tuple(mat_b.stride()), tuple(out.stride()),
                dtype_code, precision, _device_signature(mat_a.device), tile_schedule, b_stream)
@@ -247,7 +248,7 @@ def grouped_mm_swiglu(mat_a, mat_b, offs, *, out=None, config: KernelConfig | No
         if cfg is None:
             mean_m = max(1, rows // groups)
             stream_b = ragged_b_stream(mean_m, 2 * groups * k * n)
-            cfg = select_ragged_config(mean_m, n, k, mat_a.dtype)
+            cfg = select_ragged_config(mean_m, n, k, mat_a.dtype, groups=groups, sm_count=sm_count, tiles=allowed)
             if cfg.tile_key not in allowed:  # narrow outputs: the first tile that pairs gate and up
                 cfg = next((c for c in config_pool(mat_a.dtype) if c.tile_key in allowed and c.group_size_m == 8), None)
     else:

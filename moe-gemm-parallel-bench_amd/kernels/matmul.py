@@ -124,8 +124,19 @@ def select_config(m: int, n: int, k: int, dtype=None) -> KernelConfig:
     return _snap(256, 256 if n > 128 else 128, 64, dtype)
 
 
-def select_ragged_config(mean_m: int, n: int, k: int, dtype=None) -> KernelConfig:
-    """Untuned config of a group whose problems hold ``mean_m`` rows on average, unevenly.
+# Shortest K step first: 4.4, 5.5, 7.7 and 9.0 ns per unit of K with one workgroup a CU (128x256: 13.3).
+_FEW_TILES = ((16, 64, 128, 4, 4), (64, 64, 64, 4, 4), (64, 128, 64, 4, 4), (128, 128, 64, 4, 4))
+
+
+def select_ragged_config(mean_m: int, n: int, k: int, dtype=None, *, groups: int, rows=None, sm_count: int = 256,
+                         tiles=None) -> KernelConfig:
+    """Untuned config of ``groups`` problems that hold ``mean_m`` rows on average, unevenly; ``rows`` are
+    the row counts where the host knows them, ``tiles`` the tile keys the call can take (None: all).
+
+    A group whose tiles all find a CU at once takes as long as one tile, so it takes the compiled tile
+    with the shortest K step that still fits in one round.  Measured on 3281 bf16 pointer groups (2 to
+    128 problems, 1 to 512 rows, K and N of 256 to 7168): 3.7 % behind the best of twelve tiles on
+    average, where 128x256 for all of them was 42 % behind and the first problem's tile 34 %.
 
     A problem with more rows than the tile reads its B panel once per M tile, and routed row counts
     spread to about twice their mean, so the tile is taller than the mean.  Measured on bf16 groups
@@ -133,15 +144,32 @@ def select_ragged_config(mean_m: int, n: int, k: int, dtype=None) -> KernelConfi
     SwiGLU and pointer groups): from 8 to 200 rows 128x256 with eight waves is within 6 % of the best
     compiled tile on 65 of 72 points (the others 7 to 26 %), where the tile nearest the mean was up to
     35 % behind it, the first tile that pairs gate and up up to 36 % and the first problem's row count
-    up to 65 %; at 400 rows 256x256 is up to 17 % ahead, and 20 % behind at N = 512; at 2 rows the 16-row
-    and the 128-row tile are level, and the short one computes less padding."""
+    up to 65 %; at 2 rows the 16-row and the 128-row tile are level, and the short one computes less
+    padding.  256x256 (ping-pong) is 3 to 30 % ahead of 128x256 at 256 rows on seven K x N, within 9 % of
+    it either way at 200 (17 % ahead at N = 512) and 2 to 43 % behind at 160 on six of the seven; below
+    1024 columns the order changes with every round of tiles.
+
+    Few rounds of tiles make that a matter of the counts: a round of 256x256 tiles takes about as long as
+    one and a half of 128x256 tiles, and the last round takes as long as a full one.  On 245 groups (96
+    to 400 rows, seven K x N, five routings each) choosing by rounds is 0.6 % behind the better of the
+    two on average (at most 13 %), the line at 224 rows 2.1 % (31 %)."""
     if _is_f32(dtype) or n <= 128:
         return select_config(mean_m, n, k, dtype)
+    for tile in _FEW_TILES:
+        if rows is not None:
+            m_tiles = sum(-(-m // tile[0]) for m in rows)
+        else:  # about half a partial tile a problem
+            m_tiles = groups * (mean_m / tile[0] + 0.5 if 2 * mean_m > tile[0] else 1)
+        if m_tiles * -(-n // tile[1]) <= sm_count and (tiles is None or tile in tiles):
+            return KernelConfig(*tile[:3], 8, *tile[3:])
     if mean_m <= 4:
         return KernelConfig(16, 256, 64, 8, 4, 4)
-    if mean_m <= 256 or n < 1024:
-        return KernelConfig(128, 256, 64, 8, 8, 3)
-    return KernelConfig(256, 256, 32, 8, 8, 4)
+    wide = mean_m > 224 and n >= 1024
+    if rows is not None and mean_m > 64:
+        def rounds(block_m):
+            return -(-sum(-(-m // block_m) for m in rows) * -(-n // 256) // sm_count)
+        wide = rounds(128) > 1.5 * rounds(256)
+    return KernelConfig(256, 256, 32, 8, 8, 4) if wide else KernelConfig(128, 256, 64, 8, 8, 3)
 
 
 _MEMORY_SIDE_CACHE = 256 << 20  # bytes

@@ -140,7 +140,8 @@ def test_untuned_ragged_configs_are_compiled():
     for dtype in (torch.bfloat16, torch.float16, torch.float32):
         for mean in (1, 4, 5, 64, 256, 257, 4096):
             for n in (1, 64, 128, 129, 1023, 1024, 7168):
-                assert select_ragged_config(mean, n, 512, dtype).tile_key in _menu(dtype)
+                for groups in (2, 32):
+                    assert select_ragged_config(mean, n, 512, dtype, groups=groups).tile_key in _menu(dtype)
 
 
 def test_unequal_groups_default_to_the_ragged_rule():
@@ -148,7 +149,16 @@ def test_unequal_groups_default_to_the_ragged_rule():
     from kernels.matmul import select_config, select_ragged_config
 
     ragged = build_grouped_workspace([(8, 64, 256), (40, 64, 256), (72, 64, 256)], torch.bfloat16, device="cpu")
-    assert ragged.config == select_ragged_config(40, 256, 64, torch.bfloat16)
+    assert ragged.config == select_ragged_config(40, 256, 64, torch.bfloat16, groups=3, rows=(8, 40, 72))
+    # Tiles that fit one round of 256 CUs: (1 + 3 + 5) M tiles of 16 rows by 4 (28, 29) N tiles of 64.
+    for n, tile in ((256, (16, 64)), (1792, (16, 64)), (1856, (64, 64))):
+        few = build_grouped_workspace([(8, 64, n), (40, 64, n), (72, 64, n)], torch.bfloat16, device="cpu")
+        assert (few.config.block_m, few.config.block_n) == tile
+    # 512 columns, 2 N tiles: 129 problems of up to 128 rows are two rounds of 256 CUs in either tile; of
+    # 129 to 256 rows three rounds of 128-row tiles against two, and 128 such problems two against one.
+    for tall, count, block_m in ((128, 129, 128), (256, 129, 128), (256, 128, 256)):
+        ws = build_grouped_workspace([(tall - i % 2, 8, 512) for i in range(count)], torch.bfloat16, device="cpu")
+        assert ws.config.block_m == block_m, (tall, count)
     equal = build_grouped_workspace([(40, 64, 256)] * 3, torch.bfloat16, device="cpu")
     assert equal.config == select_config(40, 256, 64, torch.bfloat16)
 
