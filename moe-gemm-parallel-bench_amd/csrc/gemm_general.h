@@ -2,7 +2,8 @@
 // (gfx950).
 //
 // Operands whose inner dimension is contiguous, at any alignment and of any extent of at least 8,
-// run here; the rest (other strides, tiny extents) runs GemmTile's element-wise staging.
+// run here; the rest (other strides, negative pitches, tiny extents: general_route.h) runs GemmTile's
+// element-wise staging.
 //
 //  * Staging.  Every thread owns fixed 8-element chunks of each K slice: 16 bytes (16-bit types) or
 //    two 16-byte loads (fp32), at whatever alignment the row has (gfx950 global loads need none).
@@ -48,6 +49,7 @@
 
 #include "gemm_fast.h"
 #include "gemm_kernel.h"
+#include "general_route.h"
 
 namespace moegemm {
 
@@ -98,7 +100,7 @@ struct GeneralTile {
   using vec_t = typename std::conditional<F32, u32x4_a4_t, u32x4_a2_t>::type;
 
   // One operand's chunks of this thread.  XC: rows run along the operand's M or N dimension x.
-  // Global addresses are a uniform base plus a 32-bit offset (the caller checked the pitch).
+  // Global addresses are a uniform base plus an unsigned 32-bit offset (chunk_route checked the pitch).
   template <bool XC, int BX, int PT>
   struct Operand {
     static constexpr int CPR = XC ? BX / 8 : BK / 8;  // chunks per LDS row
@@ -556,25 +558,19 @@ struct GeneralTile {
                                                   Hook&& before_store) {
     static_assert(EPI == EPI_C || EPI == EPI_SPLIT, "the general kernel has no stream-K tail");
     if (pd.swiglu || (EPI == EPI_C && pd.splits > 1)) return;  // the host launches neither
-    // 32-bit offsets span a tile's rows (K-contiguous) or a slice's (XC).
-    constexpr int64_t kPitchLimit = (int64_t(1) << 32) / (BM > BN ? BM : BN) / 2;
-    const bool a_rows = pd.sak == 1 && pd.k >= 8 && pd.sam * ES < kPitchLimit && (int64_t)pd.k * ES < (1ll << 31);
-    const bool deep = !F32 || pd.k >= 8;  // shorter fp32 sums are closer with the fp32 instruction
-    const bool a_cols = deep && BM >= 32 && pd.sam == 1 && pd.m >= 8 && pd.sak * ES < kPitchLimit;
-    const bool b_rows = pd.sbk == 1 && pd.k >= 8 && pd.sbn * ES < kPitchLimit && (int64_t)pd.k * ES < (1ll << 31);
-    const bool b_cols = deep && pd.sbn == 1 && pd.n >= 8 && pd.sbk * ES < kPitchLimit;
+    const ChunkRoute r = chunk_route(F32, ES, BM, BN, pd.m, pd.n, pd.k, pd.sam, pd.sak, pd.sbk, pd.sbn);
     bool done = false;
     if constexpr (EPI == EPI_SPLIT) {
       // Operands Plain must stage: unit 0 of each tile computes it whole.
-      if (!((a_rows || (BM >= 32 && a_cols)) && (b_rows || b_cols)) && pd.split != 0) return;
+      if (!r.chunked() && pd.split != 0) return;
     }
-    if (a_rows && b_cols) {
+    if (r.a_rows && r.b_cols) {
       done = chunk_tile<false, false, EPI>(pd, tm, tn, smem, before_store);
-    } else if (a_rows && b_rows) {
+    } else if (r.a_rows && r.b_rows) {
       done = chunk_tile<false, true, EPI>(pd, tm, tn, smem, before_store);
-    } else if (a_cols && (b_cols || b_rows)) {
+    } else if (r.chunked()) {
       if constexpr (BM >= 32) {
-        if (b_cols)
+        if (r.b_cols)
           done = chunk_tile<true, false, EPI>(pd, tm, tn, smem, before_store);
         else
           done = chunk_tile<true, true, EPI>(pd, tm, tn, smem, before_store);

@@ -1,0 +1,32 @@
+// Which operands the general tile stages in whole chunks (GeneralTile, gemm_general.h).  Plain C++, so
+// that the rule can be compiled and checked without a GPU.
+#pragma once
+
+#include <cstdint>
+
+namespace moegemm {
+
+// A chunk is 8 elements along an operand's unit stride; rows run along K, or (cols) along M or N.
+struct ChunkRoute {
+  bool a_rows, a_cols, b_rows, b_cols;
+  constexpr bool chunked() const { return (a_rows || a_cols) && (b_rows || b_cols); }
+};
+
+// Strides in elements of `es` bytes, of any sign.  The chunks' addresses are a 64-bit base plus an unsigned
+// 32-bit offset that spans a tile's rows (rows along K) or a slice's, so a pitch must not be negative
+// (such an offset would land 4 GiB past its row) and must stay below `limit`; an operand that does not
+// meet the rule is staged element by element with signed 64-bit indices.
+constexpr ChunkRoute chunk_route(bool f32, int es, int bm, int bn, int64_t m, int64_t n, int64_t k, int64_t sam,
+                                 int64_t sak, int64_t sbk, int64_t sbn) {
+  const int64_t limit = ((int64_t(1) << 32) / (bm > bn ? bm : bn) / 2 - 1) / es;  // largest pitch
+  const bool k_fits = k >= 8 && k * es < (int64_t(1) << 31);
+  const bool deep = !f32 || k >= 8;  // shorter fp32 sums are closer with the fp32 instruction
+  ChunkRoute r{};
+  r.a_rows = sak == 1 && k_fits && sam >= 0 && sam <= limit;
+  r.a_cols = deep && bm >= 32 && sam == 1 && m >= 8 && sak >= 0 && sak <= limit;
+  r.b_rows = sbk == 1 && k_fits && sbn >= 0 && sbn <= limit;
+  r.b_cols = deep && sbn == 1 && n >= 8 && sbk >= 0 && sbk <= limit;
+  return r;
+}
+
+}  // namespace moegemm
