@@ -88,7 +88,8 @@ int moegemm_kernel_info(int dtype, int index, int32_t* out7);
  * extent, 16-byte alignment, an extent multiple of 8 (K for an operand whose rows run along K, M or
  * N for one whose rows run along it), 256 rows of a K-contiguous operand and all K + 1024 rows of
  * the other kind under 2 GiB; tiles compiled for that layout (moegemm_kernel_layouts) then run the
- * LDS-DMA kernel, others the general one.
+ * LDS-DMA kernel, others the general one.  Homogeneous launches of every kind (split-K and stream-K
+ * too) have no strides table and refuse these values.
  * Otherwise (or for fp32) the general kernel runs, which accepts any strides and alignment.
  */
 int moegemm_grouped_gemm(const int64_t* a_ptrs, const int64_t* b_ptrs, const int64_t* c_ptrs,

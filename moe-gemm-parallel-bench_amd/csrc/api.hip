@@ -291,6 +291,10 @@ int promised_layout(int32_t vector_layout) {
   }
 }
 
+int fail_transposed_homogeneous() {
+  return fail(MOEGEMM_ERR_INVALID, "homogeneous groups are row-major: transposed operands need the strides table");
+}
+
 }  // namespace
 
 extern "C" {
@@ -344,8 +348,7 @@ int grouped_impl(const int64_t* a_ptrs, const int64_t* b_ptrs, const int64_t* c_
   int rc = check_common(dtype, input_precision, group_size_m, &e, block_m, block_n, block_k, num_warps, num_stages);
   if (rc != MOEGEMM_OK) return rc;
   const int layout = promised_layout(vector_layout);
-  if (layout > 0 && homogeneous)
-    return fail(MOEGEMM_ERR_INVALID, "homogeneous groups are row-major: transposed operands need the strides table");
+  if (layout > 0 && homogeneous) return fail_transposed_homogeneous();
   if (swiglu) {
     if (dtype != DT_BF16 && dtype != DT_F16)
       return fail(MOEGEMM_ERR_INVALID, "the SwiGLU epilogue needs fp16 or bf16 operands");
@@ -557,6 +560,7 @@ static int grouped_splitk_impl(const int64_t* a_ptrs, const int64_t* b_ptrs, con
   if (!a_ptrs || !b_ptrs || !c_ptrs) return fail(MOEGEMM_ERR_INVALID, "pointer tables must be non-null");
   if (m <= 0 || n <= 0 || k <= 0)
     return fail(MOEGEMM_ERR_INVALID, "homogeneous shape must be positive (m=%d n=%d k=%d)", m, n, k);
+  if (promised_layout(vector_layout) > 0) return fail_transposed_homogeneous();
   const int layout = vector_layout && e->launch_fast ? 0 : kGeneral;
   if (layout == kGeneral && !any_layout)
     return fail(MOEGEMM_ERR_INVALID, "split-K needs fp16/bf16 operands in the vector layout");
@@ -665,6 +669,7 @@ int moegemm_grouped_gemm_streamk(const int64_t* a_ptrs, const int64_t* b_ptrs, c
   if (!a_ptrs || !b_ptrs || !c_ptrs) return fail(MOEGEMM_ERR_INVALID, "pointer tables must be non-null");
   if (m <= 0 || n <= 0 || k <= 0)
     return fail(MOEGEMM_ERR_INVALID, "homogeneous shape must be positive (m=%d n=%d k=%d)", m, n, k);
+  if (promised_layout(vector_layout) > 0) return fail_transposed_homogeneous();
   if (!vector_layout || !e->launch_fast)
     return fail(MOEGEMM_ERR_INVALID, "stream-K needs fp16/bf16 operands in the vector layout");
   const int64_t tiles = (int64_t)problem_count * cdiv(m, block_m) * cdiv(n, block_n);

@@ -353,7 +353,8 @@ def _problem_layout(a, b, c) -> int:
 
 def _group_layout(workspace: GroupedWorkspace, dtype_code: int) -> int:
     """The one LDS-DMA layout every problem meets (0 row-major, 1 to 3 transposed), or GENERAL;
-    cached per set of tensor objects."""
+    cached per set of tensor objects.  Homogeneous groups launch without a strides table, as row-major
+    ones: with K = 1 a transposed view counts as contiguous too, and stays GENERAL there."""
     if dtype_code == _native.DTYPE_F32:
         return _native.GENERAL
     key = (tuple(map(id, workspace.a)), tuple(map(id, workspace.b)), tuple(map(id, workspace.c)))
@@ -361,7 +362,8 @@ def _group_layout(workspace: GroupedWorkspace, dtype_code: int) -> int:
     if cached is not None and cached[0] == key:
         return cached[1]
     value = _problem_layout(workspace.a[0], workspace.b[0], workspace.c[0])
-    if value != _native.GENERAL and any(_problem_layout(a, b, c) != value for a, b, c in workspace.problem_tensors()):
+    if (value > 0 and workspace.homogeneous) or (value != _native.GENERAL and any(
+            _problem_layout(a, b, c) != value for a, b, c in workspace.problem_tensors())):
         value = _native.GENERAL
     workspace._layout_cache = (key, value)
     return value

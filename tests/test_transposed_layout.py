@@ -134,6 +134,56 @@ def test_transposed_groups(layout, schedule):
             assert torch.equal(z, (x.double() @ y.double()).to(z.dtype))
 
 
+def _column_view_group(count, m, n, device):
+    """K = 1 and A the transposed view of a [1, M] tensor: contiguous to torch, M-contiguous by its strides."""
+    a = [torch.arange(m, device=device).sub(3 + i).to(torch.bfloat16).view(1, m).t() for i in range(count)]
+    b = [torch.arange(n, device=device).remainder(5 + i).to(torch.bfloat16).view(1, n) for i in range(count)]
+    return a, b, [torch.full((m, n), float("nan"), device=device, dtype=torch.bfloat16) for _ in range(count)]
+
+
+def test_homogeneous_groups_are_never_transposed():
+    from kernels.grouped_gemm import _group_layout, workspace_from_tensors
+
+    a, b, c = _column_view_group(2, 64, 128, "cpu")
+    assert a[0].stride() == (1, 64) and _native.transposed_layout(a[0], b[0], c[0]) == 1
+    ws = workspace_from_tensors(a, b, c)
+    assert ws.homogeneous and _group_layout(ws, _native.DTYPE_BF16) == _native.GENERAL
+    unequal = workspace_from_tensors([a[0], a[1][:56]], b, [c[0], c[1][:56]])
+    assert not unequal.homogeneous and _group_layout(unequal, _native.DTYPE_BF16) == 1
+
+
+@pytest.mark.parametrize("flag", [0x10001, 0x20001, 0x30001])
+def test_homogeneous_launches_refuse_a_transposed_promise(flag):
+    """Checked before the workspace, so nothing is launched."""
+    lib, tables, tile = _native.library(), (64, 64, 64), (128, 128, 64, 8, 4, 4)
+    for status in (
+            lib.moegemm_grouped_gemm(*tables, None, None, 2, 64, 128, 256, 1, 0, _native.DTYPE_BF16, 0, *tile, 0, flag,
+                                     0, None),
+            lib.moegemm_grouped_gemm_splitk(*tables, 2, 64, 128, 256, _native.DTYPE_BF16, *tile, 2, 0, flag, None, 0,
+                                            0, None),
+            lib.moegemm_grouped_gemm_splitk_any(*tables, 2, 64, 128, 256, _native.DTYPE_BF16, 0, *tile, 2, 0, flag,
+                                                None, 0, 0, None),
+            lib.moegemm_grouped_gemm_streamk(*tables, 2, 64, 128, 256, _native.DTYPE_BF16, *tile, 1, 1, flag, None, 0,
+                                             0, None)):
+        assert status == _native.ERR_INVALID and "homogeneous groups are row-major" in _native.last_error()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("autotune", [False, True])
+def test_column_view_groups_launch(autotune):
+    if not torch.cuda.is_available():
+        pytest.skip("ROCm GPU unavailable")
+    from kernels.grouped_gemm import launch_grouped, workspace_from_tensors
+
+    a, b, c = _column_view_group(2, 64, 128, "cuda")
+    ws = workspace_from_tensors(a, b, c)
+    print(f"column view group autotune={autotune}", flush=True)
+    launch_grouped(ws, autotune=autotune)
+    torch.cuda.synchronize()
+    for x, y, z in zip(a, b, c):
+        assert torch.equal(z, (x.double() @ y.double()).to(z.dtype))
+
+
 def test_untuned_ragged_configs_are_compiled():
     from kernels.matmul import _menu, select_ragged_config
 
