@@ -9,6 +9,7 @@ required" error (reference kernels/grouped_gemm.py:626-627, kernels/matmul.py:34
 from __future__ import annotations
 
 import ctypes
+import threading
 import os
 from functools import lru_cache
 from pathlib import Path
@@ -309,17 +310,75 @@ def _refuse_allocation_under_capture(what: str) -> None:
 
 _SPLITK_MAX_SPLITS, _SPLITK_MAX_TILES = 64, 65536  # the split-K launches' limits (moegemm.h)
 
+# Split-K scratch of operands outside the row-major 16-bit layout (fp32, unaligned, transposed).  They must
+# run wherever a launch without scratch would, so theirs is kept apart from the workspaces above: only eager
+# launches use it, in the order of the one stream it belongs to, and no captured graph holds its address
+# (two graphs captured on one stream, or a graph beside eager calls on its capture stream, may replay at
+# once).  Each buffer is made on its own stream and used on no other, so dropping one is safe at any
+# time: its memory is reused in that stream's order.  At most 16 streams hold one, as large as the last
+# growth asked for.
+_EAGER_SCRATCH: dict[tuple[int, int], object] = {}
+_EAGER_SCRATCH_STREAMS = 16
+_EAGER_SCRATCH_LOCK = threading.Lock()
 
-def splitk_serves(device, stream_handle: int, tiles: int, splits: int, block_m: int, block_n: int) -> bool:
-    """Whether a split launch can be made: within the library's limits, and its workspace is held
-    already or can be made (not under graph capture)."""
+
+def capturing() -> bool:
+    """Whether the current stream records a graph."""
     import torch
 
-    if splits > _SPLITK_MAX_SPLITS or tiles > _SPLITK_MAX_TILES:
-        return False
-    held = _SPLITK_WORKSPACES.get((torch.device(device).index or 0, int(stream_handle)))
+    return torch.cuda.is_current_stream_capturing()
+
+
+def eager_scratch(device, stream_handle: int, tiles: int, splits: int, block_m: int, block_n: int):
+    """Zero-initialised split-K scratch for one launch on the current stream of ``device``; None when the
+    launch has to run whole: past the library's limits, under graph capture, or out of memory."""
+    import torch
+
+    if splits > _SPLITK_MAX_SPLITS or tiles > _SPLITK_MAX_TILES or capturing():
+        return None
     nbytes = splitk_workspace_bytes(tiles, splits, block_m, block_n)
-    return bool(held and held[-1].numel() >= nbytes) or not torch.cuda.is_current_stream_capturing()
+    key = (torch.device(device).index or 0, int(stream_handle))
+    held = _EAGER_SCRATCH.get(key)
+    if held is not None and held.numel() >= nbytes:
+        return held
+    try:
+        buffer = torch.zeros(nbytes, dtype=torch.uint8, device=device)
+    except torch.cuda.OutOfMemoryError:
+        return None
+    with _EAGER_SCRATCH_LOCK:
+        _EAGER_SCRATCH.pop(key, None)
+        while len(_EAGER_SCRATCH) >= _EAGER_SCRATCH_STREAMS:
+            _EAGER_SCRATCH.pop(next(iter(_EAGER_SCRATCH)))
+        _EAGER_SCRATCH[key] = buffer
+    return buffer
+
+
+class TuningScratch:
+    """What a tuner's timings use in place of ``eager_scratch``: one buffer for all candidates, which run one
+    after the other, given back when the tuner is done.  The tuner's own captured graphs may use it: each is
+    replayed and dropped before the next candidate runs."""
+
+    def __init__(self):
+        import torch
+
+        self._home = torch.cuda.current_stream()
+        self._buffer = None
+
+    def __call__(self, device, stream_handle: int, tiles: int, splits: int, block_m: int, block_n: int):
+        import torch
+
+        if splits > _SPLITK_MAX_SPLITS or tiles > _SPLITK_MAX_TILES:
+            return None
+        nbytes = splitk_workspace_bytes(tiles, splits, block_m, block_n)
+        if self._buffer is None or self._buffer.numel() < nbytes:
+            if capturing():
+                return None
+            torch.cuda.synchronize(device)  # whatever a failed candidate left on another stream
+            self._buffer = None
+            with torch.cuda.stream(self._home):  # one stream's memory, whichever stream times
+                self._buffer = torch.zeros(nbytes, dtype=torch.uint8, device=device)
+            torch.cuda.current_stream(device).wait_stream(self._home)
+        return self._buffer
 
 
 def splitk_workspace(device, stream_handle: int, nbytes: int):

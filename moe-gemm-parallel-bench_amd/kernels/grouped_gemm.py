@@ -383,20 +383,12 @@ def _check_workspace(workspace: GroupedWorkspace) -> int:
     return _native.dtype_code(a0.dtype)
 
 
-def _grouped_splits(workspace: GroupedWorkspace, cfg: KernelConfig, dtype_code: int, split_k, layout=None) -> int:
-    if layout is None:
-        layout = _group_layout(workspace, dtype_code)
+def _grouped_splits(workspace: GroupedWorkspace, cfg: KernelConfig, dtype_code: int, split_k, layout: int) -> int:
     if not workspace.homogeneous or (layout != 0 and cfg.tile_key not in _native.split_tiles(dtype_code, layout)):
         return 1
-    tiles = workspace.tile_count_for(cfg)
-    splits = split_k if split_k is not None else splitk_count(tiles, workspace.max_k, cfg.block_k, workspace.sm_count)
-    # General tiles take the unsplit launch where a split one cannot be made (graph capture before the
-    # workspace exists, or a named split_k past the library's limits).
-    if splits > 1 and layout != 0 and not _native.splitk_serves(
-            workspace.a[0].device, _native.current_stream_handle(workspace.a[0].device), tiles, splits,
-            cfg.block_m, cfg.block_n):
-        splits = 1
-    return splits
+    if split_k is not None:
+        return split_k
+    return splitk_count(workspace.tile_count_for(cfg), workspace.max_k, cfg.block_k, workspace.sm_count)
 
 
 def with_schedule_options(options, tile_schedule: str | None, streamk_ok=None) -> list:
@@ -427,23 +419,25 @@ def streamk_tail_for(workspace: GroupedWorkspace, cfg: KernelConfig, dtype_code:
 
 
 def _launch_grouped_fixed(workspace: GroupedWorkspace, cfg: KernelConfig, dtype_code: int, precision: int,
-                          split_k=None, schedule: str = "static", b_stream: int = 0, layout=None) -> int:
+                          split_k=None, schedule: str = "static", b_stream: int = 0, layout=None,
+                          scratch=_native.eager_scratch) -> int:
     """One launch; returns the K splits used.  ``schedule`` "stealing" draws the tiles from the
     work-stealing queues (unsplit launches only); ``b_stream`` 1 issues the LDS-DMA kernels' B copies
-    non-temporal."""
+    non-temporal; ``scratch`` gives the split-K scratch of groups that are not row-major 16-bit ones, or
+    None to run whole."""
     if schedule == "streamk":
         tail = streamk_tail_for(workspace, cfg, dtype_code)
         if tail:
             m, k, n = workspace.shapes[0]
             grid = workspace.sm_count
             stream = _native.current_stream_handle(workspace.a[0].device)
-            scratch = _native.splitk_workspace(workspace.a[0].device, stream,
-                                               _native.streamk_workspace_bytes(tail, grid, cfg.block_m, cfg.block_n))
+            room = _native.splitk_workspace(workspace.a[0].device, stream,
+                                            _native.streamk_workspace_bytes(tail, grid, cfg.block_m, cfg.block_n))
             status = _native.library().moegemm_grouped_gemm_streamk(
                 workspace.a_ptrs.data_ptr(), workspace.b_ptrs.data_ptr(), workspace.c_ptrs.data_ptr(),
                 workspace.problem_count, m, n, k, dtype_code,
                 cfg.block_m, cfg.block_n, cfg.block_k, cfg.group_size_m, cfg.num_warps, cfg.num_stages, tail, grid,
-                1, scratch.data_ptr(), scratch.numel(), b_stream, stream,
+                1, room.data_ptr(), room.numel(), b_stream, stream,
             )
             _native.check(status)
             return 1
@@ -453,34 +447,37 @@ def _launch_grouped_fixed(workspace: GroupedWorkspace, cfg: KernelConfig, dtype_
     splits = _grouped_splits(workspace, cfg, dtype_code, split_k, layout)
     if schedule == "stealing" and splits > 1:
         raise ValueError("the work-stealing schedule runs unsplit launches only (split_k must be 1)")
-    if splits > 1:
+    device = workspace.a[0].device
+    stream = _native.current_stream_handle(device)
+    tiles, room = workspace.tile_count_for(cfg), None
+    if splits > 1 and layout == 0:
+        room = _native.splitk_workspace(device, stream,
+                                        _native.splitk_workspace_bytes(tiles, splits, cfg.block_m, cfg.block_n))
+    elif splits > 1:
+        room = scratch(device, stream, tiles, splits, cfg.block_m, cfg.block_n)
+    if room is not None:
         m, k, n = workspace.shapes[0]
-        tiles = workspace.tile_count_for(cfg)
-        stream = _native.current_stream_handle(workspace.a[0].device)
-        scratch = _native.splitk_workspace(workspace.a[0].device, stream,
-                                           _native.splitk_workspace_bytes(tiles, splits, cfg.block_m, cfg.block_n))
         status = _native.library().moegemm_grouped_gemm_splitk_any(
             workspace.a_ptrs.data_ptr(), workspace.b_ptrs.data_ptr(), workspace.c_ptrs.data_ptr(),
             workspace.problem_count, m, n, k, dtype_code, precision,
             cfg.block_m, cfg.block_n, cfg.block_k, cfg.group_size_m, cfg.num_warps, cfg.num_stages, splits,
             max(1, min(tiles * splits, workspace.sm_count * cfg.cta_multiplier)), _native.LAYOUT_FLAGS[layout],
-            scratch.data_ptr(), scratch.numel(), b_stream, stream,
+            room.data_ptr(), room.numel(), b_stream, stream,
         )
         _native.check(status)
         return splits
     lib = _native.library()
     m, k, n = workspace.shapes[0]
-    stream = _native.current_stream_handle(workspace.a[0].device)
     args = (
         workspace.a_ptrs.data_ptr(), workspace.b_ptrs.data_ptr(), workspace.c_ptrs.data_ptr(),
         workspace.dims.data_ptr(), workspace.strides.data_ptr(),
         workspace.problem_count, m, n, k, 1 if workspace.homogeneous else 0,
-        workspace.tile_count_for(cfg), dtype_code, precision,
+        tiles, dtype_code, precision,
         cfg.block_m, cfg.block_n, cfg.block_k, cfg.group_size_m, cfg.num_warps, cfg.num_stages,
         _grid_size(workspace, cfg), _native.LAYOUT_FLAGS[layout],
     )
     if schedule == "stealing":
-        queue = _native.tile_queue(workspace.a[0].device, stream)
+        queue = _native.tile_queue(device, stream)
         status = lib.moegemm_grouped_gemm_stealing(*args, queue.data_ptr(), b_stream, stream)
     elif schedule == "static":
         status = lib.moegemm_grouped_gemm(*args, b_stream, stream)
@@ -491,6 +488,7 @@ def _launch_grouped_fixed(workspace: GroupedWorkspace, cfg: KernelConfig, dtype_
 
 
 _GROUPED_AUTOTUNE_CACHE: dict[tuple, tuple] = {}
+_GROUPED_WHOLE_OPTIONS: dict[tuple, tuple] = {}  # by the same key: the fastest static option that does not split K
 
 
 def _grouped_tuning_key(workspace: GroupedWorkspace, scheduler: str, dtype_code: int, precision: int, split_k,
@@ -513,8 +511,9 @@ def launch_grouped(
     """Launch the persistent grouped kernel (autotuned per workload key, or a fixed config).
 
     ``split_k`` (keyword-only, not in the reference's signature) as for ``launch_matmul``: None
-    splits K inside the one launch when a homogeneous 16-bit group has too few tiles to fill the
-    CUs; 1 disables it; n forces n.  ``workspace.split_k`` records what ran.
+    splits K inside the one launch when a homogeneous group has too few tiles to fill the CUs; 1
+    disables it; n forces n (operands that are not row-major 16-bit ones run whole where a split launch
+    cannot be made, as there).  ``workspace.split_k`` records what ran.
     ``tile_schedule`` (keyword-only, not in the reference's signature): "static" (tiles pid,
     pid + grid, ... as the reference's programs take them), "stealing" (per-XCD tile queues
     with stealing) or "streamk" (whole tiles in exact rounds of one workgroup per CU, then the
@@ -573,9 +572,13 @@ def launch_grouped(
             # The B copy policy is timed on the finalists where it is not pinned and the LDS-DMA kernels run.
             twin = ((lambda o: (o[0], o[1], o[2], 1))
                     if b_stream is None and layout >= 0 else None)
-            tuned = _tune(options, lambda o: _launch_grouped_fixed(workspace, o[0], dtype_code, precision, *o[1:]),
-                          twin=twin)
+            scratch = _native.TuningScratch()
+            tuned, _GROUPED_WHOLE_OPTIONS[key] = _tune(
+                options, lambda o: _launch_grouped_fixed(workspace, o[0], dtype_code, precision, *o[1:], layout, scratch),
+                twin=twin, fallback=lambda o: o[1] == 1 and o[2] == "static")
             _GROUPED_AUTOTUNE_CACHE[key] = tuned
+        if layout != 0 and tuned[1] != 1 and _native.capturing():
+            tuned = _GROUPED_WHOLE_OPTIONS.get(key) or tuned  # a captured launch has no scratch
         cfg, split_k, schedule, stream_b = tuned
     else:
         schedule = tile_schedule or "static"

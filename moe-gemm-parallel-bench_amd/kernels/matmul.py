@@ -306,6 +306,7 @@ def matmul_candidate_configs(m: int, n: int, k: int, limit: int = 10, *, dtype=N
 # Launch
 
 _AUTOTUNE_CACHE: dict[tuple, KernelConfig] = {}
+_WHOLE_OPTIONS: dict[tuple, tuple] = {}  # by the same key: the fastest option that does not split K, if any
 _LAST_AUTOTUNED: list[KernelConfig | None] = [None]
 
 
@@ -452,12 +453,8 @@ def _launch_fixed_streamk(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, 
     _native.check(status)
 
 
-def _launch_fixed_splitk(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, splits: int, b_stream: int = 0,
-                         precision: int = _native.PRECISION_IEEE) -> None:
-    tiles = -(-m // cfg.block_m) * -(-n // cfg.block_n)
-    nbytes = _native.splitk_workspace_bytes(tiles, splits, cfg.block_m, cfg.block_n)
-    stream = _native.current_stream_handle(a.device)
-    workspace = _native.splitk_workspace(a.device, stream, nbytes)
+def _launch_fixed_splitk(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, splits: int, workspace, stream: int,
+                         b_stream: int = 0, precision: int = _native.PRECISION_IEEE) -> None:
     status = _native.library().moegemm_matmul_splitk_any(
         a.data_ptr(), b.data_ptr(), c.data_ptr(), m, n, k,
         a.stride(0), a.stride(1), b.stride(0), b.stride(1), c.stride(0), c.stride(1), dtype_code, precision,
@@ -468,10 +465,11 @@ def _launch_fixed_splitk(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, s
 
 
 def _launch_fixed(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, precision: int, split_k=None,
-                  b_stream: int = 0) -> int:
+                  b_stream: int = 0, scratch=_native.eager_scratch) -> int:
     """One launch; returns the K splits used (``split_k`` None = ``splitk_count``'s choice,
     ``STREAMK`` = a stream-K tail where one applies, else the unsplit launch).  ``b_stream`` 1 issues
-    the LDS-DMA kernels' B copies non-temporal."""
+    the LDS-DMA kernels' B copies non-temporal.  ``scratch`` gives the split-K scratch of operands that
+    are not row-major 16-bit ones, or None to run whole."""
     _LAST_SCHEDULE[0] = "static"
     _LAST_B_STREAM[0] = b_stream
     if split_k == STREAMK:
@@ -481,20 +479,21 @@ def _launch_fixed(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, precisio
             _LAST_SCHEDULE[0] = STREAMK
             return 1
         split_k = 1
-    splits = 1
     layout = _operand_layout(a, b, c)
     if layout == 0 or cfg.tile_key in _native.split_tiles(dtype_code, layout):
         tiles = -(-m // cfg.block_m) * -(-n // cfg.block_n)
         splits = split_k if split_k is not None else splitk_count(tiles, k, cfg.block_k,
                                                                   _device_signature(a.device) % 1000)
-        # Other operands than row-major ones take the unsplit launch where a split one cannot be made
-        # (graph capture before the workspace exists, or a named split_k past the library's limits).
-        if splits > 1 and layout != 0 and not _native.splitk_serves(
-                a.device, _native.current_stream_handle(a.device), tiles, splits, cfg.block_m, cfg.block_n):
-            splits = 1
-    if splits > 1:
-        _launch_fixed_splitk(a, b, c, m, n, k, cfg, dtype_code, splits, b_stream, precision)
-        return splits
+        if splits > 1:
+            stream = _native.current_stream_handle(a.device)
+            if layout == 0:
+                nbytes = _native.splitk_workspace_bytes(tiles, splits, cfg.block_m, cfg.block_n)
+                workspace = _native.splitk_workspace(a.device, stream, nbytes)
+            else:
+                workspace = scratch(a.device, stream, tiles, splits, cfg.block_m, cfg.block_n)
+            if workspace is not None:
+                _launch_fixed_splitk(a, b, c, m, n, k, cfg, dtype_code, splits, workspace, stream, b_stream, precision)
+                return splits
     lib = _native.library()
     status = lib.moegemm_matmul(
         a.data_ptr(), b.data_ptr(), c.data_ptr(), m, n, k,
@@ -521,8 +520,12 @@ def launch_matmul(
     """Launch C = A @ B: autotuned per shape key, or with an explicit config when autotune is false.
 
     ``split_k`` (keyword-only, not in the reference's signature): None lets ``splitk_count`` split
-    K when the output tiles leave most CUs idle (fp16/bf16 vector layouts, one launch with a
-    deterministic in-kernel reduction); 1 disables it; n > 1 forces n splits.
+    K when the output tiles leave most CUs idle (one launch with a deterministic in-kernel
+    reduction); 1 disables it; n > 1 forces n splits.  Row-major 16-bit operands keep a workspace per
+    stream, which the first split call makes outside graph capture.  All others (fp32, unaligned,
+    transposed) run whole where a split launch cannot be made: under graph capture (with the best
+    unsplit tile the tuner saw), past 64 splits or 65536 tiles, on tiles without a split kernel and out
+    of memory; ``last_matmul_split()`` tells what ran.
     ``b_stream`` (keyword-only, not in the reference's signature): 1 issues the LDS-DMA kernels' B
     copies non-temporal, 0 as ordinary loads; None lets the tuner measure both (0 without
     autotuning).  ``last_matmul_b_stream()`` reports what ran.
@@ -543,10 +546,10 @@ def launch_matmul(
         m, n, k, tuple(a.stride()), tuple(b.stride()), tuple(c.stride()), dtype_code, precision,
         _device_signature(a.device), split_k, b_stream,
     )
+    layout = _operand_layout(a, b, c)
     best = _AUTOTUNE_CACHE.get(key)
     if best is None:
         sm_count = _device_signature(a.device) % 1000
-        layout = _operand_layout(a, b, c)
         tiles = _native.layout_tiles(dtype_code, layout) if layout > 0 else None
         configs = matmul_candidate_configs(m, n, k, dtype=a.dtype, sm_count=sm_count, tiles=tiles)
         general = _native.split_tiles(dtype_code, layout) if layout == _native.GENERAL else None
@@ -561,9 +564,13 @@ def launch_matmul(
         options = [(cfg, split, b_stream or 0) for cfg, split in options]
         # The B copy policy is timed on the finalists where it is not pinned and the LDS-DMA kernels run.
         twin = (lambda o: (o[0], o[1], 1)) if b_stream is None and layout >= 0 else None
-        best = _tune(options, lambda o: _launch_fixed(a, b, c, m, n, k, o[0], dtype_code, precision, o[1], o[2]),
-                     twin=twin)
+        scratch = _native.TuningScratch()
+        best, _WHOLE_OPTIONS[key] = _tune(
+            options, lambda o: _launch_fixed(a, b, c, m, n, k, o[0], dtype_code, precision, *o[1:], scratch), twin=twin,
+            fallback=lambda o: o[1] == 1)
         _AUTOTUNE_CACHE[key] = best
+    if layout != 0 and best[1] != 1 and _native.capturing():
+        best = _WHOLE_OPTIONS.get(key) or best  # a captured launch has no scratch
     _LAST_AUTOTUNED[0] = best[0]
     _LAST_SPLIT[0] = _launch_fixed(a, b, c, m, n, k, best[0], dtype_code, precision, best[1], best[2])
 
@@ -591,7 +598,7 @@ _FINALISTS = 5
 _FINAL_ROUNDS = 7
 
 
-def _tune(candidates, launch, prefer=None, prefer_margin: float = 0.03, twin=None):
+def _tune(candidates, launch, prefer=None, prefer_margin: float = 0.03, twin=None, fallback=None):
     """Hot-time every candidate (graph replays, bounded) after a clock warm-up, twice (a forward and a
     reverse sweep), then re-time the best five interleaved (seven rounds of A, B, C, D, E) and keep
     the lowest median, so a clock drift during tuning shifts every finalist alike instead of
@@ -602,7 +609,10 @@ def _tune(candidates, launch, prefer=None, prefer_margin: float = 0.03, twin=Non
     finalist is faster by more than ``prefer_margin``: a choice already measured on the same
     workload is not overturned by timing noise.  ``twin(option)`` (or None) names a variant of a
     finalist that only the interleaved rounds time, next to it: the non-temporal B copies, whose
-    effect depends on the workload but hardly on which of the leading tiles runs."""
+    effect depends on the workload but hardly on which of the leading tiles runs.
+
+    With ``fallback`` (a predicate of an option) the result is a pair: the choice, and the fastest measured
+    candidate that meets the predicate (the choice itself if it does; None if none does)."""
     candidates = list(candidates)
     first: dict[int, float] = {}
     failed: set[int] = set()
@@ -641,5 +651,7 @@ def _tune(candidates, launch, prefer=None, prefer_margin: float = 0.03, twin=Non
     medians = [sorted(times)[_FINAL_ROUNDS // 2] for times in rounds]
     best = finalists[medians.index(min(medians))]
     if prefer in finalists and medians[finalists.index(prefer)] <= min(medians) * (1.0 + prefer_margin):
-        return prefer
-    return best
+        best = prefer
+    if fallback is None:
+        return best
+    return best, best if fallback(best) else next((cfg for _, cfg in measured if fallback(cfg)), None)
