@@ -562,13 +562,13 @@ struct GeneralTile {
     bool done = false;
     if constexpr (EPI == EPI_SPLIT) {
       // Operands Plain must stage: unit 0 of each tile computes it whole.
-      if (!r.chunked() && pd.split != 0) return;
+      if (!((r.a_rows || (BM >= 32 && r.a_cols)) && (r.b_rows || r.b_cols)) && pd.split != 0) return;
     }
     if (r.a_rows && r.b_cols) {
       done = chunk_tile<false, false, EPI>(pd, tm, tn, smem, before_store);
     } else if (r.a_rows && r.b_rows) {
       done = chunk_tile<false, true, EPI>(pd, tm, tn, smem, before_store);
-    } else if (r.chunked()) {
+    } else if (r.a_cols && (r.b_cols || r.b_rows)) {
       if constexpr (BM >= 32) {
         if (r.b_cols)
           done = chunk_tile<true, false, EPI>(pd, tm, tn, smem, before_store);

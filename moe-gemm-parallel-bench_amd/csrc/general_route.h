@@ -18,14 +18,14 @@ struct ChunkRoute {
 // meet the rule is staged element by element with signed 64-bit indices.
 constexpr ChunkRoute chunk_route(bool f32, int es, int bm, int bn, int64_t m, int64_t n, int64_t k, int64_t sam,
                                  int64_t sak, int64_t sbk, int64_t sbn) {
-  const int64_t limit = ((int64_t(1) << 32) / (bm > bn ? bm : bn) / 2 - 1) / es;  // largest pitch
+  const uint64_t limit = ((uint64_t(1) << 32) / (bm > bn ? bm : bn) / 2 - 1) / es + 1;  // a pitch is below it
   const bool k_fits = k >= 8 && k * es < (int64_t(1) << 31);
   const bool deep = !f32 || k >= 8;  // shorter fp32 sums are closer with the fp32 instruction
   ChunkRoute r{};
-  r.a_rows = sak == 1 && k_fits && sam >= 0 && sam <= limit;
-  r.a_cols = deep && bm >= 32 && sam == 1 && m >= 8 && sak >= 0 && sak <= limit;
-  r.b_rows = sbk == 1 && k_fits && sbn >= 0 && sbn <= limit;
-  r.b_cols = deep && sbn == 1 && n >= 8 && sbk >= 0 && sbk <= limit;
+  r.a_rows = sak == 1 && k_fits && uint64_t(sam) < limit;  // unsigned: negative pitches are past any limit
+  r.a_cols = deep && bm >= 32 && sam == 1 && m >= 8 && uint64_t(sak) < limit;
+  r.b_rows = sbk == 1 && k_fits && uint64_t(sbn) < limit;
+  r.b_cols = deep && sbn == 1 && n >= 8 && uint64_t(sbk) < limit;
   return r;
 }
 
