@@ -46,6 +46,7 @@ extern "C" {
 #define MOEGEMM_LAYOUT_AT 0x10001   /* A stored [K, M] (unit row stride), B row-major */
 #define MOEGEMM_LAYOUT_BT 0x20001   /* A row-major, B stored [N, K] (unit row stride) */
 #define MOEGEMM_LAYOUT_ATBT 0x30001 /* both transposed */
+#define MOEGEMM_LAYOUT_STRIDED 0x40000 /* neither: as 0, and faster where no problem's A or none's B has a unit stride */
 
 /* Size of the tile queue of the work-stealing launches (17 int32 counters, each in a 256-byte
  * block of its own; the buffer is 256-byte aligned). */

@@ -72,14 +72,15 @@ int check_common(int dtype, int input_precision, int group_size_m, const KernelE
   return MOEGEMM_OK;
 }
 
-// `layout`: the operands' OperandLayout when they meet the LDS-DMA preconditions, else kGeneral.
-constexpr int kGeneral = -1;
+// `layout`: the operands' OperandLayout when they meet the LDS-DMA preconditions, else kGeneral, or kPlain
+// when the general tile could stage no chunk of them either.
+constexpr int kGeneral = -1, kPlain = -2;
 
 int launch(const KernelEntry* e, KParams& p, int grid, int layout, int32_t b_stream, void* stream) {
   if (b_stream != 0 && b_stream != 1) return fail(MOEGEMM_ERR_INVALID, "b_stream must be 0 or 1 (got %d)", b_stream);
   p.b_stream = b_stream;
   LaunchFn fast = layout == 0 ? e->launch_fast : layout > 0 ? e->launch_transposed[layout - 1] : nullptr;
-  LaunchFn fn = fast ? fast : e->launch_general;
+  LaunchFn fn = fast ? fast : layout == kPlain ? e->launch_plain : e->launch_general;
   if (p.sk_tiles > 0) {  // stream-K tail: the fast path's stream-K kernel (the callers checked the layout)
     if (layout != 0 || !e->launch_fast_streamk)
       return fail(MOEGEMM_ERR_INVALID, "stream-K needs fp16/bf16 operands in the vector layout");
@@ -280,9 +281,18 @@ int fast_layout(const void* a, const void* b, const void* c, int64_t m, int64_t 
   return layout == 0 ? kGeneral : layout;  // layout 0 is vector_layout_ok's rule alone
 }
 
+// `layout`, or kPlain for general operands of these strides that this tile cannot stage in chunks.
+int plain_or(int layout, const KernelEntry* e, int64_t m, int64_t n, int64_t k, int64_t sam, int64_t sak, int64_t sbk,
+             int64_t sbn) {
+  const bool f32 = e->dtype == DT_F32;
+  const bool chunked = chunk_route(f32, f32 ? 4 : 2, e->block_m, e->block_n, m, n, k, sam, sak, sbk, sbn).chunked();
+  return layout == kGeneral && !chunked ? kPlain : layout;
+}
+
 // The layout a caller of the grouped launches promises (see MOEGEMM_LAYOUT_* in moegemm.h).
 int promised_layout(int32_t vector_layout) {
   switch (vector_layout) {
+    case MOEGEMM_LAYOUT_STRIDED: return kPlain;
     case 0: return kGeneral;
     case MOEGEMM_LAYOUT_AT: return kAT;
     case MOEGEMM_LAYOUT_BT: return kBT;
@@ -481,6 +491,8 @@ static int matmul_splitk_impl(const void* a, const void* b, void* c, int32_t m, 
   p.tf32 = input_precision == MOEGEMM_PRECISION_TF32;
   rc = setup_splits(p, tiles, k, splits, block_m, block_n, block_k, workspace, workspace_bytes);
   if (rc != MOEGEMM_OK) return rc;
+  layout = plain_or(layout, e, m, n, k, stride_am, stride_ak, stride_bk, stride_bn);
+  if (layout == kPlain) p.splits = 1;  // GemmTile computes whole tiles
   const int64_t units = (int64_t)p.total_tiles * p.splits;
   const int grid = grid_size <= 0 || grid_size > units ? (int)units : grid_size;
   return launch(e, p, grid, layout, b_stream, stream);
@@ -560,8 +572,9 @@ static int grouped_splitk_impl(const int64_t* a_ptrs, const int64_t* b_ptrs, con
   if (!a_ptrs || !b_ptrs || !c_ptrs) return fail(MOEGEMM_ERR_INVALID, "pointer tables must be non-null");
   if (m <= 0 || n <= 0 || k <= 0)
     return fail(MOEGEMM_ERR_INVALID, "homogeneous shape must be positive (m=%d n=%d k=%d)", m, n, k);
-  if (promised_layout(vector_layout) > 0) return fail_transposed_homogeneous();
-  const int layout = vector_layout && e->launch_fast ? 0 : kGeneral;
+  const int promised = promised_layout(vector_layout);
+  if (promised > 0) return fail_transposed_homogeneous();
+  const int layout = promised == 0 && e->launch_fast ? 0 : kGeneral;
   if (layout == kGeneral && !any_layout)
     return fail(MOEGEMM_ERR_INVALID, "split-K needs fp16/bf16 operands in the vector layout");
   if (layout == kGeneral && !e->launch_general_split)
@@ -669,8 +682,9 @@ int moegemm_grouped_gemm_streamk(const int64_t* a_ptrs, const int64_t* b_ptrs, c
   if (!a_ptrs || !b_ptrs || !c_ptrs) return fail(MOEGEMM_ERR_INVALID, "pointer tables must be non-null");
   if (m <= 0 || n <= 0 || k <= 0)
     return fail(MOEGEMM_ERR_INVALID, "homogeneous shape must be positive (m=%d n=%d k=%d)", m, n, k);
-  if (promised_layout(vector_layout) > 0) return fail_transposed_homogeneous();
-  if (!vector_layout || !e->launch_fast)
+  const int promised = promised_layout(vector_layout);
+  if (promised > 0) return fail_transposed_homogeneous();
+  if (promised != 0 || !e->launch_fast)
     return fail(MOEGEMM_ERR_INVALID, "stream-K needs fp16/bf16 operands in the vector layout");
   const int64_t tiles = (int64_t)problem_count * cdiv(m, block_m) * cdiv(n, block_n);
   if (tiles > INT32_MAX) return fail(MOEGEMM_ERR_INVALID, "tile count %lld exceeds int32", (long long)tiles);
@@ -827,8 +841,9 @@ int moegemm_matmul(const void* a, const void* b, void* c, int32_t m, int32_t n, 
   p.tf32 = input_precision == MOEGEMM_PRECISION_TF32;
   p.total_tiles = (int32_t)tiles;
   int grid = grid_size <= 0 ? p.total_tiles : (grid_size < p.total_tiles ? grid_size : p.total_tiles);
-  return launch(e, p, grid, fast_layout(a, b, c, m, n, k, stride_am, stride_ak, stride_bk, stride_bn, stride_cm,
-                                        stride_cn, dtype), b_stream, stream);
+  const int layout = fast_layout(a, b, c, m, n, k, stride_am, stride_ak, stride_bk, stride_bn, stride_cm, stride_cn,
+                                 dtype);
+  return launch(e, p, grid, plain_or(layout, e, m, n, k, stride_am, stride_ak, stride_bk, stride_bn), b_stream, stream);
 }
 
 }  // extern "C"

@@ -60,7 +60,7 @@ typedef uint32_t u32x2_a2_t __attribute__((ext_vector_type(2), aligned(2)));
 // PARTS: bf16 panels per operand (3 = fp32 operands, 2 = TF32 operands, 1 = 16-bit operands).
 template <class E, int BM_, int BN_, int BK_, int WM_, int WN_, int PARTS_>
 struct GeneralTile {
-  using Plain = GemmTile<E, BM_, BN_, BK_, WM_, WN_>;
+  using Plain = GemmTile<E, BM_, BN_, BK_, WM_, WN_, true>;
   static constexpr int BM = BM_, BN = BN_, BK = BK_, WM = WM_, WN = WN_, PARTS = PARTS_;
   static constexpr bool F32 = E::is_f32;
   static constexpr int ES = sizeof(typename E::raw);

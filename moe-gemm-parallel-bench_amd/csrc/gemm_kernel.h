@@ -271,7 +271,9 @@ __device__ __forceinline__ int swz_b(int row, int chunks) {
 }
 
 // ---------------------------------------------------------------------------------------------
-template <class E, int BM_, int BN_, int BK_, int WM_, int WN_>
+// SHARED: the tile is compiled into the kernel of a larger one (GeneralTile), so its fp32 K steps are
+// unrolled by two only: the eight steps' fragments took more registers than the whole of that loop.
+template <class E, int BM_, int BN_, int BK_, int WM_, int WN_, bool SHARED_ = false>
 struct GemmTile {
   using raw_t = typename E::raw;
   static constexpr int BM = BM_, BN = BN_, BK = BK_, WM = WM_, WN = WN_;
@@ -415,11 +417,10 @@ struct GemmTile {
   __device__ static __forceinline__ void compute_stage(acc_t (&acc)[FM][FN], const char* lds_a, const char* lds_b,
                                                        int wave_m, int wave_n) {
     const int lane = threadIdx.x & 63;
-    if constexpr (F32) {
-      // Unrolled by two only: fully unrolled, the eight steps' fragments took more registers than the
-      // whole of GeneralTile's loop, which shares a kernel with this one.
-#pragma unroll 2
-      for (int kk = 0; kk < BK / MIK; ++kk) {
+    constexpr int kUnroll = F32 && SHARED_ ? 2 : BK / MIK;
+#pragma unroll kUnroll
+    for (int kk = 0; kk < BK / MIK; ++kk) {
+      if constexpr (F32) {
         // v_mfma_f32_16x16x4_f32, swapped: first operand B^T (row n = lane%16, k = lane/16),
         // second operand A^T (col m = lane%16, k = lane/16).
         float af[FM], bf[FN];
@@ -443,12 +444,7 @@ struct GemmTile {
 #pragma unroll
           for (int fn = 0; fn < FN; ++fn)
             acc[fm][fn] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[fn], af[fm], acc[fm][fn], 0, 0, 0);
-      }
-      return;
-    }
-#pragma unroll
-    for (int kk = 0; kk < BK / MIK; ++kk) {
-      if constexpr (!F32) {
+      } else {
         i16x8_t af[FM], bf[FN];
 #pragma unroll
         for (int fm = 0; fm < FM; ++fm) {
@@ -507,7 +503,7 @@ struct GemmTile {
   __device__ static __forceinline__ void store_tile(const acc_t (&acc)[FM][FN], const ProblemDesc& pd, int m0,
                                                     int n0, int wave_m, int wave_n) {
     const int lane = threadIdx.x & 63;
-    // The SwiGLU and split-K epilogues run only in the LDS-DMA tiles (the host enforces it).
+    // The host launches no SwiGLU or split-K epilogue of this tile.
     if (pd.swiglu || pd.splits > 1) return;
     const bool vec_c = pd.scn == 1 && (pd.scm % 4) == 0 && (pd.n % 4) == 0 &&
                        ((reinterpret_cast<uintptr_t>(pd.c) & (4 * ES - 1)) == 0);
@@ -538,11 +534,11 @@ struct GemmTile {
 
   // -------------------------------------------------------------------------------------------
   // `before_store` runs once the K loop is done, before the C stores (the work-stealing scheduler
-  // draws its next ticket there).  Split-K runs only on the LDS-DMA tiles: EPI is always EPI_C here.
+  // draws its next ticket there).  GemmTile computes whole tiles only: EPI is always EPI_C here.
   template <int EPI, class Hook>
   __device__ static __forceinline__ void run_tile(const ProblemDesc& pd, int tm, int tn, char* smem, bool tf32,
                                                   Hook&& before_store) {
-    static_assert(EPI == EPI_C, "the general kernel has no split-K epilogue");
+    static_assert(EPI == EPI_C, "GemmTile has no split-K epilogue");
     const int wave = threadIdx.x >> 6;
     const int wave_m = wave / WN, wave_n = wave % WN;
     const int m0 = tm * BM, n0 = tn * BN;

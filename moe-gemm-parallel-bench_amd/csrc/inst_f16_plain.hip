@@ -1,0 +1,5 @@
+// Compiled f16 kernels for operands staged element by element.
+#include "registry.h"
+namespace moegemm {
+MOEGEMM_MENU_16BIT(MOEGEMM_INST_PLAIN, EF16)
+}  // namespace moegemm

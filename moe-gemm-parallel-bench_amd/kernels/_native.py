@@ -191,12 +191,14 @@ def swiglu_tiles(dtype_code: int) -> frozenset:
     return frozenset(keys)
 
 
-# Operand layouts of the LDS-DMA kernels: 0 row-major, else these bits; GENERAL runs the general kernel.
+# Operand layouts of the LDS-DMA kernels: 0 row-major, else these bits; GENERAL runs the general kernel, and
+# STRIDED (an operand without a unit stride) the element-wise one.
 GENERAL = -1
+STRIDED = -2
 A_TRANSPOSED = 1
 B_TRANSPOSED = 2
 # vector_layout argument of the grouped launches per layout (MOEGEMM_LAYOUT_* for transposed operands).
-LAYOUT_FLAGS = {GENERAL: 0, 0: 1, 1: 0x10001, 2: 0x20001, 3: 0x30001}
+LAYOUT_FLAGS = {STRIDED: 0x40000, GENERAL: 0, 0: 1, 1: 0x10001, 2: 0x20001, 3: 0x30001}
 
 
 GENERAL_SPLIT = 4  # moegemm_kernel_layouts' bit for a general tile with a split-K kernel
@@ -219,6 +221,8 @@ def layout_tiles(dtype_code: int, layout: int) -> frozenset:
 
 def split_tiles(dtype_code: int, layout: int) -> frozenset:
     """Tile keys that can split K over operands of this layout."""
+    if layout == STRIDED:
+        return frozenset()
     return layout_tiles(dtype_code, GENERAL_SPLIT if layout == GENERAL else layout)
 
 
@@ -237,6 +241,12 @@ def _operand_layout(tensor, x_dim: int) -> int:
     if sx == 1 and sk % 8 == 0 and sk >= extent and extent % 8 == 0 and (k + _COPIED_PAST_K) * sk * 2 < _TWO_GIB:
         return 1
     return -1
+
+
+def strided_or(layout: int, a, b) -> int:
+    """``layout``, or STRIDED for general operands of which one has no unit stride: no tile stages such an
+    operand in chunks, or splits its K."""
+    return STRIDED if layout == GENERAL and (1 not in a.stride() or 1 not in b.stride()) else layout
 
 
 def transposed_layout(a, b, c) -> int:

@@ -352,18 +352,22 @@ def _problem_layout(a, b, c) -> int:
 
 
 def _group_layout(workspace: GroupedWorkspace, dtype_code: int) -> int:
-    """The one LDS-DMA layout every problem meets (0 row-major, 1 to 3 transposed), or GENERAL;
-    cached per set of tensor objects.  Homogeneous groups launch without a strides table, as row-major
+    """The one LDS-DMA layout every problem meets (0 row-major, 1 to 3 transposed), or GENERAL, or STRIDED
+    where every problem is; cached per set of tensor objects.  Homogeneous groups launch without a strides table, as row-major
     ones: with K = 1 a transposed view counts as contiguous too, and stays GENERAL there."""
-    if dtype_code == _native.DTYPE_F32:
+    if dtype_code == _native.DTYPE_F32 and workspace.homogeneous:
         return _native.GENERAL
     key = (tuple(map(id, workspace.a)), tuple(map(id, workspace.b)), tuple(map(id, workspace.c)))
     cached = getattr(workspace, "_layout_cache", None)
     if cached is not None and cached[0] == key:
         return cached[1]
-    value = _problem_layout(workspace.a[0], workspace.b[0], workspace.c[0])
+    def layout_of(a, b, c):
+        layout = _native.GENERAL if dtype_code == _native.DTYPE_F32 else _problem_layout(a, b, c)
+        return _native.strided_or(layout, a, b)
+
+    value = layout_of(workspace.a[0], workspace.b[0], workspace.c[0])
     if (value > 0 and workspace.homogeneous) or (value != _native.GENERAL and any(
-            _problem_layout(a, b, c) != value for a, b, c in workspace.problem_tensors())):
+            layout_of(a, b, c) != value for a, b, c in workspace.problem_tensors())):
         value = _native.GENERAL
     workspace._layout_cache = (key, value)
     return value

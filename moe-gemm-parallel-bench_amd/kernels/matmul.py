@@ -479,7 +479,7 @@ def _launch_fixed(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, precisio
             _LAST_SCHEDULE[0] = STREAMK
             return 1
         split_k = 1
-    layout = _operand_layout(a, b, c)
+    layout = _native.strided_or(_operand_layout(a, b, c), a, b)
     if layout == 0 or cfg.tile_key in _native.split_tiles(dtype_code, layout):
         tiles = -(-m // cfg.block_m) * -(-n // cfg.block_n)
         splits = split_k if split_k is not None else splitk_count(tiles, k, cfg.block_k,
@@ -546,7 +546,7 @@ def launch_matmul(
         m, n, k, tuple(a.stride()), tuple(b.stride()), tuple(c.stride()), dtype_code, precision,
         _device_signature(a.device), split_k, b_stream,
     )
-    layout = _operand_layout(a, b, c)
+    layout = _native.strided_or(_operand_layout(a, b, c), a, b)
     best = _AUTOTUNE_CACHE.get(key)
     if best is None:
         sm_count = _device_signature(a.device) % 1000

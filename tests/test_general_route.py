@@ -132,3 +132,59 @@ def test_negative_pitches(dtype, splits):
             _native.check(status)
             torch.cuda.synchronize()
             assert torch.equal(c, expected.to(dtype)), (form, tile)
+
+
+def _strided(rows, cols, dtype, device, gen):
+    """Integers as every second column of every second row: no unit stride."""
+    wide = torch.full((2 * rows, 2 * cols), float("nan"), device=device, dtype=dtype)
+    view = wide[::2, ::2]
+    return view.copy_(torch.randint(-2, 3, (rows, cols), generator=gen, device=device).to(dtype))
+
+
+def test_strided_operands_take_their_own_layout():
+    from kernels import _native
+    from kernels.grouped_gemm import _group_layout, workspace_from_tensors
+    from kernels.matmul import _operand_layout
+
+    gen = torch.Generator().manual_seed(1)
+    for dtype, code in ((torch.float32, _native.DTYPE_F32), (torch.float16, _native.DTYPE_F16)):
+        a, b, c = torch.zeros((24, 40), dtype=dtype), torch.zeros((40, 32), dtype=dtype), torch.zeros((24, 32), dtype=dtype)
+        odd = _strided(24, 40, dtype, "cpu", gen)
+        assert _native.strided_or(_operand_layout(odd, b, c), odd, b) == _native.STRIDED
+        assert _native.strided_or(_operand_layout(a, b, c), a, b) == (_native.GENERAL if code == _native.DTYPE_F32 else 0)
+        assert _native.strided_or(_operand_layout(a.t(), b, c), a.t().contiguous().t(), b) != _native.STRIDED
+        both = workspace_from_tensors([odd, odd[:8]], [b, b], [c, c[:8].clone()])
+        mixed = workspace_from_tensors([odd, a[:8]], [b, b], [c, c[:8].clone()])
+        assert _group_layout(both, code) == _native.STRIDED and _group_layout(mixed, code) == _native.GENERAL
+        assert _native.split_tiles(code, _native.STRIDED) == frozenset()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("shape", [(1, 1, 1), (70, 5, 67), (129, 203, 131)])
+def test_strided_operands_every_tile(dtype, shape):
+    """Alone and in groups whose problems all are strided, or only one is; K below and above one chunk."""
+    if not torch.cuda.is_available():
+        pytest.skip("ROCm GPU unavailable")
+    from kernels.grouped_gemm import launch_grouped, workspace_from_tensors
+    from kernels.matmul import KernelConfig, _menu, launch_matmul
+
+    m, k, n = shape
+    gen = torch.Generator(device="cuda").manual_seed(m + k)
+    a, b = _strided(m, k, dtype, "cuda", gen), _strided(k, n, dtype, "cuda", gen)
+    flat = b.contiguous()
+    expected = (a.double() @ b.double()).to(dtype)
+    for bm, bn, bk, warps, stages in _menu(dtype):
+        cfg = KernelConfig(bm, bn, bk, 8, warps, stages)
+        for precision in ("ieee", "tf32"):
+            print(f"strided {dtype} shape={shape} tile={cfg.tile_key} {precision}", flush=True)
+            c = torch.full((m, n + 3), float("nan"), device="cuda", dtype=dtype)[:, 1:n + 1]
+            launch_matmul(a, b, c, cfg, precision, autotune=False)
+            torch.cuda.synchronize()
+            assert torch.equal(c, expected), cfg
+        for second in (b, flat):
+            outs = [torch.full((m, n), float("nan"), device="cuda", dtype=dtype) for _ in range(2)]
+            ws = workspace_from_tensors([a, a.contiguous() if second is flat else a], [b, second], outs)
+            launch_grouped(ws, config=cfg, autotune=False)
+            torch.cuda.synchronize()
+            assert all(torch.equal(z, expected) for z in outs), cfg
