@@ -43,8 +43,13 @@
 //    (gemm_fast.h, split_store); nobody waits for another unit.
 //  * Range.  The split is exact and its products neither overflow nor lose their small parts while
 //    every non-zero operand lies in [2^-96, 2^60).  Each thread keeps the extremes of what it
-//    loaded, and the accumulators show overflow; a tile that left the range (infinities and NaN
-//    included) is computed again by GemmTile, with the fp32 instruction.
+//    loaded, and the accumulators show overflow.  A tile with smaller values reads its operands' largest
+//    value and keeps its sums if what the small ones may lack cannot show in any output (small_shows): a few
+//    such values among ordinary ones cost 12 to 29 % (fp32 [4096,2048]@[2048,1536] 153 -> 184 us,
+//    [1024,2048]@[2048,1536] 55 -> 70; the fp32 instruction alone 307 and 95).  A tile whose outputs are as
+//    small or zero, and one with infinities, NaN or (TF32) values from 2^60, is computed again by GemmTile
+//    with the fp32 instruction, which is up to three times slower than a kernel of it alone (291 us for
+//    [1024,2048]@[2048,1536]).
 #pragma once
 
 #include "gemm_fast.h"
@@ -252,6 +257,37 @@ struct GeneralTile {
 #pragma unroll
         for (int i = 0; i < ACC; ++i) worst += acc[fm][fn][i] - acc[fm][fn][i];
     return worst == 0.0f;
+  }
+  __device__ static __forceinline__ float block_max(uint32_t bits) {
+    __shared__ uint32_t s_max;
+    if (threadIdx.x == 0) s_max = 0;
+    __syncthreads();
+    atomicMax(&s_max, bits);
+    __syncthreads();
+    return __builtin_bit_cast(float, s_max);
+  }
+  // Whether what the parts lose of values below 2^-96 may show in an output of this lane.  Such a value is
+  // held to within 2^-125 (its parts below the smallest normal number may be lost), and a product of parts to
+  // within 2^-126, so a sum of `depth` products of values up to `peak` is off by less than
+  // depth * 2^-123 * (1 + 2 peak).  That is an eighth of a unit in the last place of any output from 2^27 times as
+  // much on; smaller outputs, zeros among them, ask for the fp32 instruction.
+  __device__ static __forceinline__ bool small_shows(const acc_t (&acc)[FM][FN], const ProblemDesc& pd, int m0, int n0,
+                                                     int wave_m, int wave_n, int depth, float peak) {
+    const int lane = threadIdx.x & 63;
+    const int row0 = m0 + wave_m * WTM + lane % MI;
+    const int col0 = n0 + wave_n * WTN + ((MI == 32) ? (lane >> 5) * 4 : (lane >> 4) * 4);
+    float least = __builtin_inff();
+#pragma unroll
+    for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+      for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+        for (int i = 0; i < ACC; ++i) {
+          const int gn = col0 + fn * MI + (i / 4) * 8 + i % 4;
+          const bool stored = row0 + fm * MI < pd.m && gn < pd.n;
+          least = __builtin_fminf(least, stored ? __builtin_fabsf(acc[fm][fn][i]) : __builtin_inff());
+        }
+    return least < (float)depth * 0x1p-96f * (1.0f + 2.0f * peak);
   }
   // Bits of 2^60, and twice those of 2^-96 less one.
   static constexpr uint32_t kTooLarge = (127u + 60u) << 23;
@@ -538,10 +574,32 @@ struct GeneralTile {
     for (; kt < last; kt += UNROLL) steps(std::true_type{}, kt, last);
     compute(acc, smem + (last & 1) * STAGE_BYTES, fa, fb);
     bool bad = false;
-    if constexpr (F32)  // also the barrier between this tile's LDS reads and the next tile's writes
-      bad = __syncthreads_or(range[1] < kTooSmall || (PARTS == 2 ? range[0] >= kTooLarge : !all_finite(acc))) != 0;
-    else
+    if constexpr (F32) {
+      const bool past = PARTS == 2 ? range[0] >= kTooLarge : !all_finite(acc);
+      // Also the barrier between this tile's LDS reads and the next tile's writes.
+      if (__syncthreads_or(past || range[1] < kTooSmall)) {
+        bad = __syncthreads_or(past) != 0;
+        if (!bad) {  // small values only: do they show in an output?
+          uint32_t peak = 0;  // largest |x|, as float bits
+#pragma unroll 4
+          for (int kt = 0; kt <= last; ++kt) {
+            u32x4_t va[A_PT][VL], vb[B_PT][VL];
+            a.load(va, k_first + kt * BK);
+            b.load(vb, k_first + kt * BK);
+#pragma unroll
+            for (int v = 0; v < VL * 4; ++v) {
+#pragma unroll
+              for (int i = 0; i < A_PT; ++i) peak = max(peak, va[i][v / 4][v % 4] & 0x7fffffffu);
+#pragma unroll
+              for (int i = 0; i < B_PT; ++i) peak = max(peak, vb[i][v / 4][v % 4] & 0x7fffffffu);
+            }
+          }
+          bad = __syncthreads_or(small_shows(acc, pd, m0, n0, wave_m, wave_n, k_end - k_first, block_max(peak))) != 0;
+        }
+      }
+    } else {
       __syncthreads();
+    }
     if constexpr (EPI == EPI_SPLIT) {
       const int left = reduce_splits(acc, pd, bad);
       if (left != 1) return left == 0;

@@ -225,3 +225,38 @@ def test_split_k_past_the_limits_runs_whole(shape, splits):
     expected = (a.double() @ b.double()).float()
     for out in (c[0], c[1], ws.c[0]):
         assert torch.equal(out, expected)
+
+
+@pytest.mark.parametrize("precision", ["ieee", "tf32"])
+@pytest.mark.parametrize("splits", [1, 4])
+@pytest.mark.parametrize("rows", ["mixed", "small", "zero"])
+def test_fp32_values_below_the_split_range(rows, splits, precision):
+    """Values under 2^-96 among ordinary ones, in rows of their own (whose outputs only the fp32 instruction
+    gives) and beside rows of zeros: every output within the rounding of its own sum, K products of 2^-24 each,
+    half of that for the store and half a smallest denormal."""
+    from kernels import _native
+    from kernels.matmul import launch_matmul
+
+    m, k, n = 150, 515, 140
+    gen = torch.Generator(device="cuda").manual_seed(12)
+    a = torch.randn((m, k), device="cuda", generator=gen)
+    b = torch.randn((k, n), device="cuda", generator=gen)
+    a[::7, ::5] *= 2.0**-110
+    b[3::11, 1::4] *= 2.0**-120
+    if rows == "small":
+        a[5::9] = torch.randn((len(range(5, m, 9)), k), device="cuda", generator=gen) * 2.0**-112
+    if rows == "zero":
+        a[100:120] = 0
+    x, y = a, b
+    if precision == "tf32":
+        x, y = (((t.view(torch.int32) + 0x1000) & -0x2000).view(torch.float32) for t in (a, b))
+    reference = x.double() @ y.double()
+    bound = (k + 1) * 2.0**-24 * (x.double().abs() @ y.double().abs()) + 2.0**-150
+    for cfg in _tiles(torch.float32):
+        if splits > 1 and cfg.tile_key not in _native.split_tiles(_native.DTYPE_F32, _native.GENERAL):
+            continue
+        c = torch.full((m, n), float("nan"), device="cuda")
+        print(f"fp32 below the split range {rows} {cfg.tile_key} {precision} splits={splits}", flush=True)
+        launch_matmul(a, b, c, cfg, precision, autotune=False, split_k=splits)
+        torch.cuda.synchronize()
+        assert ((c.double() - reference).abs() <= bound).all(), cfg
