@@ -553,9 +553,8 @@ def launch_grouped(
     scheduler = "homogeneous_persistent" if workspace.homogeneous else "generic_persistent"
     layout = _group_layout(workspace, dtype_code)
     if autotune:
-        # Transposed operands run other kernels than row-major ones of the same shapes.
-        key = _grouped_tuning_key(workspace, scheduler, dtype_code, precision, split_k, tile_schedule, b_stream,
-                                  max(layout, 0))
+        # Operands of the same shapes run other kernels, with other candidates, in another layout.
+        key = _grouped_tuning_key(workspace, scheduler, dtype_code, precision, split_k, tile_schedule, b_stream, layout)
         tuned = _GROUPED_AUTOTUNE_CACHE.get(key)
         if tuned is None:
             candidates = grouped_candidate_configs(
@@ -696,7 +695,7 @@ def launch_gate_up_swiglu(
         if tuned is None:
             # The plain W13 GEMM of the same workload, if already tuned, gives the preferred tile and
             # B copy policy: the activation changes only the epilogue, so a different pick would be
-            # timing noise.
+            # timing noise.  (Its operands are row-major, layout 0.)
             scheduler = "homogeneous_persistent" if workspace.homogeneous else "generic_persistent"
             plain = _GROUPED_AUTOTUNE_CACHE.get(_grouped_tuning_key(
                 workspace, scheduler, dtype_code, _native.PRECISION_IEEE, None, None))

@@ -377,6 +377,11 @@ def _operand_layout(a, b, c) -> int:
     return 0 if _vector_ok(a, b, c) else _native.transposed_layout(a, b, c)
 
 
+def _launch_layout(a, b, c) -> int:
+    """``_operand_layout``, or STRIDED."""
+    return _native.strided_or(_operand_layout(a, b, c), a, b)
+
+
 def splitk_count(tiles: int, k: int, block_k: int, sm_count: int) -> int:
     """K splits for a launch with ``tiles`` output tiles: 1 unless the tiles leave over half the CUs
     idle; otherwise enough splits to give every CU a unit, each at least 4 K slices, at most 16."""
@@ -465,11 +470,11 @@ def _launch_fixed_splitk(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, s
 
 
 def _launch_fixed(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, precision: int, split_k=None,
-                  b_stream: int = 0, scratch=_native.eager_scratch) -> int:
+                  b_stream: int = 0, *, layout: int | None = None, scratch=_native.eager_scratch) -> int:
     """One launch; returns the K splits used (``split_k`` None = ``splitk_count``'s choice,
     ``STREAMK`` = a stream-K tail where one applies, else the unsplit launch).  ``b_stream`` 1 issues
     the LDS-DMA kernels' B copies non-temporal.  ``scratch`` gives the split-K scratch of operands that
-    are not row-major 16-bit ones, or None to run whole."""
+    are not row-major 16-bit ones, or None to run whole; ``layout`` is ``_launch_layout``'s."""
     _LAST_SCHEDULE[0] = "static"
     _LAST_B_STREAM[0] = b_stream
     if split_k == STREAMK:
@@ -479,7 +484,8 @@ def _launch_fixed(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, precisio
             _LAST_SCHEDULE[0] = STREAMK
             return 1
         split_k = 1
-    layout = _native.strided_or(_operand_layout(a, b, c), a, b)
+    if layout is None:
+        layout = _launch_layout(a, b, c)
     if layout == 0 or cfg.tile_key in _native.split_tiles(dtype_code, layout):
         tiles = -(-m // cfg.block_m) * -(-n // cfg.block_n)
         splits = split_k if split_k is not None else splitk_count(tiles, k, cfg.block_k,
@@ -504,6 +510,13 @@ def _launch_fixed(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, precisio
     )
     _native.check(status)
     return 1
+
+
+def _tuning_key(a, b, c, layout: int, dtype_code: int, precision: int, split_k, b_stream) -> tuple:
+    """What a tuned option holds for.  The layout, which depends on alignment too, is part of it: operands of
+    the same shape and strides run other kernels, with other candidates, in another layout."""
+    return (tuple(a.shape), b.shape[1], a.stride(), b.stride(), c.stride(), layout, dtype_code, precision,
+            _device_signature(a.device), split_k, b_stream)
 
 
 def launch_matmul(
@@ -538,15 +551,13 @@ def launch_matmul(
         raise ValueError("split_k must be None or a positive integer")
     if b_stream not in (None, 0, 1):
         raise ValueError(f"b_stream must be None, 0 or 1, got {b_stream!r}")
+    layout = _launch_layout(a, b, c)
     if not autotune:
-        cfg = config or layout_config(select_config(m, n, k, a.dtype), dtype_code, _operand_layout(a, b, c), a.dtype)
-        _LAST_SPLIT[0] = _launch_fixed(a, b, c, m, n, k, cfg, dtype_code, precision, split_k, b_stream or 0)
+        cfg = config or layout_config(select_config(m, n, k, a.dtype), dtype_code, layout, a.dtype)
+        _LAST_SPLIT[0] = _launch_fixed(a, b, c, m, n, k, cfg, dtype_code, precision, split_k, b_stream or 0,
+                                       layout=layout)
         return
-    key = (
-        m, n, k, tuple(a.stride()), tuple(b.stride()), tuple(c.stride()), dtype_code, precision,
-        _device_signature(a.device), split_k, b_stream,
-    )
-    layout = _native.strided_or(_operand_layout(a, b, c), a, b)
+    key = _tuning_key(a, b, c, layout, dtype_code, precision, split_k, b_stream)
     best = _AUTOTUNE_CACHE.get(key)
     if best is None:
         sm_count = _device_signature(a.device) % 1000
@@ -566,13 +577,14 @@ def launch_matmul(
         twin = (lambda o: (o[0], o[1], 1)) if b_stream is None and layout >= 0 else None
         scratch = _native.TuningScratch()
         best, _WHOLE_OPTIONS[key] = _tune(
-            options, lambda o: _launch_fixed(a, b, c, m, n, k, o[0], dtype_code, precision, *o[1:], scratch), twin=twin,
-            fallback=lambda o: o[1] == 1)
+            options, lambda o: _launch_fixed(a, b, c, m, n, k, o[0], dtype_code, precision, *o[1:], layout=layout,
+                                             scratch=scratch), twin=twin, fallback=lambda o: o[1] == 1)
         _AUTOTUNE_CACHE[key] = best
     if layout != 0 and best[1] != 1 and _native.capturing():
         best = _WHOLE_OPTIONS.get(key) or best  # a captured launch has no scratch
     _LAST_AUTOTUNED[0] = best[0]
-    _LAST_SPLIT[0] = _launch_fixed(a, b, c, m, n, k, best[0], dtype_code, precision, best[1], best[2])
+    _LAST_SPLIT[0] = _launch_fixed(a, b, c, m, n, k, best[0], dtype_code, precision, best[1], best[2],
+                                   layout=layout)
 
 
 def _warm_clocks(launch, budget_ms: float = 100.0) -> None:
