@@ -262,6 +262,7 @@ def transposed_layout(a, b, c) -> int:
     return (A_TRANSPOSED if la == 1 else 0) | (B_TRANSPOSED if lb == 0 else 0) or GENERAL
 
 
+@lru_cache(maxsize=4096)
 def splitk_workspace_bytes(tiles: int, splits: int, block_m: int, block_n: int) -> int:
     out = _i64(0)
     check(library().moegemm_splitk_workspace_bytes(tiles, splits, block_m, block_n, ctypes.byref(out)))

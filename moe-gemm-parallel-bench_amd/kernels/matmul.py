@@ -19,6 +19,7 @@ from __future__ import annotations
 
 import math
 from dataclasses import asdict, dataclass
+from functools import lru_cache
 
 from utils.benchmark import hot_autotune_bench
 
@@ -89,6 +90,7 @@ _MATMUL_CONFIG_POOL: tuple[KernelConfig, ...] = config_pool()
 _MATMUL_CONFIG_POOL_F32: tuple[KernelConfig, ...] = config_pool("fp32")
 
 
+@lru_cache(maxsize=4096)
 def _snap(block_m: int, block_n: int, block_k: int, dtype=None, group: int = 8, tiles=None) -> KernelConfig:
     """The compiled tile nearest to a wanted (block_m, block_n, block_k), in log2 distance, among the
     tile keys ``tiles`` (all when None)."""
@@ -310,6 +312,7 @@ _WHOLE_OPTIONS: dict[tuple, tuple] = {}  # by the same key: the fastest option t
 _LAST_AUTOTUNED: list[KernelConfig | None] = [None]
 
 
+@lru_cache(maxsize=None)
 def _device_signature(device) -> int:
     import torch
 
@@ -350,9 +353,7 @@ def _require_runtime(tensor=None) -> None:
 
 def _vector_ok(a, b, c) -> bool:
     """Preconditions of the LDS-DMA kernels for one 16-bit problem (see include/moegemm.h)."""
-    import torch
-
-    if a.dtype not in (torch.float16, torch.bfloat16):
+    if a.element_size() != 2:
         return False
     k = a.shape[1]
     n = b.shape[1]
@@ -377,9 +378,13 @@ def _operand_layout(a, b, c) -> int:
     return 0 if _vector_ok(a, b, c) else _native.transposed_layout(a, b, c)
 
 
-def _launch_layout(a, b, c) -> int:
+def _launch_layout(a, b, c, dtype_code: int) -> int:
     """``_operand_layout``, or STRIDED."""
-    return _native.strided_or(_operand_layout(a, b, c), a, b)
+    if dtype_code != _native.DTYPE_F32:
+        layout = 0 if _vector_ok(a, b, c) else _native.transposed_layout(a, b, c)
+        if layout != _native.GENERAL:
+            return layout
+    return _native.strided_or(_native.GENERAL, a, b)
 
 
 def splitk_count(tiles: int, k: int, block_k: int, sm_count: int) -> int:
@@ -485,7 +490,7 @@ def _launch_fixed(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, precisio
             return 1
         split_k = 1
     if layout is None:
-        layout = _launch_layout(a, b, c)
+        layout = _launch_layout(a, b, c, dtype_code)
     if layout == 0 or cfg.tile_key in _native.split_tiles(dtype_code, layout):
         tiles = -(-m // cfg.block_m) * -(-n // cfg.block_n)
         splits = split_k if split_k is not None else splitk_count(tiles, k, cfg.block_k,
@@ -551,7 +556,7 @@ def launch_matmul(
         raise ValueError("split_k must be None or a positive integer")
     if b_stream not in (None, 0, 1):
         raise ValueError(f"b_stream must be None, 0 or 1, got {b_stream!r}")
-    layout = _launch_layout(a, b, c)
+    layout = _launch_layout(a, b, c, dtype_code)
     if not autotune:
         cfg = config or layout_config(select_config(m, n, k, a.dtype), dtype_code, layout, a.dtype)
         _LAST_SPLIT[0] = _launch_fixed(a, b, c, m, n, k, cfg, dtype_code, precision, split_k, b_stream or 0,

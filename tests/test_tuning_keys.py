@@ -58,3 +58,20 @@ def test_aligned_and_unaligned_groups_are_tuned_apart(tuned):
         b, c = ([_offset(*shape, torch.float16, 0) for _ in range(2)] for shape in ((256, 64), (64, 64)))
         grouped_gemm.launch_grouped(grouped_gemm.workspace_from_tensors(a, b, c))
         assert len(grouped_gemm._GROUPED_AUTOTUNE_CACHE) == min(count, 2)
+
+
+def test_repeated_untuned_calls_search_no_menu(tuned, monkeypatch):
+    """An untuned call's tile is looked up, not searched for again: the search took as long as a small launch."""
+    operands = []
+    for dtype, flip in ((torch.bfloat16, True), (torch.bfloat16, False), (torch.float32, False)):
+        b = _offset(104, 264, dtype, 0).t() if flip else _offset(264, 104, dtype, 0)
+        operands.append((_offset(24, 264, dtype, 0), b, _offset(24, 104, dtype, 0)))
+    for a, b, c in operands:
+        matmul.launch_matmul(a, b, c, autotune=False)
+
+    def searched(dtype=None):
+        raise AssertionError("the menu was searched")
+
+    monkeypatch.setattr(matmul, "_menu", searched)
+    for a, b, c in operands:
+        matmul.launch_matmul(a, b, c, autotune=False)
