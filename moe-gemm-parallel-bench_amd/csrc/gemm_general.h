@@ -23,12 +23,16 @@
 //    are exact in the fp32 accumulation.  The six largest are computed; the three dropped ones
 //    (x1 y2, x2 y1, x2 y2) are below 2^-25 of the product, less than the rounding of one fp32
 //    addition.  TF32 operands (11 significand bits) are the exact sum of two bf16 values, and all
-//    four products are computed.  The accumulator is rounded once per 16 (32) products instead of
-//    once per product, so results are closer to the exact product than the fp32 instruction's.
-//    Chunks are split on their way into LDS, once per workgroup, into one LDS panel per part.
+//    four products are computed.  The accumulator is rounded once per 16 (32) products and part instead of
+//    once per product, so long sums of like products are closer to the exact ones than the fp32
+//    instruction's.  Chunks are split on their way into LDS, once per workgroup, into one LDS panel per part.
 //    Relative error against 64 bits, normal operands, fp32 instruction -> parts: 1.45e-7 -> 1.10e-7
-//    at K = 64, 1.51e-6 -> 1.34e-6 at K = 7168; TF32 1.34e-7 -> 0.88e-7 and 1.51e-6 -> 1.06e-6.
-//    Below K = 8 the fp32 instruction is closer and runs.
+//    at K = 64, 1.51e-6 -> 1.34e-6 at K = 7168; TF32 1.34e-7 -> 0.88e-7 and 1.51e-6 -> 1.06e-6; the same
+//    at scales down to products of 2^-125, whose subnormal parts the matrix cores keep.  Sums of few products
+//    are further off, because all parts of a product round into one sum: rows of K = 512 with one value
+//    other than zero 2.5e-8 -> 3.5e-8 (at most 0.5 -> 1.4 units in the last place), two 3.1e-8 -> 5.2e-8,
+//    eight 5.4e-8 -> 1.1e-7; TF32 0 -> 0, 1.7e-8 -> 1.9e-8, 4.6e-8 -> 5.2e-8.  Below K = 8 the fp32
+//    instruction runs.
 //  * Bound and measured.  Large fp32 tiles are bound by the matrix cores and by the split's vector
 //    instructions (about 7.5 an element in IEEE mode, 7 in TF32), so the eight-wave 256x128 tile, which
 //    splits each element for twice the MFMAs of a 64-wide tile, leads: 4 x [2048,4096]@[4096,4096] runs

@@ -260,3 +260,57 @@ def test_fp32_values_below_the_split_range(rows, splits, precision):
         launch_matmul(a, b, c, cfg, precision, autotune=False, split_k=splits)
         torch.cuda.synchronize()
         assert ((c.double() - reference).abs() <= bound).all(), cfg
+
+
+@pytest.mark.parametrize("precision", ["ieee", "tf32"])
+@pytest.mark.parametrize("total", [-108, -116, -122, -128])
+def test_fp32_products_near_the_smallest_normal_number(total, precision):
+    """Products of about 2^total, whose smaller parts are subnormal: the matrix cores keep those.  Bounds as for
+    ordinary values, and each output off by half a smallest subnormal for the six (four) sums of its every 16
+    products and its store."""
+    from kernels.matmul import launch_matmul
+
+    k = 64
+    bound = (2 * (k / 2) ** 0.5 + 2) * 2.0**-25
+    for a_scale in (total // 2, -20):
+        gen = torch.Generator(device="cuda").manual_seed(k)
+        a = torch.randn((130, k), device="cuda", generator=gen) * 2.0**a_scale
+        b = torch.randn((k, 129), device="cuda", generator=gen) * 2.0 ** (total - a_scale)
+        x, y = a, b
+        if precision == "tf32":
+            x, y = (((t.view(torch.int32) + 0x1000) & -0x2000).view(torch.float32) for t in (a, b))
+        expected = x.double() @ y.double()
+        subnormal = (6 * k / 16 + 1) * 2.0**-150 * expected.numel() ** 0.5
+        for cfg in _tiles(torch.float32):
+            c = torch.empty((130, 129), device="cuda")
+            print(f"fp32 small products {cfg.tile_key} {precision} 2^{a_scale} x 2^{total - a_scale}", flush=True)
+            launch_matmul(a, b, c, cfg, precision, autotune=False)
+            torch.cuda.synchronize()
+            error = float((c.double() - expected).norm())
+            assert error <= bound * float(expected.norm()) + subnormal, (cfg, error)
+
+
+@pytest.mark.parametrize("precision", ["ieee", "tf32"])
+@pytest.mark.parametrize("terms", [1, 2, 8])
+def test_fp32_sums_of_few_products(terms, precision):
+    """Rows of A with few values other than zero.  Six (four) instructions add a product's parts, each off by at
+    most 2^-23 of what the sum holds then; the dropped parts are below 2^-25 of their product."""
+    from kernels.matmul import launch_matmul
+
+    m, k, n = 150, 512, 140
+    gen = torch.Generator(device="cuda").manual_seed(21)
+    a, rows = torch.zeros((m, k), device="cuda"), torch.arange(m, device="cuda")
+    for j in range(terms):
+        a[rows, (rows * 7 + 61 * j) % k] = torch.randn(m, device="cuda", generator=gen)
+    b = torch.randn((k, n), device="cuda", generator=gen)
+    x, y = a, b
+    if precision == "tf32":
+        x, y = (((t.view(torch.int32) + 0x1000) & -0x2000).view(torch.float32) for t in (a, b))
+    reference = x.double() @ y.double()
+    bound = ((6 * terms) * 2.0**-23 + 2.0**-25) * (x.double().abs() @ y.double().abs())
+    for cfg in _tiles(torch.float32):
+        c = torch.full((m, n), float("nan"), device="cuda")
+        print(f"fp32 sums of {terms} products {cfg.tile_key} {precision}", flush=True)
+        launch_matmul(a, b, c, cfg, precision, autotune=False)
+        torch.cuda.synchronize()
+        assert ((c.double() - reference).abs() <= bound).all(), cfg
