@@ -23,16 +23,19 @@
 //    are exact in the fp32 accumulation.  The six largest are computed; the three dropped ones
 //    (x1 y2, x2 y1, x2 y2) are below 2^-25 of the product, less than the rounding of one fp32
 //    addition.  TF32 operands (11 significand bits) are the exact sum of two bf16 values, and all
-//    four products are computed.  The accumulator is rounded once per 16 (32) products and part instead of
-//    once per product, so long sums of like products are closer to the exact ones than the fp32
-//    instruction's.  Chunks are split on their way into LDS, once per workgroup, into one LDS panel per part.
-//    Relative error against 64 bits, normal operands, fp32 instruction -> parts: 1.45e-7 -> 1.10e-7
-//    at K = 64, 1.51e-6 -> 1.34e-6 at K = 7168; TF32 1.34e-7 -> 0.88e-7 and 1.51e-6 -> 1.06e-6; the same
-//    at scales down to products of 2^-125, whose subnormal parts the matrix cores keep.  Sums of few products
-//    are further off, because all parts of a product round into one sum: rows of K = 512 with one value
-//    other than zero 2.5e-8 -> 3.5e-8 (at most 0.5 -> 1.4 units in the last place), two 3.1e-8 -> 5.2e-8,
-//    eight 5.4e-8 -> 1.1e-7; TF32 0 -> 0, 1.7e-8 -> 1.9e-8, 4.6e-8 -> 5.2e-8.  Below K = 8 the fp32
-//    instruction runs.
+//    four products are computed.  Products whose parts are not both the first are summed apart from the
+//    rest and added once, at the end of the tile: in one sum all parts of a product would round at the size of
+//    the whole.  So sums are as close to the exact ones as the fp32 instruction's, few products or many
+//    (error against 64 bits, fp32 instruction -> one sum of all parts -> now, normal operands, 2-norms):
+//      K = 64                      1.43e-7 -> 1.07e-7 -> 4.8e-8     TF32 1.30e-7 -> 8.5e-8 -> 4.8e-8
+//      K = 2048                                 7.0e-7 -> 2.7e-7              5.6e-7 -> 1.8e-7
+//      rows of K = 512 with 8 values other than zero
+//                                  5.4e-8 -> 1.09e-7 -> 2.9e-8      TF32 4.6e-8 -> 5.2e-8 -> 2.9e-8
+//      with one                    2.54e-8 -> 3.5e-8 -> 2.60e-8     TF32 0 -> 0 -> 0
+//    and the same at scales down to products of 2^-125, whose subnormal parts the matrix cores keep.  It
+//    costs 3 to 8 % on large fp32 calls (8 x [512,2048]@[2048,1536] 149 -> 159 us, 4 x [2048,4096]@[4096,4096]
+//    1324 -> 1362 us), 2 to 8 % in TF32, nothing on small ones.  Below K = 8 the fp32 instruction runs.
+//    Chunks are split on their way into LDS, once per workgroup, into one LDS panel per part.
 //  * Bound and measured.  Large fp32 tiles are bound by the matrix cores and by the split's vector
 //    instructions (about 7.5 an element in IEEE mode, 7 in TF32), so the eight-wave 256x128 tile, which
 //    splits each element for twice the MFMAs of a 64-wide tile, leads: 4 x [2048,4096]@[4096,4096] runs
@@ -82,6 +85,9 @@ struct GeneralTile {
   static constexpr int FM = WTM / MI, FN = WTN / MI;
   static constexpr int ACC = MI * MI / 64;
   static constexpr int PRODUCTS = PARTS == 3 ? 6 : PARTS * PARTS;  // MFMAs per fragment pair and K step
+  static constexpr int LM = PARTS > 1 ? FM : 1, LN = PARTS > 1 ? FN : 1;  // sums of the small products
+  // Two sums of 64 registers and all of a K step's fragments are more than a wave's registers hold.
+  static constexpr bool TIGHT = PARTS == 3 && FM * FN * ACC >= 64 && NW == 8;
   static constexpr int VL = ES / 2;  // 16-byte loads per 8-element chunk
   static constexpr int A_CHUNKS = BM * BK / 8, B_CHUNKS = BK * BN / 8;
   static constexpr int A_PT = (A_CHUNKS + NT - 1) / NT, B_PT = (B_CHUNKS + NT - 1) / NT;
@@ -360,38 +366,74 @@ struct GeneralTile {
   static constexpr bool READ_AHEAD =
       NW <= 4 && KK * STEP_REGS + FM * FN * ACC + DEPTH * SLICE_REGS <= (WAVES_PER_EU == 1 ? 320 : 160);
 
+  // Products whose parts are not both the first go to sums of their own: those parts then round into a sum
+  // of their size, and the first parts' products, which have 16 significant bits, hardly round at all.
   template <class FA, class FB>
-  __device__ static __forceinline__ void compute(acc_t (&acc)[FM][FN], const char* lds, const FA& fa, const FB& fb) {
+  __device__ static __forceinline__ void compute(acc_t (&acc)[FM][FN], acc_t (&low)[LM][LN], const char* lds,
+                                                 const FA& fa, const FB& fb) {
     i16x8_t af[KK][PARTS][FM], bf[KK][PARTS][FN];
-    auto read = [&](int kk) {
+    auto read_a = [&](int kk, int q) {
 #pragma unroll
-      for (int q = 0; q < PARTS; ++q) {
-#pragma unroll
-        for (int fm = 0; fm < FM; ++fm) af[kk][q][fm] = fa.get(lds + q * A_BYTES, fm, kk);
-#pragma unroll
-        for (int fn = 0; fn < FN; ++fn) bf[kk][q][fn] = fb.get(lds + PARTS * A_BYTES + q * B_BYTES, fn, kk);
-      }
+      for (int fm = 0; fm < FM; ++fm) af[kk][q][fm] = fa.get(lds + q * A_BYTES, fm, kk);
     };
+    auto read_b = [&](int kk, int q) {
+#pragma unroll
+      for (int fn = 0; fn < FN; ++fn) bf[kk][q][fn] = fb.get(lds + PARTS * A_BYTES + q * B_BYTES, fn, kk);
+    };
+    auto multiply = [&](int kk, int qa, int qb) {
+#pragma unroll
+      for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+        for (int fn = 0; fn < FN; ++fn) {
+          acc_t& to = qa + qb > 0 ? low[fm % LM][fn % LN] : acc[fm][fn];
+          to = mfma(bf[kk][qb][fn], af[kk][qa][fm], to);
+        }
+    };
+    constexpr int kMemoryMayCross = 0x0216;  // vector, scalar, global memory and LDS writes may cross
     if constexpr (READ_AHEAD) {
 #pragma unroll
-      for (int kk = 0; kk < KK; ++kk) read(kk);
-      __builtin_amdgcn_sched_barrier(0x0216);  // vector, scalar, global memory and LDS writes may cross
+      for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+        for (int q = 0; q < PARTS; ++q) {
+          read_a(kk, q);
+          read_b(kk, q);
+        }
+      __builtin_amdgcn_sched_barrier(kMemoryMayCross);
     }
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
-      if constexpr (!READ_AHEAD) read(kk);
-      // Products in falling order of the parts' sum: the small ones are added first.
+      if constexpr (TIGHT) {  // A's parts one ahead of their products
+        read_a(kk, 2);
+        read_b(kk, 0);
+        read_a(kk, 1);
+        read_b(kk, 1);
+        read_b(kk, 2);
+        __builtin_amdgcn_sched_barrier(kMemoryMayCross);
+        multiply(kk, 2, 0);
+        read_a(kk, 0);
+        __builtin_amdgcn_sched_barrier(kMemoryMayCross);
+        multiply(kk, 1, 1);
+        multiply(kk, 1, 0);
+        multiply(kk, 0, 2);
+        multiply(kk, 0, 1);
+        multiply(kk, 0, 0);
+      } else {
+        if constexpr (!READ_AHEAD) {
 #pragma unroll
-      for (int sum = PARTS == 3 ? 2 : 2 * (PARTS - 1); sum >= 0; --sum)
-#pragma unroll
-        for (int qa = 0; qa < PARTS; ++qa) {
-          const int qb = sum - qa;
-          if (qb < 0 || qb >= PARTS) continue;
-#pragma unroll
-          for (int fm = 0; fm < FM; ++fm)
-#pragma unroll
-            for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = mfma(bf[kk][qb][fn], af[kk][qa][fm], acc[fm][fn]);
+          for (int q = 0; q < PARTS; ++q) {
+            read_a(kk, q);
+            read_b(kk, q);
+          }
         }
+        // Products in falling order of the parts' sum: the small ones are added first.
+#pragma unroll
+        for (int sum = PARTS == 3 ? 2 : 2 * (PARTS - 1); sum >= 0; --sum)
+#pragma unroll
+          for (int qa = 0; qa < PARTS; ++qa) {
+            const int qb = sum - qa;
+            if (qb >= 0 && qb < PARTS) multiply(kk, qa, qb);
+          }
+      }
     }
   }
 
@@ -514,13 +556,13 @@ struct GeneralTile {
     Frags<!BT, BN, FN> fb;
     fa.setup(wave_m * WTM);
     fb.setup(wave_n * WTN);
-    acc_t acc[FM][FN];
+    acc_t acc[FM][FN], low[LM][LN];
 #pragma unroll
     for (int fm = 0; fm < FM; ++fm)
 #pragma unroll
       for (int fn = 0; fn < FN; ++fn)
 #pragma unroll
-        for (int i = 0; i < ACC; ++i) acc[fm][fn][i] = 0.0f;
+        for (int i = 0; i < ACC; ++i) acc[fm][fn][i] = low[fm % LM][fn % LN][i] = 0.0f;
     uint32_t range[2] = {0u, 0xffffffffu};
 
     // K slices first .. first + last, from k_first on; a unit's range starts at a whole slice.
@@ -549,7 +591,7 @@ struct GeneralTile {
       using ahead = std::integral_constant<int, (J + DEPTH) % UNROLL>;
       using next = std::integral_constant<int, (J + 1) % UNROLL>;
       load(ahead{}, kt + DEPTH);
-      compute(acc, smem + (J % 2) * STAGE_BYTES, fa, fb);
+      compute(acc, low, smem + (J % 2) * STAGE_BYTES, fa, fb);
       store(next{}, edge, kt + 1);
       __syncthreads();
     };
@@ -576,9 +618,15 @@ struct GeneralTile {
       for (; kt + UNROLL < inner; kt += UNROLL) steps(std::false_type{}, kt, 0);
     }
     for (; kt < last; kt += UNROLL) steps(std::true_type{}, kt, last);
-    compute(acc, smem + (last & 1) * STAGE_BYTES, fa, fb);
+    compute(acc, low, smem + (last & 1) * STAGE_BYTES, fa, fb);
     bool bad = false;
     if constexpr (F32) {
+#pragma unroll
+      for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+        for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+          for (int i = 0; i < ACC; ++i) acc[fm][fn][i] += low[fm % LM][fn % LN][i];
       const bool past = PARTS == 2 ? range[0] >= kTooLarge : !all_finite(acc);
       // Also the barrier between this tile's LDS reads and the next tile's writes.
       if (__syncthreads_or(past || range[1] < kTooSmall)) {
