@@ -366,14 +366,24 @@ def eager_scratch(device, stream_handle: int, tiles: int, splits: int, block_m: 
 
 class TuningScratch:
     """What a tuner's timings use in place of ``eager_scratch``: one buffer for all candidates, which run one
-    after the other, given back when the tuner is done.  The tuner's own captured graphs may use it: each is
-    replayed and dropped before the next candidate runs."""
+    after the other, given back when the ``with`` block ends.  The tuner's own captured graphs may use it:
+    each is replayed and dropped before the next candidate runs."""
 
     def __init__(self):
         import torch
 
         self._home = torch.cuda.current_stream()
         self._buffer = None
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *error):
+        import torch
+
+        if self._buffer is not None:
+            torch.cuda.synchronize(self._buffer.device)  # whatever a failed candidate left on another stream
+            self._buffer = None
 
     def __call__(self, device, stream_handle: int, tiles: int, splits: int, block_m: int, block_n: int):
         import torch
@@ -384,7 +394,7 @@ class TuningScratch:
         if self._buffer is None or self._buffer.numel() < nbytes:
             if capturing():
                 return None
-            torch.cuda.synchronize(device)  # whatever a failed candidate left on another stream
+            torch.cuda.synchronize(device)  # as in __exit__
             self._buffer = None
             with torch.cuda.stream(self._home):  # one stream's memory, whichever stream times
                 self._buffer = torch.zeros(nbytes, dtype=torch.uint8, device=device)

@@ -575,10 +575,11 @@ def launch_grouped(
             # The B copy policy is timed on the finalists where it is not pinned and the LDS-DMA kernels run.
             twin = ((lambda o: (o[0], o[1], o[2], 1))
                     if b_stream is None and layout >= 0 else None)
-            scratch = _native.TuningScratch()
-            tuned, _GROUPED_WHOLE_OPTIONS[key] = _tune(
-                options, lambda o: _launch_grouped_fixed(workspace, o[0], dtype_code, precision, *o[1:], layout, scratch),
-                twin=twin, fallback=lambda o: o[1] == 1 and o[2] == "static")
+            with _native.TuningScratch() as scratch:
+                tuned, _GROUPED_WHOLE_OPTIONS[key] = _tune(
+                    options, lambda o: _launch_grouped_fixed(workspace, o[0], dtype_code, precision, *o[1:], layout,
+                                                             scratch),
+                    twin=twin, fallback=lambda o: o[1] == 1 and o[2] == "static")
             _GROUPED_AUTOTUNE_CACHE[key] = tuned
         if layout != 0 and tuned[1] != 1 and _native.capturing():
             tuned = _GROUPED_WHOLE_OPTIONS.get(key) or tuned  # a captured launch has no scratch

@@ -154,7 +154,12 @@ def select_ragged_config(mean_m: int, n: int, k: int, dtype=None, *, groups: int
     Few rounds of tiles make that a matter of the counts: a round of 256x256 tiles takes about as long as
     one and a half of 128x256 tiles, and the last round takes as long as a full one.  On 245 groups (96
     to 400 rows, seven K x N, five routings each) choosing by rounds is 0.6 % behind the better of the
-    two on average (at most 13 %), the line at 224 rows 2.1 % (31 %)."""
+    two on average (at most 13 %), the line at 224 rows 2.1 % (31 %).
+
+    Pointer groups of other layouts use the same rule (the nearest tile compiled for theirs).  On 18 groups
+    each (2 to 64 problems, 4 to 256 rows, five K x N) it is 3.6 % behind the best tile on average with
+    weights stored [N, K] (at most 30 %; the first problem's tile 28 %) and 0.7 % with unaligned rows (12 %;
+    the first problem's tile 95 %)."""
     if _is_f32(dtype) or n <= 128:
         return select_config(mean_m, n, k, dtype)
     for tile in _FEW_TILES:
@@ -580,10 +585,10 @@ def launch_matmul(
         options = [(cfg, split, b_stream or 0) for cfg, split in options]
         # The B copy policy is timed on the finalists where it is not pinned and the LDS-DMA kernels run.
         twin = (lambda o: (o[0], o[1], 1)) if b_stream is None and layout >= 0 else None
-        scratch = _native.TuningScratch()
-        best, _WHOLE_OPTIONS[key] = _tune(
-            options, lambda o: _launch_fixed(a, b, c, m, n, k, o[0], dtype_code, precision, *o[1:], layout=layout,
-                                             scratch=scratch), twin=twin, fallback=lambda o: o[1] == 1)
+        with _native.TuningScratch() as scratch:
+            best, _WHOLE_OPTIONS[key] = _tune(
+                options, lambda o: _launch_fixed(a, b, c, m, n, k, o[0], dtype_code, precision, *o[1:], layout=layout,
+                                                 scratch=scratch), twin=twin, fallback=lambda o: o[1] == 1)
         _AUTOTUNE_CACHE[key] = best
     if layout != 0 and best[1] != 1 and _native.capturing():
         best = _WHOLE_OPTIONS.get(key) or best  # a captured launch has no scratch

@@ -185,6 +185,9 @@ def test_strided_operands_every_tile(dtype, shape):
         for second in (b, flat):
             outs = [torch.full((m, n), float("nan"), device="cuda", dtype=dtype) for _ in range(2)]
             ws = workspace_from_tensors([a, a.contiguous() if second is flat else a], [b, second], outs)
-            launch_grouped(ws, config=cfg, autotune=False)
-            torch.cuda.synchronize()
-            assert all(torch.equal(z, expected) for z in outs), cfg
+            for schedule in ("static", "stealing"):
+                for z in outs:
+                    z.fill_(float("nan"))
+                launch_grouped(ws, config=cfg, autotune=False, tile_schedule=schedule)
+                torch.cuda.synchronize()
+                assert all(torch.equal(z, expected) for z in outs), (cfg, schedule)

@@ -3,6 +3,8 @@ when their alignment differs."""
 
 from __future__ import annotations
 
+import contextlib
+
 import pytest
 import torch
 
@@ -24,7 +26,7 @@ def tuned(monkeypatch):
 
     monkeypatch.setattr(_native, "library", Nothing)
     monkeypatch.setattr(_native, "current_stream_handle", lambda device: 7)
-    monkeypatch.setattr(_native, "TuningScratch", lambda: None)
+    monkeypatch.setattr(_native, "TuningScratch", contextlib.nullcontext)
     monkeypatch.setattr(_native, "eager_scratch", lambda *args: None)
     monkeypatch.setattr(_native, "capturing", lambda: False)
     monkeypatch.setattr(matmul, "_device_signature", lambda device: 950256)
