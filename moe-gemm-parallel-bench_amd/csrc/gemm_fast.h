@@ -128,8 +128,8 @@ __device__ __forceinline__ void wait_vmcnt() {
 // pass or a register shuffle: only the copy addresses and the fragment reads differ.  Bound as the
 // row-major tiles are (HBM at few rows, matrix cores otherwise); the general kernel, which took such
 // operands before, was bound by its 2-byte gathers.  Measured (bf16, tuned, before -> after):
-// [16,4096]@[4096,14336] with B stored [N, K] 110 -> 24 us (4.9 TB/s); dC B^T and A^T dC of
-// [1024,4096]@[4096,3584] together 253 -> 63 us (957 TFLOP/s).
+// [16,4096]@[4096,14336] with B stored [N, K] 110 -> 24 to 26 us by card (4.5 to 4.9 TB/s); dC B^T and A^T dC of
+// [1024,4096]@[4096,3584] together 253 -> 62 to 68 us (890 to 970 TFLOP/s).
 template <class E, int BM_, int BN_, int BK_, int WM_, int WN_, int STAGES_, int LAY_ = 0>
 struct FastTile {
   static_assert(!E::is_f32, "the DMA fast path is for 16-bit operands");

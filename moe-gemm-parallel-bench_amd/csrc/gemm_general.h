@@ -38,16 +38,19 @@
 //    Chunks are split on their way into LDS, once per workgroup, into one LDS panel per part.
 //  * Bound and measured.  Large fp32 tiles are bound by the matrix cores and by the split's vector
 //    instructions (about 7.5 an element in IEEE mode, 7 in TF32), so the eight-wave 256x128 tile, which
-//    splits each element for twice the MFMAs of a 64-wide tile, leads: 4 x [2048,4096]@[4096,4096] runs
-//    at 190 TFLOP/s (1140 of bf16 MFMA work), TF32 at 255; the fp32 instruction's nominal peak is 157.
-//    8 x [512,2048]@[2048,1536] 458 -> 185 us; TF32 [1024,4096]@[4096,3584] 669 -> 131 us; fp16
-//    [777,2881]@[2881,1443] 148 -> 38 us (element-wise gathers before); bf16
-//    [4001,4003]@[4003,4005] runs at 814 TFLOP/s.
+//    splits each element for twice the MFMAs of a 64-wide tile, leads: 4 x [2048,4096]@[4096,4096] runs at 202
+//    TFLOP/s (1211 of bf16 MFMA work; matrix cores busy in 57 % of the cycles, vector issue in 35 %), TF32 on
+//    128x128 tiles at 253 (46 and 49 %); the fp32 instruction's nominal peak is 157.  8 x [512,2048]@[2048,1536]
+//    459 -> 168 us (192 tiles on 256 CUs: 37 and 24 %); TF32 [1024,4096]@[4096,3584] 676 -> 132 us.  16-bit
+//    tiles are bound by the latency of a slice's loads where few workgroups share a CU: fp16
+//    [777,2881]@[2881,1443] 148 -> 39 us whole, 29 in three splits (element-wise gathers before), with the
+//    matrix cores busy in 8 %; bf16 [4001,4003]@[4003,4005] runs at 873 TFLOP/s.
 //  * Split-K.  Few tiles leave the chip idle, and a lone workgroup on a CU runs at the latency of its
 //    steps, so a tile's K slices can be shared by several workgroups (fp32 [64,4096]@[4096,1024]:
-//    66 us whole, 21 us in eight; the reduction costs about 5 us, so large groups stay whole): each stores its fp32 partial, and the last to arrive sums them in split order
-//    (deterministic) and stores C.  Counters, partial layout and coherence are FastTile's
-//    (gemm_fast.h, split_store); nobody waits for another unit.
+//    64 us whole, 17 us in sixteen; the reduction costs about 5 us, so large groups stay whole): each
+//    stores its fp32 partial, and the last to arrive sums them in split order (deterministic) and stores C.
+//    Counters, partial layout and coherence are FastTile's (gemm_fast.h, split_store); nobody waits for
+//    another unit.
 //  * Range.  The split is exact and its products neither overflow nor lose their small parts while
 //    every non-zero operand lies in [2^-96, 2^60).  Each thread keeps the extremes of what it
 //    loaded, and the accumulators show overflow.  A tile with smaller values reads its operands' largest
@@ -55,8 +58,8 @@
 //    such values among ordinary ones cost 12 to 29 % (fp32 [4096,2048]@[2048,1536] 153 -> 184 us,
 //    [1024,2048]@[2048,1536] 55 -> 70; the fp32 instruction alone 307 and 95).  A tile whose outputs are as
 //    small or zero, and one with infinities, NaN or (TF32) values from 2^60, is computed again by GemmTile
-//    with the fp32 instruction, which is up to three times slower than a kernel of it alone (291 us for
-//    [1024,2048]@[2048,1536]).
+//    with the fp32 instruction, which is up to four times slower than a kernel of it alone
+//    ([1024,2048]@[2048,1536] with an infinity in every tile: 348 us against 95).
 #pragma once
 
 #include "gemm_fast.h"
@@ -232,8 +235,8 @@ struct GeneralTile {
   // wraps to the top).  range[0], TF32 only: the largest |x| (as float bits; a NaN stays), because
   // rounding can turn a NaN into a number.  In IEEE mode large values need no watch: whatever
   // overflows in the parts or their products (infinities and NaN too) leaves an accumulator that is
-  // not finite (all_finite).  The register it saves ended spills in the 256x128 loop: 214 -> 185 us on
-  // 8 x [512,2048]@[2048,1536].
+  // not finite (all_finite).  The register it saves ended most spills of the 256x128 loop (185 -> 157 us on
+  // 8 x [512,2048]@[2048,1536] when it went).
   __device__ static __forceinline__ void split(const u32x4_t (&in)[VL], u32x4_t (&part)[PARTS], uint32_t (&range)[2]) {
     if constexpr (!F32) {
       part[0] = in[0];
