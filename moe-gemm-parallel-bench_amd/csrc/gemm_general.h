@@ -33,18 +33,18 @@
 //                                  5.4e-8 -> 1.09e-7 -> 2.9e-8      TF32 4.6e-8 -> 5.2e-8 -> 2.9e-8
 //      with one                    2.54e-8 -> 3.5e-8 -> 2.60e-8     TF32 0 -> 0 -> 0
 //    and the same at scales down to products of 2^-125, whose subnormal parts the matrix cores keep.  It
-//    costs 3 to 8 % on large fp32 calls (8 x [512,2048]@[2048,1536] 149 -> 159 us, 4 x [2048,4096]@[4096,4096]
-//    1324 -> 1362 us), 2 to 8 % in TF32, nothing on small ones.  Below K = 8 the fp32 instruction runs.
+//    costs up to 5 % on large calls (8 x [512,2048]@[2048,1536] 152 -> 154 us, 4 x [2048,4096]@[4096,4096]
+//    1382 -> 1403 us, TF32 1071 -> 1097 us).  Below K = 8 the fp32 instruction runs.
 //    Chunks are split on their way into LDS, once per workgroup, into one LDS panel per part.
 //  * Bound and measured.  Large fp32 tiles are bound by the matrix cores and by the split's vector
 //    instructions (about 7.5 an element in IEEE mode, 7 in TF32), so the eight-wave 256x128 tile, which
-//    splits each element for twice the MFMAs of a 64-wide tile, leads: 4 x [2048,4096]@[4096,4096] runs at 202
-//    TFLOP/s (1211 of bf16 MFMA work; matrix cores busy in 57 % of the cycles, vector issue in 35 %), TF32 on
-//    128x128 tiles at 253 (46 and 49 %); the fp32 instruction's nominal peak is 157.  8 x [512,2048]@[2048,1536]
-//    459 -> 168 us (192 tiles on 256 CUs: 37 and 24 %); TF32 [1024,4096]@[4096,3584] 676 -> 132 us.  16-bit
+//    splits each element for twice the MFMAs of a 64-wide tile, leads: 4 x [2048,4096]@[4096,4096] runs at 196 to
+//    202 TFLOP/s by card (1176 to 1211 of bf16 MFMA work; matrix cores busy in 57 % of the cycles, vector issue in 35 %), TF32 on
+//    128x128 tiles at 250 (46 and 49 %); the fp32 instruction's nominal peak is 157.  8 x [512,2048]@[2048,1536]
+//    459 -> 160 us (192 tiles on 256 CUs: 37 and 24 %); TF32 [1024,4096]@[4096,3584] 676 -> 132 us.  16-bit
 //    tiles are bound by the latency of a slice's loads where few workgroups share a CU: fp16
-//    [777,2881]@[2881,1443] 148 -> 39 us whole, 29 in three splits (element-wise gathers before), with the
-//    matrix cores busy in 8 %; bf16 [4001,4003]@[4003,4005] runs at 873 TFLOP/s.
+//    [777,2881]@[2881,1443] 148 -> 39 us whole, 28 in three splits (element-wise gathers before), with the
+//    matrix cores busy in 8 %; bf16 [4001,4003]@[4003,4005] runs at 854 to 873 TFLOP/s.
 //  * Split-K.  Few tiles leave the chip idle, and a lone workgroup on a CU runs at the latency of its
 //    steps, so a tile's K slices can be shared by several workgroups (fp32 [64,4096]@[4096,1024]:
 //    64 us whole, 17 us in sixteen; the reduction costs about 5 us, so large groups stay whole): each
@@ -58,8 +58,8 @@
 //    such values among ordinary ones cost 12 to 29 % (fp32 [4096,2048]@[2048,1536] 153 -> 184 us,
 //    [1024,2048]@[2048,1536] 55 -> 70; the fp32 instruction alone 307 and 95).  A tile whose outputs are as
 //    small or zero, and one with infinities, NaN or (TF32) values from 2^60, is computed again by GemmTile
-//    with the fp32 instruction, which is up to four times slower than a kernel of it alone
-//    ([1024,2048]@[2048,1536] with an infinity in every tile: 348 us against 95).
+//    with the fp32 instruction, a split unit over its own part of K; that is up to 2.3 times slower than a
+//    kernel of it alone ([1024,2048]@[2048,1536] with an infinity in every tile: 185 us against 95).
 #pragma once
 
 #include "gemm_fast.h"
@@ -470,45 +470,63 @@ struct GeneralTile {
     }
   }
 
-  // Split-K: stores the unit's partial (unless `bad`: a value outside the split's range was met) and
-  // arrives at the tile's counter (arrivals in bits 0-15, bad units above).  The last unit to arrive
-  // re-arms the counter and sums the partials into acc, in split order.  Returns what is left to
-  // this workgroup: 0 nothing, 1 store acc, 2 compute the whole tile with the fp32 instruction.
-  static constexpr int CHUNKS = FM * FN * (ACC / 4);  // 16-byte accumulator chunks per lane
-  __device__ static __forceinline__ int reduce_splits(acc_t (&acc)[FM][FN], const ProblemDesc& pd, bool bad) {
-    __shared__ int s_left;
-    constexpr int kBytes = BM * BN * 4;
+  // Split-K.  A unit's fp32 partial: 16-byte accumulator chunks in the order of acc, 64 lanes each.
+  static constexpr int CHUNKS = FM * FN * (ACC / 4);  // chunks per lane
+  __device__ static __forceinline__ auto partial(const ProblemDesc& pd, int split) {
+    return __builtin_amdgcn_make_buffer_rsrc(pd.partials + ((int64_t)pd.slot0 + split) * (BM * BN), (short)0, BM * BN * 4,
+                                             (int)kBufferFlags);
+  }
+  __device__ static __forceinline__ void store_partial(const acc_t (&acc)[FM][FN], const ProblemDesc& pd) {
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane_off = (wave * CHUNKS * 64 + (int)(threadIdx.x & 63)) * 16;
-    auto partial = [&](int split) {
-      return __builtin_amdgcn_make_buffer_rsrc(pd.partials + ((int64_t)pd.slot0 + split) * (BM * BN), (short)0, kBytes,
-                                               (int)kBufferFlags);
-    };
-    if (!bad) {
-      const auto mine = partial(pd.split);
+    const auto mine = partial(pd, pd.split);
 #pragma unroll
-      for (int c = 0; c < CHUNKS; ++c) {
-        const acc_t& t = acc[c / (ACC / 4) / FN][c / (ACC / 4) % FN];
-        const int q = c % (ACC / 4);
-        const f32x4_t v = {t[q * 4 + 0], t[q * 4 + 1], t[q * 4 + 2], t[q * 4 + 3]};
-        __builtin_amdgcn_raw_buffer_store_b128(v, mine, lane_off + c * 1024, 0, kDeviceCoherent);
-      }
+    for (int c = 0; c < CHUNKS; ++c) {
+      const acc_t& t = acc[c / (ACC / 4) / FN][c / (ACC / 4) % FN];
+      const int q = c % (ACC / 4);
+      const f32x4_t v = {t[q * 4 + 0], t[q * 4 + 1], t[q * 4 + 2], t[q * 4 + 3]};
+      __builtin_amdgcn_raw_buffer_store_b128(v, mine, lane_off + c * 1024, 0, kDeviceCoherent);
     }
+  }
+  // The same of a unit that left the split's range, by the fp32 instruction.  Both layouts give a lane four
+  // consecutive columns at a time, so whole chunks change places.
+  __device__ static __forceinline__ void store_plain_partial(const ProblemDesc& pd, int tm, int tn, char* smem,
+                                                             bool tf32) {
+    ProblemDesc unit = pd;
+    unit.a += (int64_t)pd.k_begin * pd.sak * ES;
+    unit.b += (int64_t)pd.k_begin * pd.sbk * ES;
+    unit.k = pd.k_end - pd.k_begin;
+    typename Plain::acc_t sums[Plain::FM][Plain::FN];
+    Plain::accumulate(sums, unit, tm, tn, smem, tf32);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const auto mine = partial(pd, pd.split);
+#pragma unroll
+    for (int fm = 0; fm < Plain::FM; ++fm)
+#pragma unroll
+      for (int fn = 0; fn < Plain::FN; ++fn) {
+        const int row = fm * 16 + lane % 16, col = fn * 16 + lane / 16 * 4;  // in the wave's sub-tile
+        const int chunk = (row / MI * FN + col / MI) * (ACC / 4) + (MI == 32 ? col % 32 / 8 : 0);
+        const int holder = MI == 32 ? row % 32 + col % 8 / 4 * 32 : lane;
+        const auto& t = sums[fm][fn];
+        const f32x4_t v = {t[0], t[1], t[2], t[3]};
+        __builtin_amdgcn_raw_buffer_store_b128(v, mine, ((wave * CHUNKS + chunk) * 64 + holder) * 16, 0, kDeviceCoherent);
+      }
+  }
+  // Arrives at the tile's counter.  The last unit to do so re-arms it, sums the partials into acc in split
+  // order, and returns true.
+  __device__ static __forceinline__ bool reduce_splits(acc_t (&acc)[FM][FN], const ProblemDesc& pd) {
+    __shared__ int s_last;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane_off = (wave * CHUNKS * 64 + (int)(threadIdx.x & 63)) * 16;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (threadIdx.x == 0) {
       int32_t* word = pd.counters + pd.tile;
-      const int old = atomicAdd(word, bad ? 0x10001 : 1);
-      int left = 0;
-      if ((old & 0xffff) == pd.splits - 1) {
-        atomicExch(word, 0);
-        left = bad || (old >> 16) ? 2 : 1;
-      }
-      s_left = left;
+      s_last = atomicAdd(word, 1) == pd.splits - 1;
+      if (s_last) atomicExch(word, 0);
     }
     __syncthreads();
-    const int left = uniform(s_left);
-    if (left != 1) return left;
+    if (!uniform(s_last)) return false;
     constexpr int GC = CHUNKS < 4 ? CHUNKS : 4, WAYS = 4;  // chunks and partials read at a time
 #pragma unroll
     for (int c0 = 0; c0 < CHUNKS; c0 += GC) {
@@ -519,7 +537,7 @@ struct GeneralTile {
         f32x4_t v[WAYS][GC];
 #pragma unroll
         for (int w = 0; w < WAYS; ++w) {
-          const auto from = partial(min(s0 + w, pd.splits - 1));
+          const auto from = partial(pd, min(s0 + w, pd.splits - 1));
 #pragma unroll
           for (int i = 0; i < GC; ++i)
             v[w][i] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
@@ -541,13 +559,14 @@ struct GeneralTile {
         for (int e = 0; e < 4; ++e) acc[c / (ACC / 4) / FN][c / (ACC / 4) % FN][c % (ACC / 4) * 4 + e] = sum[i][e];
       }
     }
-    return 1;
+    return true;
   }
 
-  // The tile with both operands in 8-element chunks; false when it must be computed by Plain.
-  template <bool AT, bool BT, int EPI, class Hook>
-  __device__ static __forceinline__ bool chunk_tile(const ProblemDesc& pd, int tm, int tn, char* smem,
-                                                    Hook&& before_store) {
+  // The sums of the tile (split-K: of the unit's K range) with both operands in 8-element chunks; false when
+  // Plain must compute them.
+  template <bool AT, bool BT, int EPI>
+  __device__ static __forceinline__ bool chunk_tile(acc_t (&acc)[FM][FN], const ProblemDesc& pd, int tm, int tn,
+                                                    char* smem) {
     const int wave = threadIdx.x >> 6;
     const int wave_m = wave / WN, wave_n = wave % WN;
     const int m0 = tm * BM, n0 = tn * BN;
@@ -559,7 +578,7 @@ struct GeneralTile {
     Frags<!BT, BN, FN> fb;
     fa.setup(wave_m * WTM);
     fb.setup(wave_n * WTN);
-    acc_t acc[FM][FN], low[LM][LN];
+    acc_t low[LM][LN];
 #pragma unroll
     for (int fm = 0; fm < FM; ++fm)
 #pragma unroll
@@ -655,15 +674,7 @@ struct GeneralTile {
     } else {
       __syncthreads();
     }
-    if constexpr (EPI == EPI_SPLIT) {
-      const int left = reduce_splits(acc, pd, bad);
-      if (left != 1) return left == 0;
-    } else {
-      if (bad) return false;
-    }
-    before_store();
-    store_tile(acc, pd, m0, n0, wave_m, wave_n);
-    return true;
+    return !bad;
   }
 
   template <int EPI, class Hook>
@@ -672,24 +683,46 @@ struct GeneralTile {
     static_assert(EPI == EPI_C || EPI == EPI_SPLIT, "the general kernel has no stream-K tail");
     if (pd.swiglu || (EPI == EPI_C && pd.splits > 1)) return;  // the host launches neither
     const ChunkRoute r = chunk_route(F32, ES, BM, BN, pd.m, pd.n, pd.k, pd.sam, pd.sak, pd.sbk, pd.sbn);
+    acc_t acc[FM][FN];
+    // Whole tiles share one copy of what follows their K loops, after all four loops; split units store their
+    // partials within each and share the reduction.  Otherwise that code took registers from the loops: fp32
+    // 256x128 spilled 382 of them and keeps 89 this way, 16-bit split 256x256 1228 and 103.
+    auto run = [&](auto at, auto bt) {
+      if constexpr (EPI == EPI_SPLIT) {
+        acc_t sums[FM][FN];
+        const bool ok = chunk_tile<decltype(at)::value, decltype(bt)::value, EPI>(sums, pd, tm, tn, smem);
+        if (ok) store_partial(sums, pd);
+        return ok;
+      } else {
+        return chunk_tile<decltype(at)::value, decltype(bt)::value, EPI>(acc, pd, tm, tn, smem);
+      }
+    };
+    using yes = std::true_type;
+    using no = std::false_type;
     bool done = false;
-    if constexpr (EPI == EPI_SPLIT) {
-      // Operands Plain must stage: unit 0 of each tile computes it whole.
-      if (!((r.a_rows || (BM >= 32 && r.a_cols)) && (r.b_rows || r.b_cols)) && pd.split != 0) return;
-    }
     if (r.a_rows && r.b_cols) {
-      done = chunk_tile<false, false, EPI>(pd, tm, tn, smem, before_store);
+      done = run(no{}, no{});
     } else if (r.a_rows && r.b_rows) {
-      done = chunk_tile<false, true, EPI>(pd, tm, tn, smem, before_store);
+      done = run(no{}, yes{});
     } else if (r.a_cols && (r.b_cols || r.b_rows)) {
-      if constexpr (BM >= 32) {
-        if (r.b_cols)
-          done = chunk_tile<true, false, EPI>(pd, tm, tn, smem, before_store);
-        else
-          done = chunk_tile<true, true, EPI>(pd, tm, tn, smem, before_store);
+      if constexpr (BM >= 32) done = r.b_cols ? run(yes{}, no{}) : run(yes{}, yes{});
+    }
+    if constexpr (EPI == EPI_SPLIT) {
+      if ((r.a_rows || (BM >= 32 && r.a_cols)) && (r.b_rows || r.b_cols)) {
+        if constexpr (F32) {
+          if (!done) store_plain_partial(pd, tm, tn, smem, tf32);
+        }
+        if (!reduce_splits(acc, pd)) return;
+        done = true;
+      } else if (pd.split != 0) {
+        return;  // operands Plain must stage: unit 0 of each tile computes it whole
       }
     }
-    if (!done) {
+    if (done) {
+      before_store();
+      const int wave = threadIdx.x >> 6;
+      store_tile(acc, pd, tm * BM, tn * BN, wave / WN, wave % WN);
+    } else {
       ProblemDesc whole = pd;
       whole.splits = 1;
       Plain::template run_tile<EPI_C>(whole, tm, tn, smem, tf32, before_store);

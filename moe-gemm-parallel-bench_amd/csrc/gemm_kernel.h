@@ -533,12 +533,9 @@ struct GemmTile {
   }
 
   // -------------------------------------------------------------------------------------------
-  // `before_store` runs once the K loop is done, before the C stores (the work-stealing scheduler
-  // draws its next ticket there).  GemmTile computes whole tiles only: EPI is always EPI_C here.
-  template <int EPI, class Hook>
-  __device__ static __forceinline__ void run_tile(const ProblemDesc& pd, int tm, int tn, char* smem, bool tf32,
-                                                  Hook&& before_store) {
-    static_assert(EPI == EPI_C, "GemmTile has no split-K epilogue");
+  // The tile's sums over pd's K; ends with a barrier.
+  __device__ static __forceinline__ void accumulate(acc_t (&acc)[FM][FN], const ProblemDesc& pd, int tm, int tn,
+                                                    char* smem, bool tf32) {
     const int wave = threadIdx.x >> 6;
     const int wave_m = wave / WN, wave_n = wave % WN;
     const int m0 = tm * BM, n0 = tn * BN;
@@ -547,7 +544,6 @@ struct GemmTile {
     const bool vec_b = pd.sbn == 1 && (pd.n % EPC) == 0 && (pd.sbk % EPC) == 0 &&
                        ((reinterpret_cast<uintptr_t>(pd.b) & 15) == 0);
 
-    acc_t acc[FM][FN];
 #pragma unroll
     for (int fm = 0; fm < FM; ++fm)
 #pragma unroll
@@ -572,8 +568,19 @@ struct GemmTile {
       if (more) store_stage(st, nxt, nxt + A_BYTES);
       __syncthreads();
     }
+  }
+
+  // `before_store` runs once the K loop is done, before the C stores (the work-stealing scheduler
+  // draws its next ticket there).  GemmTile computes whole tiles only: EPI is always EPI_C here.
+  template <int EPI, class Hook>
+  __device__ static __forceinline__ void run_tile(const ProblemDesc& pd, int tm, int tn, char* smem, bool tf32,
+                                                  Hook&& before_store) {
+    static_assert(EPI == EPI_C, "GemmTile has no split-K epilogue");
+    const int wave = threadIdx.x >> 6;
+    acc_t acc[FM][FN];
+    accumulate(acc, pd, tm, tn, smem, tf32);
     before_store();
-    store_tile(acc, pd, m0, n0, wave_m, wave_n);
+    store_tile(acc, pd, tm * BM, tn * BN, wave / WN, wave % WN);
   }
 };
 

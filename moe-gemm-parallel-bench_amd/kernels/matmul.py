@@ -407,7 +407,7 @@ def with_split_options(configs, tiles_of, k: int, sm_count: int, split_k, splitt
     ``split_k`` pins the split of every candidate.  ``general``: tile keys of the general kernels that
     can split (None for the LDS-DMA kernels).  Those run one slice's latency at a time and most fit a CU
     twice, so the count that gives every CU two units, and two splits of up to three tiles a CU, are
-    timed too: fp16 [777,2881]@[2881,1443] 39 us unsplit, 29 in three (156 tiles of 64x128); fp32
+    timed too: fp16 [777,2881]@[2881,1443] 39 us unsplit, 28 in three (156 tiles of 64x128); fp32
     [64,4096]@[4096,1024] 64 us unsplit, 17 in sixteen."""
     out = []
     for cfg in configs:

@@ -316,3 +316,36 @@ def test_fp32_sums_of_few_products(terms, precision):
         torch.cuda.synchronize()
         error = float((c.double() - reference).norm() / reference.norm())
         assert error <= bound, (cfg, error, bound)
+
+
+@pytest.mark.parametrize("precision", ["ieee", "tf32"])
+@pytest.mark.parametrize("splits", [2, 5])
+def test_split_units_outside_the_range(splits, precision):
+    """Values that only the fp32 instruction takes, in one unit of some tiles and in all units of others; the
+    other units keep their bf16 parts and the sums stay those of integers."""
+    from kernels import _native
+    from kernels.matmul import launch_matmul
+
+    m, k, n = 300, 640, 270
+    gen = torch.Generator(device="cuda").manual_seed(31)
+    a = torch.randint(-2, 3, (m, k), generator=gen, device="cuda").float()
+    b = torch.randint(1, 3, (k, n), generator=gen, device="cuda").float()
+    a[7, 630], a[140, 3], a[299, ::40] = float("inf"), float("-inf"), float("nan")
+    a[200, ::50] = 2.0**61  # TF32 mode's own limit; exact in fp32 beside sums that it swallows
+    reference = a.cpu().double() @ b.cpu().double()
+    bound = k * 2.0**-24 * (a.cpu().double().abs() @ b.cpu().double().abs())
+    for cfg in _tiles(torch.float32):
+        if cfg.tile_key not in _native.split_tiles(_native.DTYPE_F32, _native.GENERAL):
+            continue
+        for _ in range(2):  # the counters are re-armed
+            c = torch.full((m, n), 5.0, device="cuda")
+            print(f"split units outside the range {cfg.tile_key} {precision} splits={splits}", flush=True)
+            launch_matmul(a, b, c, cfg, precision, autotune=False, split_k=splits)
+            torch.cuda.synchronize()
+            got = c.cpu().double()
+            assert torch.equal(torch.isnan(got), torch.isnan(reference)), cfg
+            infinite = torch.isinf(reference)
+            assert torch.equal(got[infinite], reference[infinite]), cfg
+            plain = [i for i in range(m) if i not in (7, 140, 200, 299)]
+            assert torch.equal(got[plain], reference[plain]), cfg
+            assert ((got[200] - reference[200]).abs() <= bound[200]).all(), cfg
