@@ -25,26 +25,26 @@
 //    addition.  TF32 operands (11 significand bits) are the exact sum of two bf16 values, and all
 //    four products are computed.  Products whose parts are not both the first are summed apart from the
 //    rest and added once, at the end of the tile: in one sum all parts of a product would round at the size of
-//    the whole.  So sums are as close to the exact ones as the fp32 instruction's, few products or many
-//    (error against 64 bits, fp32 instruction -> one sum of all parts -> now, normal operands, 2-norms):
+//    the whole.  So sums are closer to the exact ones than the fp32 instruction's, and single products about
+//    as close (error against 64 bits, fp32 instruction -> one sum of all parts -> now, normal operands, 2-norms):
 //      K = 64                      1.43e-7 -> 1.07e-7 -> 4.8e-8     TF32 1.30e-7 -> 8.5e-8 -> 4.8e-8
 //      K = 2048                                 7.0e-7 -> 2.7e-7              5.6e-7 -> 1.8e-7
 //      rows of K = 512 with 8 values other than zero
 //                                  5.4e-8 -> 1.09e-7 -> 2.9e-8      TF32 4.6e-8 -> 5.2e-8 -> 2.9e-8
 //      with one                    2.54e-8 -> 3.5e-8 -> 2.60e-8     TF32 0 -> 0 -> 0
 //    and the same at scales down to products of 2^-125, whose subnormal parts the matrix cores keep.  It
-//    costs up to 5 % on large calls (8 x [512,2048]@[2048,1536] 152 -> 154 us, 4 x [2048,4096]@[4096,4096]
+//    costs up to 7 % on large calls (8 x [512,2048]@[2048,1536] 152 -> 154 us, 4 x [2048,4096]@[4096,4096]
 //    1382 -> 1403 us, TF32 1071 -> 1097 us).  Below K = 8 the fp32 instruction runs.
 //    Chunks are split on their way into LDS, once per workgroup, into one LDS panel per part.
 //  * Bound and measured.  Large fp32 tiles are bound by the matrix cores and by the split's vector
 //    instructions (about 7.5 an element in IEEE mode, 7 in TF32), so the eight-wave 256x128 tile, which
-//    splits each element for twice the MFMAs of a 64-wide tile, leads: 4 x [2048,4096]@[4096,4096] runs at 196 to
-//    202 TFLOP/s by card (1176 to 1211 of bf16 MFMA work; matrix cores busy in 57 % of the cycles, vector issue in 35 %), TF32 on
-//    128x128 tiles at 250 (46 and 49 %); the fp32 instruction's nominal peak is 157.  8 x [512,2048]@[2048,1536]
-//    459 -> 160 us (192 tiles on 256 CUs: 37 and 24 %); TF32 [1024,4096]@[4096,3584] 676 -> 132 us.  16-bit
-//    tiles are bound by the latency of a slice's loads where few workgroups share a CU: fp16
-//    [777,2881]@[2881,1443] 148 -> 39 us whole, 28 in three splits (element-wise gathers before), with the
-//    matrix cores busy in 8 %; bf16 [4001,4003]@[4003,4005] runs at 854 to 873 TFLOP/s.
+//    splits each element for twice the MFMAs of a 64-wide tile, leads: 4 x [2048,4096]@[4096,4096] runs at
+//    196 to 202 TFLOP/s by card (1176 to 1211 of bf16 MFMA work; matrix cores busy in 57 % of the cycles, vector
+//    issue in 35 %), TF32 at 250 (46 and 49 % on 128x128 tiles); the fp32 instruction's nominal peak is 157.  8 x [512,2048]@[2048,1536] 459 -> 160 us (192 tiles
+//    on 256 CUs: 39 and 25 %); TF32 [1024,4096]@[4096,3584] 676 -> 132 us.  16-bit tiles are bound by the latency
+//    of a slice's loads where few workgroups share a CU: fp16 [777,2881]@[2881,1443] 148 -> 39 us whole, 28 in
+//    three splits (element-wise gathers before), with the matrix cores busy in 8 %; bf16
+//    [4001,4003]@[4003,4005] runs at 854 to 873 TFLOP/s.
 //  * Split-K.  Few tiles leave the chip idle, and a lone workgroup on a CU runs at the latency of its
 //    steps, so a tile's K slices can be shared by several workgroups (fp32 [64,4096]@[4096,1024]:
 //    64 us whole, 17 us in sixteen; the reduction costs about 5 us, so large groups stay whole): each

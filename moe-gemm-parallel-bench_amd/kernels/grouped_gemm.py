@@ -361,14 +361,17 @@ def _group_layout(workspace: GroupedWorkspace, dtype_code: int) -> int:
     cached = getattr(workspace, "_layout_cache", None)
     if cached is not None and cached[0] == key:
         return cached[1]
-    def layout_of(a, b, c):
-        layout = _native.GENERAL if dtype_code == _native.DTYPE_F32 else _problem_layout(a, b, c)
-        return _native.strided_or(layout, a, b)
+    sixteen = dtype_code != _native.DTYPE_F32
+    if sixteen and all(map(_problem_vector_ok, workspace.a, workspace.b, workspace.c)):
+        value = 0
+    else:
+        def layout_of(a, b, c):
+            return _native.strided_or(_problem_layout(a, b, c) if sixteen else _native.GENERAL, a, b)
 
-    value = layout_of(workspace.a[0], workspace.b[0], workspace.c[0])
-    if (value > 0 and workspace.homogeneous) or (value != _native.GENERAL and any(
-            layout_of(a, b, c) != value for a, b, c in workspace.problem_tensors())):
-        value = _native.GENERAL
+        value = layout_of(workspace.a[0], workspace.b[0], workspace.c[0])
+        if (value > 0 and workspace.homogeneous) or (value != _native.GENERAL and any(
+                layout_of(a, b, c) != value for a, b, c in workspace.problem_tensors())):
+            value = _native.GENERAL
     workspace._layout_cache = (key, value)
     return value
 
