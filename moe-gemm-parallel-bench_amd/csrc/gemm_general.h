@@ -40,11 +40,11 @@
 //    instructions (about 7.5 an element in IEEE mode, 7 in TF32), so the eight-wave 256x128 tile, which
 //    splits each element for twice the MFMAs of a 64-wide tile, leads: 4 x [2048,4096]@[4096,4096] runs at
 //    196 to 202 TFLOP/s by card (1176 to 1211 of bf16 MFMA work; matrix cores busy in 57 % of the cycles, vector
-//    issue in 35 %), TF32 at 250 (46 and 49 % on 128x128 tiles); the fp32 instruction's nominal peak is 157.  8 x [512,2048]@[2048,1536] 459 -> 160 us (192 tiles
-//    on 256 CUs: 39 and 25 %); TF32 [1024,4096]@[4096,3584] 676 -> 132 us.  16-bit tiles are bound by the latency
-//    of a slice's loads where few workgroups share a CU: fp16 [777,2881]@[2881,1443] 148 -> 39 us whole, 28 in
-//    three splits (element-wise gathers before), with the matrix cores busy in 8 %; bf16
-//    [4001,4003]@[4003,4005] runs at 854 to 873 TFLOP/s.
+//    issue in 35 %), TF32 at 250 (46 and 49 % on 128x128 tiles); the fp32 instruction's nominal peak is 157.
+//    8 x [512,2048]@[2048,1536] 459 -> 160 us (192 tiles on 256 CUs: 39 and 25 %); TF32 [1024,4096]@[4096,3584]
+//    676 -> 132 us.  16-bit tiles are bound by the latency of a slice's loads where few workgroups share a
+//    CU: fp16 [777,2881]@[2881,1443] 148 -> 39 us whole, 28 in three splits (element-wise gathers before),
+//    with the matrix cores busy in 8 %; bf16 [4001,4003]@[4003,4005] runs at 854 to 873 TFLOP/s.
 //  * Split-K.  Few tiles leave the chip idle, and a lone workgroup on a CU runs at the latency of its
 //    steps, so a tile's K slices can be shared by several workgroups (fp32 [64,4096]@[4096,1024]:
 //    64 us whole, 17 us in sixteen; the reduction costs about 5 us, so large groups stay whole): each
