@@ -326,10 +326,10 @@ _SPLITK_MAX_SPLITS, _SPLITK_MAX_TILES = 64, 65536  # the split-K launches' limit
 # launches use it, in the order of the one stream it belongs to, and no captured graph holds its address
 # (two graphs captured on one stream, or a graph beside eager calls on its capture stream, may replay at
 # once).  Each buffer is made on its own stream and used on no other, so dropping one is safe at any
-# time: its memory is reused in that stream's order.  At most 16 streams hold one, as large as the last
-# growth asked for.
+# time: its memory is reused in that stream's order.  At most 33 streams hold one (torch's stream pool and
+# the default stream), as large as the last growth asked for.
 _EAGER_SCRATCH: dict[tuple[int, int], object] = {}
-_EAGER_SCRATCH_STREAMS = 16
+_EAGER_SCRATCH_STREAMS = 33
 _EAGER_SCRATCH_LOCK = threading.Lock()
 
 
