@@ -473,8 +473,8 @@ struct GeneralTile {
   // Split-K.  A unit's fp32 partial: 16-byte accumulator chunks in the order of acc, 64 lanes each.
   static constexpr int CHUNKS = FM * FN * (ACC / 4);  // chunks per lane
   __device__ static __forceinline__ auto partial(const ProblemDesc& pd, int split) {
-    return __builtin_amdgcn_make_buffer_rsrc(pd.partials + ((int64_t)pd.slot0 + split) * (BM * BN), (short)0, BM * BN * 4,
-                                             (int)kBufferFlags);
+    return __builtin_amdgcn_make_buffer_rsrc(pd.partials + ((int64_t)pd.slot0 + split) * (BM * BN), (short)0,
+                                             BM * BN * 4, (int)kBufferFlags);
   }
   __device__ static __forceinline__ void store_partial(const acc_t (&acc)[FM][FN], const ProblemDesc& pd) {
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -509,7 +509,8 @@ struct GeneralTile {
         const int holder = MI == 32 ? row % 32 + col % 8 / 4 * 32 : lane;
         const auto& t = sums[fm][fn];
         const f32x4_t v = {t[0], t[1], t[2], t[3]};
-        __builtin_amdgcn_raw_buffer_store_b128(v, mine, ((wave * CHUNKS + chunk) * 64 + holder) * 16, 0, kDeviceCoherent);
+        const int at = ((wave * CHUNKS + chunk) * 64 + holder) * 16;
+        __builtin_amdgcn_raw_buffer_store_b128(v, mine, at, 0, kDeviceCoherent);
       }
   }
   // Arrives at the tile's counter.  The last unit to do so re-arms it, sums the partials into acc in split

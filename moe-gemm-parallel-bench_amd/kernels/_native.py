@@ -9,8 +9,8 @@ required" error (reference kernels/grouped_gemm.py:626-627, kernels/matmul.py:34
 from __future__ import annotations
 
 import ctypes
-import threading
 import os
+import threading
 from functools import lru_cache
 from pathlib import Path
 

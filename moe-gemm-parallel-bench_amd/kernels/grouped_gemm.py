@@ -353,8 +353,9 @@ def _problem_layout(a, b, c) -> int:
 
 def _group_layout(workspace: GroupedWorkspace, dtype_code: int) -> int:
     """The one LDS-DMA layout every problem meets (0 row-major, 1 to 3 transposed), or GENERAL, or STRIDED
-    where every problem is; cached per set of tensor objects.  Homogeneous groups launch without a strides table, as row-major
-    ones: with K = 1 a transposed view counts as contiguous too, and stays GENERAL there."""
+    where every problem is; cached per set of tensor objects.  Homogeneous groups launch without a
+    strides table, as row-major ones: with K = 1 a transposed view counts as contiguous too, and stays
+    GENERAL there."""
     if dtype_code == _native.DTYPE_F32 and workspace.homogeneous:
         return _native.GENERAL
     key = (tuple(map(id, workspace.a)), tuple(map(id, workspace.b)), tuple(map(id, workspace.c)))

@@ -376,20 +376,14 @@ def _vector_ok(a, b, c) -> bool:
 
 def _operand_layout(a, b, c) -> int:
     """Layout of the LDS-DMA kernels these operands meet: 0 row-major, 1 to 3 transposed, GENERAL."""
-    import torch
-
-    if a.dtype not in (torch.float16, torch.bfloat16):
+    if a.element_size() != 2:
         return _native.GENERAL
     return 0 if _vector_ok(a, b, c) else _native.transposed_layout(a, b, c)
 
 
-def _launch_layout(a, b, c, dtype_code: int) -> int:
+def _launch_layout(a, b, c) -> int:
     """``_operand_layout``, or STRIDED."""
-    if dtype_code != _native.DTYPE_F32:
-        layout = 0 if _vector_ok(a, b, c) else _native.transposed_layout(a, b, c)
-        if layout != _native.GENERAL:
-            return layout
-    return _native.strided_or(_native.GENERAL, a, b)
+    return _native.strided_or(_operand_layout(a, b, c), a, b)
 
 
 def splitk_count(tiles: int, k: int, block_k: int, sm_count: int) -> int:
@@ -495,7 +489,7 @@ def _launch_fixed(a, b, c, m, n, k, cfg: KernelConfig, dtype_code: int, precisio
             return 1
         split_k = 1
     if layout is None:
-        layout = _launch_layout(a, b, c, dtype_code)
+        layout = _launch_layout(a, b, c)
     if layout == 0 or cfg.tile_key in _native.split_tiles(dtype_code, layout):
         tiles = -(-m // cfg.block_m) * -(-n // cfg.block_n)
         splits = split_k if split_k is not None else splitk_count(tiles, k, cfg.block_k,
@@ -561,7 +555,7 @@ def launch_matmul(
         raise ValueError("split_k must be None or a positive integer")
     if b_stream not in (None, 0, 1):
         raise ValueError(f"b_stream must be None, 0 or 1, got {b_stream!r}")
-    layout = _launch_layout(a, b, c, dtype_code)
+    layout = _launch_layout(a, b, c)
     if not autotune:
         cfg = config or layout_config(select_config(m, n, k, a.dtype), dtype_code, layout, a.dtype)
         _LAST_SPLIT[0] = _launch_fixed(a, b, c, m, n, k, cfg, dtype_code, precision, split_k, b_stream or 0,
